@@ -204,11 +204,23 @@ size_t scratch_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k)
     return 0;
 }
 
+// The tile GEMM's K-slice partials (the rest of a product's scratch), and
+// whether the path counts slices: the Q4_0 float GEMMs.
+size_t part_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
+    return p == Path::Gemm && t == WType::Q4_0 && !native && m > rdl::GEMM_XTILE_M && k <= rdl::GEMM_TILE_MAX_K
+               ? rdl::gemm_part_bytes(m, n, k)
+               : 0;
+}
+bool wants_counters(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
+    return p == Path::Gemm && t == WType::Q4_0 && !native &&
+           (m <= rdl::GEMM_SMALL_M || part_bytes(t, p, native, m, n, k) > 0);
+}
+
 // Run the product on `s`; `work` holds scratch_bytes(path) bytes of device
-// memory, `counters` gemm_counter_count(n, k) ints of the GEMM (zero between calls).
+// memory, `part` part_bytes (or is NULL: unsplit), `counters` gemm_counter_count(n, k) ints of the GEMM (zero between calls).
 rdl_status run_linear(WType t, bool native, const uint8_t* w_dev, size_t n, size_t k,
-                      const float* x_dev, size_t m, float* y_dev, void* work, int* counters, hipStream_t s,
-                      Path path) {
+                      const float* x_dev, size_t m, float* y_dev, void* work, float* part, int* counters,
+                      hipStream_t s, Path path) {
     if (m == 0 || n == 0) return RDL_OK;
     // k == 0: no blocks; the GEMV then writes zeros (empty dot, as in the reference).
     if (k == 0) {
@@ -221,11 +233,11 @@ rdl_status run_linear(WType t, bool native, const uint8_t* w_dev, size_t n, size
     }
     if (path == Path::Gemm) {
         if (t != WType::Q4_0)
-            HIP_TRY(rdl::launch_gemm_typed(t, w_dev, n, k, x_dev, m, y_dev, work, s));
+            HIP_TRY(rdl::launch_gemm_typed(t, w_dev, n, k, x_dev, m, y_dev, work, part, counters, s));
         else if (native)
             HIP_TRY(rdl::launch_gemm_q4_0_native(w_dev, n, k, x_dev, m, y_dev, nullptr, work, s));
         else
-            HIP_TRY(rdl::launch_gemm_q4_0(w_dev, n, k, x_dev, m, y_dev, work, counters, s));
+            HIP_TRY(rdl::launch_gemm_q4_0(w_dev, n, k, x_dev, m, y_dev, work, part, counters, s));
         return RDL_OK;
     }
     void* xrec = work;
@@ -243,10 +255,14 @@ rdl_status run_linear(WType t, bool native, const uint8_t* w_dev, size_t n, size
 // from hipGetSymbolAddress, taken once per device (with that device current)
 // and kept in scratch_dev[]; only that address is ever passed to kernels.
 __device__ __align__(256) uint8_t scratch[RDL_NOALLOC_SCRATCH_BYTES];
+// The tile GEMM's K-slice partials have an array of their own: a product's
+// other scratch alone decides whether it fits.
+__device__ __align__(256) float scratch_part[rdl::GEMM_PART_BYTES / sizeof(float)];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex scratch_mu;
 void* scratch_dev[MAX_DEVICES] = {};
+void* scratch_part_dev[MAX_DEVICES] = {};
 
 // The last NOALLOC_COUNTER_BYTES of `scratch` hold the prefill GEMM's counters
 // (zero from load time and left at zero by every launch); nothing else is
@@ -254,8 +270,8 @@ void* scratch_dev[MAX_DEVICES] = {};
 constexpr size_t NOALLOC_COUNTER_BYTES = 64 * 1024;
 constexpr size_t NOALLOC_DATA_BYTES = (size_t)RDL_NOALLOC_SCRATCH_BYTES - NOALLOC_COUNTER_BYTES;
 
-// The current device's address of `scratch`.
-rdl_status noalloc_scratch(void** out) {
+// The current device's addresses of `scratch` and `scratch_part`.
+rdl_status noalloc_scratch(void** out, void** part) {
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= MAX_DEVICES) return fail(RDL_ERR_UNSUPPORTED, "device index %d beyond %d", dev, MAX_DEVICES);
@@ -265,9 +281,15 @@ rdl_status noalloc_scratch(void** out) {
         const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !p)
             return fail(RDL_ERR_HIP, "hipGetSymbolAddress(scratch) failed: %s", hipGetErrorString(e));
+        void* q = nullptr;
+        const hipError_t e2 = hipGetSymbolAddress(&q, HIP_SYMBOL(scratch_part));
+        if (e2 != hipSuccess || !q)
+            return fail(RDL_ERR_HIP, "hipGetSymbolAddress(scratch_part) failed: %s", hipGetErrorString(e2));
         scratch_dev[dev] = p;
+        scratch_part_dev[dev] = q;
     }
     *out = scratch_dev[dev];
+    *part = scratch_part_dev[dev];
     return RDL_OK;
 }
 
@@ -382,13 +404,15 @@ rdl_status host_matmul(WType t, bool native, const float* x, size_t x_len, const
     HIP_TRY(hipMemcpy(dx.p, x, m * k * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dw.p, w, wb, hipMemcpyHostToDevice));
     const Path path = pick_path(t, native, m, n, k, (const float*)dx.p);
-    const size_t sb = scratch_bytes(t, path, native, m, n, k);
-    if (sb) HIP_TRY(dr.alloc(sb));
+    const size_t sb = (scratch_bytes(t, path, native, m, n, k) + 255) & ~(size_t)255;
+    const size_t pb = part_bytes(t, path, native, m, n, k);
+    if (sb + pb) HIP_TRY(dr.alloc(sb + pb));
     DevBuf dc;
     HIP_TRY(dc.alloc(rdl::gemm_counter_count(n, k) * sizeof(int)));
     HIP_TRY(hipMemset(dc.p, 0, rdl::gemm_counter_count(n, k) * sizeof(int)));
     st = run_linear(t, native, (const uint8_t*)dw.p, n, k, (const float*)dx.p, m, (float*)dy.p,
-                    dr.p, (int*)dc.p, nullptr, path);
+                    dr.p, pb ? reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(dr.p) + sb) : nullptr, (int*)dc.p,
+                    nullptr, path);
     if (st != RDL_OK) return st;
     HIP_TRY(hipMemcpy(y, dy.p, m * n * sizeof(float), hipMemcpyDeviceToHost));
     return ok();
@@ -618,11 +642,13 @@ rdl_status rdl_linear_forward_dev(const rdl_weight* w, const float* x_dev, size_
     const bool native = mode == RDL_MODE_NATIVE && (w->type == WType::Q4_0 || w->type == WType::Q4_1);
     hipStream_t s = (hipStream_t)stream;
     const Path path = pick_path(w->type, native, m, w->n, w->k, x_dev);
-    const bool want_counters = path == Path::Gemm && w->type == WType::Q4_0 && !native && m <= rdl::GEMM_SMALL_M;
+    const size_t sb = (scratch_bytes(w->type, path, native, m, w->n, w->k) + 255) & ~(size_t)255;
+    const size_t pb = part_bytes(w->type, path, native, m, w->n, w->k);
     CallWork cw;
-    rdl_status st = cw.get(w, s, scratch_bytes(w->type, path, native, m, w->n, w->k), want_counters);
+    rdl_status st = cw.get(w, s, sb + pb, wants_counters(w->type, path, native, m, w->n, w->k));
     if (st != RDL_OK) return st;
-    st = run_linear(w->type, native, (const uint8_t*)w->dev, w->n, w->k, x_dev, m, y_dev, cw.p, cw.counters, s,
+    float* part = pb ? reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(cw.p) + sb) : nullptr;
+    st = run_linear(w->type, native, (const uint8_t*)w->dev, w->n, w->k, x_dev, m, y_dev, cw.p, part, cw.counters, s,
                     path);
     const rdl_status rs = cw.release(s);
     if (st != RDL_OK) return st;
@@ -673,11 +699,12 @@ rdl_status rdl_linear_forward_dev_noalloc(const rdl_weight* w, const float* x_de
                     m, w->k, rb, NOALLOC_DATA_BYTES);
     if (rdl::gemm_counter_count(w->n, w->k) * sizeof(int) > NOALLOC_COUNTER_BYTES)
         return fail(RDL_ERR_UNSUPPORTED, "out_features %zu beyond the static scratch's GEMM counters", w->n);
-    void* work = nullptr;
-    rdl_status st = noalloc_scratch(&work);
+    void *work = nullptr, *part = nullptr;
+    rdl_status st = noalloc_scratch(&work, &part);
     if (st != RDL_OK) return st;
     int* counters = reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(work) + NOALLOC_DATA_BYTES);
-    st = run_linear(w->type, native, (const uint8_t*)w->dev, w->n, w->k, x_dev, m, y_dev, work, counters,
+    st = run_linear(w->type, native, (const uint8_t*)w->dev, w->n, w->k, x_dev, m, y_dev, work,
+                    part_bytes(w->type, path, native, m, w->n, w->k) ? (float*)part : nullptr, counters,
                     (hipStream_t)stream, path);
     return st == RDL_OK ? ok() : st;
 }

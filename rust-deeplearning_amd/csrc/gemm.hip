@@ -915,6 +915,7 @@ std::atomic<bool> combine_coherent{false};  // testing switch: every combine coh
 // never while `s` is being captured into a graph (that call takes the
 // coherent combine); false while the testing switch asks for the coherent
 // combine.
+}  // namespace
 bool xcd_round_robin(hipStream_t s) {
     if (combine_coherent.load()) return false;
     int dev = 0;
@@ -940,6 +941,7 @@ bool xcd_round_robin(hipStream_t s) {
     xcd_state[dev] = ok ? 1 : 2;
     return ok;
 }
+namespace {
 
 // ---- skinny GEMM (m <= GEMM_SMALL_M) ----------------------------------------------
 // With few x rows, x is the costly operand: a workgroup that owns a strip of
@@ -1810,7 +1812,8 @@ hipError_t launch_zero_counters(int* counters, size_t count, hipStream_t s) {
     return hipGetLastError();
 }
 
-size_t gemm_counter_count(size_t n, size_t) { return (n + 63) / 64 + 1; }  // a counter per strip of 64 (or 128) rows
+// a counter per strip of 64 (or 128) rows, or per tile of a split tile GEMM
+size_t gemm_counter_count(size_t n, size_t) { return std::max((n + 63) / 64 + 1, GEMM_SPLIT_TILES); }
 
 size_t gemm_scratch_bytes(size_t m, size_t n, size_t k, bool native) {
     if (!native && m >= 1 && m <= GEMM_XTILE_M) {  // the K-slice partials of the x-tile kernel
@@ -1837,8 +1840,10 @@ size_t gemm_tiles_scratch_bytes(size_t m, size_t k) {
 }
 
 hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
-                            void* scratch, int* counters, hipStream_t s) {
+                            void* scratch, float* tpart, int* counters, hipStream_t s) {
     if (n == 0 || m == 0) return hipSuccess;
+    if (m > GEMM_XTILE_M && k <= GEMM_TILE_MAX_K)
+        return launch_gemm_tile(WType::Q4_0, w, n, k, x, m, y, scratch, tpart, counters, 0, nullptr, 0.0f, false, s);
     if (m <= GEMM_XTILE_M) {
         float* part = reinterpret_cast<float*>(scratch);  // the K-slice partials
         const hipError_t e = launch_xtile(w, (int)n, (int)(k / QK), x, (int)m, y, part, counters, s);
@@ -1863,7 +1868,8 @@ hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x
 }
 
 hipError_t launch_gemm_tiles_ex(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
-                                void* scratch, int pro, const float* g, float eps, bool accumulate, hipStream_t s) {
+                                void* scratch, float* part, int* counters, int pro, const float* g, float eps,
+                                bool accumulate, hipStream_t s) {
     if (n == 0 || m == 0) return hipSuccess;
     const bool q40 = t == WType::Q4_0;
     if ((!q40 && t != WType::Q4_K && t != WType::Q6_K && t != WType::Q8_0 && t != WType::Q4_1) || k == 0 ||
@@ -1877,6 +1883,8 @@ hipError_t launch_gemm_tiles_ex(WType t, const uint8_t* w, size_t n, size_t k, c
     // 32-bit buffer offsets, out-of-range slots at RSRC_OOB
     const size_t wb = n * (k / block_elems(t)) * block_bytes(t);
     if (wb > FUSED_MAX_WEIGHT_BYTES || m * k * 2 > FUSED_MAX_WEIGHT_BYTES) return hipErrorInvalidValue;
+    if (q40 && k <= GEMM_TILE_MAX_K)
+        return launch_gemm_tile(t, w, n, k, x, m, y, scratch, part, counters, pro, g, eps, accumulate, s);
     const size_t xb = (m * k * 2 + 255) & ~(size_t)255;
     _Float16* xh = reinterpret_cast<_Float16*>(scratch);
     _Float16* xl = reinterpret_cast<_Float16*>(reinterpret_cast<uint8_t*>(scratch) + xb);
@@ -1909,9 +1917,9 @@ hipError_t launch_gemm_tiles_ex(WType t, const uint8_t* w, size_t n, size_t k, c
 }
 
 hipError_t launch_gemm_typed(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
-                             void* scratch, hipStream_t s) {
+                             void* scratch, float* part, int* counters, hipStream_t s) {
     if (t == WType::Q4_0) return hipErrorInvalidValue;  // launch_gemm_q4_0
-    return launch_gemm_tiles_ex(t, w, n, k, x, m, y, scratch, 0, nullptr, 0.0f, false, s);
+    return launch_gemm_tiles_ex(t, w, n, k, x, m, y, scratch, part, counters, 0, nullptr, 0.0f, false, s);
 }
 
 hipError_t launch_gemm_q4_0_native(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,

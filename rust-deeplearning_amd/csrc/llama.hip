@@ -647,7 +647,8 @@ struct LlamaModel {
     int *tokens = nullptr, *pos = nullptr, *step = nullptr, *out_tokens = nullptr;
     size_t out_cap = 0;
     void* gemm_scratch = nullptr;
-    int* gemm_cnt = nullptr;  // the skinny GEMMs' strip counters (zero between launches)
+    float* gemm_part = nullptr;  // the tile GEMM's K-slice partials
+    int* gemm_cnt = nullptr;     // the split GEMMs' strip and tile counters (zero between launches)
     float* att_part = nullptr;  // [max_batch][n_heads][spans of max_seq][hd + 2]
     int* att_cnt = nullptr;     // [max_batch][n_heads] finished-chunk counters (zero between launches)
     int att_nspan = 0;
@@ -702,9 +703,10 @@ struct LlamaModel {
         if (m <= 4) return launch_gemv_fused(w.type, native, w.dev, w.n, w.k, xin, m, y, stream);
         if (w.type == WType::Q4_0)
             return native ? launch_gemm_q4_0_native(w.dev, w.n, w.k, xin, m, y, nullptr, gemm_scratch, stream)
-                          : launch_gemm_q4_0(w.dev, w.n, w.k, xin, m, y, gemm_scratch, gemm_cnt, stream);
+                          : launch_gemm_q4_0(w.dev, w.n, w.k, xin, m, y, gemm_scratch, gemm_part, gemm_cnt, stream);
         if (kgemm(w, m, native)) {
-            const hipError_t e = launch_gemm_typed(w.type, w.dev, w.n, w.k, xin, m, y, gemm_scratch, stream);
+            const hipError_t e = launch_gemm_typed(w.type, w.dev, w.n, w.k, xin, m, y, gemm_scratch, gemm_part, gemm_cnt,
+                                                   stream);
             if (e != hipErrorInvalidValue) return e;
         }
         // rows four at a time through the fused GEMV (other types, or scales
@@ -964,7 +966,7 @@ struct LlamaModel {
         const bool nat = L.native;
         bool qkv_done = false;
         if (np == 1 && q4t(L.qkv)) {
-            e = launch_gemm_tiles_ex(L.qkv.type, L.qkv.dev, L.qkv.n, L.qkv.k, x, m, qkv, gemm_scratch, 1,
+            e = launch_gemm_tiles_ex(L.qkv.type, L.qkv.dev, L.qkv.n, L.qkv.k, x, m, qkv, gemm_scratch, gemm_part, gemm_cnt, 1,
                                      L.attn_norm, cfg.norm_eps, false, stream);
             if (e != hipSuccess && e != hipErrorInvalidValue) return e;
             qkv_done = e == hipSuccess;
@@ -1005,7 +1007,7 @@ struct LlamaModel {
         e = cfg.kv_f16 ? layer_attention<_Float16>(l, m, !rope_fused) : layer_attention<float>(l, m, !rope_fused);
         if (e != hipSuccess) return e;
         // ---- x += att . Wo^T ----
-        e = q4t(L.o) ? launch_gemm_tiles_ex(L.o.type, L.o.dev, L.o.n, L.o.k, att, m, x, gemm_scratch, 0, nullptr,
+        e = q4t(L.o) ? launch_gemm_tiles_ex(L.o.type, L.o.dev, L.o.n, L.o.k, att, m, x, gemm_scratch, gemm_part, gemm_cnt, 0, nullptr,
                                             0.0f, true, stream)
                      : hipErrorInvalidValue;
         if (e != hipSuccess && e != hipErrorInvalidValue) return e;
@@ -1023,7 +1025,7 @@ struct LlamaModel {
         // x split forms h from them
         bool gu_raw = false;
         if (!L.split_gu && q4t(L.gu) && q4t(L.down)) {
-            e = launch_gemm_tiles_ex(L.gu.type, L.gu.dev, L.gu.n, L.gu.k, x, m, gu, gemm_scratch, 1, L.ffn_norm,
+            e = launch_gemm_tiles_ex(L.gu.type, L.gu.dev, L.gu.n, L.gu.k, x, m, gu, gemm_scratch, gemm_part, gemm_cnt, 1, L.ffn_norm,
                                      cfg.norm_eps, false, stream);
             if (e != hipSuccess && e != hipErrorInvalidValue) return e;
             gu_raw = e == hipSuccess;
@@ -1049,7 +1051,7 @@ struct LlamaModel {
         }
         // ---- x += h . Wdown^T ----
         if (gu_raw) {
-            e = launch_gemm_tiles_ex(L.down.type, L.down.dev, L.down.n, L.down.k, gu, m, x, gemm_scratch, 2, nullptr,
+            e = launch_gemm_tiles_ex(L.down.type, L.down.dev, L.down.n, L.down.k, gu, m, x, gemm_scratch, gemm_part, gemm_cnt, 2, nullptr,
                                      0.0f, true, stream);
             if (e != hipSuccess && e != hipErrorInvalidValue) return e;
             if (e == hipErrorInvalidValue) {  // the SwiGLU on its own, then the product
@@ -1371,6 +1373,7 @@ rdl_status rdl_llama_create_typed(const rdl_llama_config* cfg, const int32_t* ty
         gsb = std::max(gsb, rdl::gemm_tiles_scratch_bytes(mb, sh[1]));
     }
     if ((e = M.alloc(&M.gemm_scratch, gsb)) != hipSuccess) return fail_free(e);
+    if ((e = M.alloc_t(&M.gemm_part, rdl::GEMM_PART_BYTES / sizeof(float))) != hipSuccess) return fail_free(e);
     if ((e = M.alloc_t(&M.gemm_cnt, gcc)) != hipSuccess) return fail_free(e);
     if ((e = hipMemset(M.gemm_cnt, 0, gcc * sizeof(int))) != hipSuccess)
         return fail_free(e);

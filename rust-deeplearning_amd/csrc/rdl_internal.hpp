@@ -189,8 +189,23 @@ bool combine_is_coherent();
 // True when the current device's next combine runs XCD-local (placement
 // probed and a rotation, switch off); does not probe.
 bool combine_local_now();
+// part: gemm_part_bytes(m, n, k) bytes for the K-slice partials of the tile
+// GEMM (m > GEMM_XTILE_M); NULL (or no counters): that GEMM runs unsplit.
 hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
-                            void* scratch, int* counters, hipStream_t s);
+                            void* scratch, float* part, int* counters, hipStream_t s);
+// True when workgroup b of a launch runs on XCD (b + o) % 8 on the current
+// device (gemm.hip).
+bool xcd_round_robin(hipStream_t s);
+// The tile GEMM (gemm_tiles.hip; arguments as launch_gemm_tiles_ex, k <=
+// GEMM_TILE_MAX_K): its K-slice partials take gemm_part_bytes(m, n, k), at
+// most GEMM_PART_BYTES, and one counter a tile of at most GEMM_SPLIT_TILES.
+constexpr size_t GEMM_TILE_MAX_K = 16384;
+constexpr size_t GEMM_PART_BYTES = 16u << 20;
+constexpr size_t GEMM_SPLIT_TILES = 256;
+size_t gemm_part_bytes(size_t m, size_t n, size_t k);
+hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
+                            void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
+                            hipStream_t s);
 hipError_t launch_gemm_q4_0_native(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                                    int32_t* partials, void* scratch, hipStream_t s);
 // Float-mode products on the LDS tile GEMM, Q4_0 (more than GEMM_XTILE_M
@@ -202,14 +217,15 @@ hipError_t launch_gemm_q4_0_native(const uint8_t* w, size_t n, size_t k, const f
 // residual add) instead of y = product.  scratch: gemm_tiles_scratch_bytes(m,
 // k) bytes (Q4_0 needs only gemm_scratch_bytes(m, n, k, false) of them).
 hipError_t launch_gemm_tiles_ex(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
-                                void* scratch, int pro, const float* g, float eps, bool accumulate, hipStream_t s);
+                                void* scratch, float* part, int* counters, int pro, const float* g, float eps,
+                                bool accumulate, hipStream_t s);
 size_t gemm_tiles_scratch_bytes(size_t m, size_t k);
 // The float-mode product y = x W^T of Q4_K, Q6_K, Q8_0 or Q4_1 weights on
 // the LDS tile GEMM (the reference's dequantize_q4k / dequantize_q6k + F32
 // matmul, parser.rs:510-593; matmul_f32_q8, quantize.rs:201-260;
 // matmul_f32_q4_1, quantize.rs:429-495).
 hipError_t launch_gemm_typed(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
-                             void* scratch, hipStream_t s);
+                             void* scratch, float* part, int* counters, hipStream_t s);
 
 // Decoder fusion of the Q4_0 float-mode fused GEMV (m <= 4, k / 32 even,
 // x 16-byte aligned): prologue 0 none, 1 RMSNorm with weights g and eps,
