@@ -204,16 +204,14 @@ size_t scratch_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k)
     return 0;
 }
 
-// The tile GEMM's K-slice partials (the rest of a product's scratch), and
-// whether the path counts slices: the Q4_0 float GEMMs.
+// The tile GEMM's K-slice partials (beside scratch_bytes).
 size_t part_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
-    return p == Path::Gemm && t == WType::Q4_0 && !native && m > rdl::GEMM_XTILE_M && k <= rdl::GEMM_TILE_MAX_K
-               ? rdl::gemm_part_bytes(m, n, k)
-               : 0;
+    return p == Path::Gemm && !native && rdl::gemm_tile_takes(t, m, n, k) ? rdl::gemm_part_bytes(m, n, k) : 0;
 }
+// Whether the path counts K slices (the Q4_0 x-tile kernel, split tile GEMMs).
 bool wants_counters(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
-    return p == Path::Gemm && t == WType::Q4_0 && !native &&
-           (m <= rdl::GEMM_SMALL_M || part_bytes(t, p, native, m, n, k) > 0);
+    return part_bytes(t, p, native, m, n, k) > 0 ||
+           (p == Path::Gemm && t == WType::Q4_0 && !native && m <= rdl::GEMM_SMALL_M);
 }
 
 // Run the product on `s`; `work` holds scratch_bytes(path) bytes of device

@@ -1842,7 +1842,7 @@ size_t gemm_tiles_scratch_bytes(size_t m, size_t k) {
 hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* tpart, int* counters, hipStream_t s) {
     if (n == 0 || m == 0) return hipSuccess;
-    if (m > GEMM_XTILE_M && k <= GEMM_TILE_MAX_K)
+    if (gemm_tile_takes(WType::Q4_0, m, n, k))
         return launch_gemm_tile(WType::Q4_0, w, n, k, x, m, y, scratch, tpart, counters, 0, nullptr, 0.0f, false, s);
     if (m <= GEMM_XTILE_M) {
         float* part = reinterpret_cast<float*>(scratch);  // the K-slice partials
@@ -1883,7 +1883,7 @@ hipError_t launch_gemm_tiles_ex(WType t, const uint8_t* w, size_t n, size_t k, c
     // 32-bit buffer offsets, out-of-range slots at RSRC_OOB
     const size_t wb = n * (k / block_elems(t)) * block_bytes(t);
     if (wb > FUSED_MAX_WEIGHT_BYTES || m * k * 2 > FUSED_MAX_WEIGHT_BYTES) return hipErrorInvalidValue;
-    if (q40 && k <= GEMM_TILE_MAX_K)
+    if (gemm_tile_takes(t, m, n, k))
         return launch_gemm_tile(t, w, n, k, x, m, y, scratch, part, counters, pro, g, eps, accumulate, s);
     const size_t xb = (m * k * 2 + 255) & ~(size_t)255;
     _Float16* xh = reinterpret_cast<_Float16*>(scratch);

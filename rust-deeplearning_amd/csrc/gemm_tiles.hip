@@ -32,6 +32,7 @@
 // 14336: 30.7 / 73 / 84 -> 25.6 / 44 / 49 us (split over K, below).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "rdl_device.hpp"
@@ -41,9 +42,10 @@ namespace rdl {
 
 namespace {
 
-// K slices of one product: S slices of kbs blocks on tile shape cfg.
+// One product: tile shape cfg, the first `full` tiles whole, the others in S
+// slices of kbs blocks.
 struct TilePlan {
-    int cfg, S, kbs;
+    int cfg, full, S, kbs;
 };
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -168,7 +170,8 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
 // sc1 (device scope).
 constexpr int CPOL_NT = 2, CPOL_SC1 = 16;
 
-constexpr int WF_Q4_0 = 0;
+// Weight formats: Q4_0 (d (q - 8)) and Q8_0 (d q, tensor.rs:535-639).
+constexpr int WF_Q4_0 = 0, WF_Q8_0 = 1;
 
 template <int WF, int FI, int WJ, int KS>
 struct TileCfg {
@@ -176,16 +179,23 @@ struct TileCfg {
     static constexpr int NW = WJ * KS, NT = NW * 64;
     static constexpr int TJ = WJ * 64, TI = FI * 16;
     static constexpr int CB = KS;                // blocks a chunk: one a K group of waves
-    static constexpr int NIB_BLOCK = WJ * 1024;  // bytes of one block's nibbles: [wj][g][64 rows] dwords
+    // one block's codes: [wj][g][64 rows] dwords of nibbles, or (Q8_0) that twice,
+    // bytes 4g .. 4g+3 and 16+4g .. 16+4g+3
+    static constexpr bool BYTES = WF == WF_Q8_0;
+    static constexpr int HALF = WJ * 1024;
+    static constexpr int NIB_BLOCK = (BYTES ? 2 : 1) * HALF;
     static constexpr int W_BYTES = CB * NIB_BLOCK;
-    static constexpr int D_BYTES = CB * TJ * 2;  // f16 d: [block][row]
+    static constexpr int D_BYTES = CB * TJ * 2;    // f16 d: [block][row]
     static constexpr int X_PART = 1024;          // one 16-row tile of one block, hi or lo
     static constexpr int X_BYTES = CB * (TI / 16) * 2 * X_PART;
     static constexpr int STAGE = W_BYTES + D_BYTES + X_BYTES;
+    static constexpr int WWORDS = BYTES ? 9 : 5;            // dwords a weight block's loads bring
     static constexpr int WU = (TJ * CB + NT - 1) / NT;      // weight blocks a thread stages
     static constexpr int XU = (TI * CB * 4 + NT - 1) / NT;  // 16-byte pieces a thread stages, hi and lo each
     static constexpr int RED = (KS - 1) * WJ * FI * FJ * 1024;
-    static constexpr int LDS = 3 * STAGE > RED ? 3 * STAGE : RED;
+    // three stages, or the sums at the end; the x rows' exponents behind them
+    static constexpr int XE_AT = 3 * STAGE > RED ? 3 * STAGE : RED;
+    static constexpr int LDS = XE_AT + TI * 4;
     static constexpr bool W_ALL = TJ * CB % NT == 0;        // no idle threads in the last weight unit
     static_assert(TI * CB * 4 % NT == 0, "whole x pieces a thread");
     static_assert(CB % 2 == 0, "eight consecutive pieces of an x row");
@@ -213,53 +223,70 @@ __device__ __forceinline__ half8_t q4_f16(uint32_t n, const Q4Consts& k) {
     return half8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
+// f16 q of the eight codes n0, n1 (staged as q + 128), in the K order above:
+// 0x6400 | (q + 128) = 1152 + q.
+__device__ __forceinline__ half8_t q8_f16(uint32_t n0, uint32_t n1) {
+    const half2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    constexpr uint32_t MAGIC = 0x64646464u;
+    const half2_t a = __builtin_bit_cast(half2_t, perm(MAGIC, n0, 0x04020400u)) - off;
+    const half2_t b = __builtin_bit_cast(half2_t, perm(MAGIC, n1, 0x04020400u)) - off;
+    const half2_t c = __builtin_bit_cast(half2_t, perm(MAGIC, n0, 0x04030401u)) - off;
+    const half2_t d = __builtin_bit_cast(half2_t, perm(MAGIC, n1, 0x04030401u)) - off;
+    return half8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
 template <int WF, int FI, int WJ, int KS, bool LOCAL>
 __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const uint8_t* __restrict__ W, int n, int nb, const void* __restrict__ XH, const void* __restrict__ XL,
-    const int* __restrict__ XE, int m, float* __restrict__ Y, int accy, int S, int kbs, float* __restrict__ part,
+    const int* __restrict__ XE, int m, float* __restrict__ Y, int accy, int full, int SR, int kbs, float* __restrict__ part,
     int* __restrict__ cnt) {
     using C = TileCfg<WF, FI, WJ, KS>;
     constexpr int CB = C::CB, FJ = 4;
+    constexpr bool BYTES = C::BYTES;
+    constexpr uint32_t BB = BYTES ? 34u : 18u;  // bytes a block
     static_assert(FI == 4 || FI == 8, "x tiles of a wave");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ks = wave % KS, wj = wave / KS;
     const int g = lane >> 4, r = lane & 15;
-    // Workgroups go round-robin to the 8 XCDs.  Unsplit: each XCD takes a
-    // contiguous run of tiles (one L2), four x tiles deep before the next
-    // weight tile.  Split over K: a tile's S slices have one b % 8 (LOCAL: one
-    // XCD, whose L2 holds their partials).
+    // The first `full` tiles (whole rounds of workgroups, or all) are unsplit,
+    // the others take SR slices of kbs blocks.  Workgroups go round-robin to the
+    // 8 XCDs: each XCD takes a contiguous run of the unsplit tiles (one L2),
+    // four x tiles deep before the next weight tile; a split tile's slices have
+    // one b % 8 (LOCAL: one XCD, whose L2 holds their partials; full % 8 == 0).
     const int nj = (n + C::TJ - 1) / C::TJ, ni = (m + C::TI - 1) / C::TI, total = nj * ni;
-    int t = blockIdx.x, slice = 0;
-    if (S > 1) {
+    int t = blockIdx.x, slice = 0, S = 1;
+    if (t < full) {
+        if (full % 8 == 0) t = (t % 8) * (full / 8) + t / 8;
+    } else {
+        const int b = t - full;
+        S = SR;
         if constexpr (LOCAL) {
-            slice = (t / 8) % S;
-            t = t / (8 * S) * 8 + t % 8;
+            slice = (b / 8) % S;
+            t = full + b / (8 * S) * 8 + b % 8;
         } else {
-            slice = t % S;
-            t /= S;
+            slice = b % S;
+            t = full + b / S;
         }
         if (t >= total) return;  // grid rounded up to whole XCD rounds (whole workgroup)
-    } else if (total % 8 == 0) {
-        t = (t % 8) * (total / 8) + t / 8;
     }
     constexpr int GI = 4;
     const int band = t / (GI * nj), rem = t % (GI * nj);
     const int bh = min(GI, ni - band * GI);
     const int j0 = (rem / bh) * C::TJ, i0 = (band * GI + rem % bh) * C::TI;
-    const int kb0 = slice * kbs, kb1 = min(nb, kb0 + kbs);  // this slice's blocks (kb0 a multiple of CB)
+    const int kb0 = slice * kbs, kb1 = S > 1 ? min(nb, kb0 + kbs) : nb;  // this slice's blocks (kb0 a multiple of CB)
 
-    const uint32_t k = (uint32_t)nb * 32u, row_bytes = (uint32_t)nb * 18u, wbytes = (uint32_t)n * row_bytes;
+    const uint32_t k = (uint32_t)nb * 32u, row_bytes = (uint32_t)nb * BB, wbytes = (uint32_t)n * row_bytes;
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(W, wbytes);
     const __amdgpu_buffer_rsrc_t hrs = make_rsrc(XH, (uint32_t)m * k * 2u);
     const __amdgpu_buffer_rsrc_t lrs = make_rsrc(XL, (uint32_t)m * k * 2u);
     const int nchunks = (kb1 - kb0 + CB - 1) / CB;
 
-    struct WRegs { uint32_t w[C::WU][5]; };
+    struct WRegs { uint32_t w[C::WU][C::WWORDS]; };
     struct XRegs { u32x4 h[C::XU], l[C::XU]; };
-    // unit u of a thread: block b0 + c CB of row j; CB is even, so a block's
-    // place within its dword (2 bytes past it when j nb + b is odd) is the same
-    // in every chunk.  Rows past n start out of range.
+    // unit u of a thread: block b0 + c CB of row j; CB is even, so a Q4_0 or Q8_0
+    // block's place within its dword (2 bytes past it when j nb + b is odd) is
+    // the same in every chunk.  Rows past n start out of range.
     uint32_t wbase[C::WU], wsel[C::WU];
     int wblk[C::WU];
 #pragma unroll
@@ -267,7 +294,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         const int idx = tid + u * C::NT, j = j0 + idx / CB;
         wblk[u] = idx % CB;
         const bool ok = (C::W_ALL || idx < C::TJ * CB) && j < n;
-        wbase[u] = ok ? ((uint32_t)j * row_bytes + (uint32_t)(kb0 + wblk[u]) * 18u) & ~3u : RSRC_OOB;
+        wbase[u] = ok ? ((uint32_t)j * row_bytes + (uint32_t)(kb0 + wblk[u]) * BB) & ~3u : RSRC_OOB;
         wsel[u] = (((uint32_t)j * (uint32_t)nb + (uint32_t)wblk[u]) & 1u) ? 0x07060504u : 0x05040302u;
     }
     // the matrix may end 2 bytes into a window's last dword: that dword is read
@@ -276,12 +303,21 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     auto load_w = [&](int c, WRegs& R) {
 #pragma unroll
         for (int u = 0; u < C::WU; u++) {
-            const uint32_t base = kb0 + wblk[u] + c * CB < kb1 ? wbase[u] + (uint32_t)c * (CB * 18u) : RSRC_OOB;
+            const uint32_t base = kb0 + wblk[u] + c * CB < kb1 ? wbase[u] + (uint32_t)c * (CB * BB) : RSRC_OOB;
             const u32x4 v = buf_load_b128(wrs, base);
             R.w[u][0] = v.x, R.w[u][1] = v.y, R.w[u][2] = v.z, R.w[u][3] = v.w;
-            R.w[u][4] = buf_load_b32(wrs, min(base + 16u, wlast));
+            if constexpr (BYTES) {
+                const u32x4 v1 = buf_load_b128(wrs, base == RSRC_OOB ? RSRC_OOB : base + 16u);
+                R.w[u][4] = v1.x, R.w[u][5] = v1.y, R.w[u][6] = v1.z, R.w[u][7] = v1.w;
+                R.w[u][8] = buf_load_b32(wrs, min(base + 32u, wlast));
+            } else {
+                R.w[u][4] = buf_load_b32(wrs, min(base + 16u, wlast));
+            }
         }
     };
+    int* const xe = reinterpret_cast<int*>(lds + C::XE_AT);
+    if (tid < C::TI) xe[tid] = i0 + tid < m ? XE[i0 + tid] : 0;
+
     uint32_t xbase[C::XU];
 #pragma unroll
     for (int u = 0; u < C::XU; u++) {
@@ -304,13 +340,19 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         for (int u = 0; u < C::WU; u++) {
             const int idx = tid + u * C::NT, jl = idx / CB, bl = idx % CB;
             if (!C::W_ALL && idx >= C::TJ * CB) continue;
-            const uint32_t end = wbase[u] + (uint32_t)c * (CB * 18u) + 16u;
-            const uint32_t w4 = end > wlast ? R.w[u][4] >> 16 : R.w[u][4];
+            const uint32_t end = wbase[u] + (uint32_t)c * (CB * BB) + (BYTES ? 32u : 16u);
+            const uint32_t tail = R.w[u][C::WWORDS - 1];
+            const uint32_t wt = end > wlast ? tail >> 16 : tail;
             uint32_t* dst = reinterpret_cast<uint32_t*>(st + bl * C::NIB_BLOCK + (jl >> 6) * 1024) + (jl & 63);
-            dst[0] = perm(R.w[u][1], R.w[u][0], wsel[u]);
-            dst[64] = perm(R.w[u][2], R.w[u][1], wsel[u]);
-            dst[128] = perm(R.w[u][3], R.w[u][2], wsel[u]);
-            dst[192] = perm(w4, R.w[u][3], wsel[u]);
+            if constexpr (BYTES) {
+#pragma unroll
+                for (int q = 0; q < 8; q++)
+                    dst[(q & 3) * 64 + (q >> 2) * (C::HALF / 4)] =
+                        perm(q == 7 ? wt : R.w[u][q + 1], R.w[u][q], wsel[u]) ^ 0x80808080u;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; q++) dst[q * 64] = perm(q == 3 ? wt : R.w[u][q + 1], R.w[u][q], wsel[u]);
+            }
             uint16_t* wd = reinterpret_cast<uint16_t*>(st + C::W_BYTES);
             wd[bl * C::TJ + jl] = (uint16_t)(R.w[u][0] >> ((wsel[u] & 2u) << 3 ^ 16u));
         }
@@ -345,7 +387,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // Past the end every load reads zeros (x 0, d 0).
     constexpr int RB = FI / 2;
     const Q4Consts qc = q4_consts();
-    u32x4 nv;
+    u32x4 nv, nv2;    // codes of the next block (nv2: Q8_0's second half)
     uint2 dd;
     half8_t wq[2][4];
     float dv[2][4];
@@ -353,6 +395,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     f32x4 p[2][FJ];
     auto read_w = [&](const uint8_t* st) {
         nv = *reinterpret_cast<const u32x4*>(st + ks * C::NIB_BLOCK + wj * 1024 + g * 256 + r * 16);
+        if constexpr (BYTES)
+            nv2 = *reinterpret_cast<const u32x4*>(st + ks * C::NIB_BLOCK + C::HALF + wj * 1024 + g * 256 + r * 16);
         dd = *reinterpret_cast<const uint2*>(st + C::W_BYTES + (ks * C::TJ + wj * 64 + r * 4) * 2);
     };
     auto read_x = [&](const uint8_t* st, int s) {
@@ -362,7 +406,13 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         xl[s & 1] = *reinterpret_cast<const half8_t*>(xb + C::X_PART);
     };
     auto conv = [&](int o, int a) {
-        wq[o][a] = q4_f16(a == 0 ? nv.x : a == 1 ? nv.y : a == 2 ? nv.z : nv.w, qc);
+        const uint32_t n0 = a == 0 ? nv.x : a == 1 ? nv.y : a == 2 ? nv.z : nv.w;
+        if constexpr (BYTES) {
+            const uint32_t n1 = a == 0 ? nv2.x : a == 1 ? nv2.y : a == 2 ? nv2.z : nv2.w;
+            wq[o][a] = q8_f16(n0, n1);
+        } else {
+            wq[o][a] = q4_f16(n0, qc);
+        }
         dv[o][a] = h2f(a == 0 ? dd.x & 0xFFFFu : a == 1 ? dd.x >> 16 : a == 2 ? dd.y & 0xFFFFu : dd.y >> 16);
         // f32 here once a block: left to itself the compiler folds the conversion
         // into every scale FMA (v_fma_mix_f32: 1,240 against 546 us, 2048 x 14336 x 4096)
@@ -374,7 +424,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
 #pragma unroll
             for (int u = 0; u < 4; u++) acc[b][a][u] = fmaf(dv[o][a], p[ps][a][u], acc[b][a][u]);
     };
-    constexpr int DX = FI == 8 ? 1 : 2, DW = 2;  // chunks the loads run ahead (FI 8: no registers for x two ahead)
+    // chunks the loads run ahead (FI 8: no registers for more)
+    constexpr int DX = FI == 8 ? 1 : 2, DW = FI == 8 && BYTES ? 1 : 2;
     WRegs w[DW];
     XRegs x1[DX];
     uint8_t *bc = lds, *bn = lds + C::STAGE, *bf = lds + 2 * C::STAGE;  // chunk c, c + 1, free
@@ -426,8 +477,9 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
 #pragma unroll
     for (int q = 0; q < DW; q++) {
         load_w(q, w[q]);
-        if (q < DX) load_x(q, x1[q]);
     }
+#pragma unroll
+    for (int q = 0; q < DX; q++) load_x(q, x1[q]);
     store_w(0, bc, w[0]);
     store_x(bc, x1[0]);
     load_w(DW, w[0]);
@@ -442,7 +494,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         p[1][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
     // (chunks past the slice's end: zeros; no branch, so that the waits stay exact)
-    for (int c = 0; c < nchunks; c += DW) {
+    for (int c = 0; c < nchunks; c += 2) {
         chunk(c, std::integral_constant<int, 0>{});
         chunk(c + 1, std::integral_constant<int, 1>{});
     }
@@ -455,7 +507,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         for (int u = 0; u < 4; u++) {
             const int i = i0 + b * 16 + g * 4 + u;
             if (i >= m) continue;
-            const int e = XE[i];
+            const int e = xe[i - i0];
             f32x4 v = {ldexpf(v4[0][u], e), ldexpf(v4[1][u], e), ldexpf(v4[2][u], e), ldexpf(v4[3][u], e)};
             float* yp = Y + (size_t)i * n + j;
             // accy: y += the product (the residual add, one rounding as x + y)
@@ -509,7 +561,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // ---- slices of the tile: partials, counter, the last one adds them in slice order
     if (S > 1) {
         constexpr int UNITS = C::NW * FO * FJ * 64;  // f32x4 results of a tile
-        const __amdgpu_buffer_rsrc_t prs = make_rsrc(part + (size_t)t * S * UNITS * 4, (uint32_t)S * UNITS * 16u);
+        const __amdgpu_buffer_rsrc_t prs = make_rsrc(part + (size_t)(t - full) * S * UNITS * 4, (uint32_t)S * UNITS * 16u);
         const uint32_t u0 = (uint32_t)wave * (FO * FJ * 64) + lane;
 #pragma unroll
         for (int b = 0; b < FO; b++)
@@ -523,9 +575,9 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         int* last_sh = reinterpret_cast<int*>(lds);
         if (tid == 0) {
             constexpr int SCOPE = LOCAL ? __HIP_MEMORY_SCOPE_WORKGROUP : __HIP_MEMORY_SCOPE_AGENT;
-            const int old = __hip_atomic_fetch_add(cnt + t, 1, __ATOMIC_RELAXED, SCOPE);
+            const int old = __hip_atomic_fetch_add(cnt + t - full, 1, __ATOMIC_RELAXED, SCOPE);
             *last_sh = old == S - 1;
-            if (old == S - 1) __hip_atomic_store(cnt + t, 0, __ATOMIC_RELAXED, SCOPE);
+            if (old == S - 1) __hip_atomic_store(cnt + t - full, 0, __ATOMIC_RELAXED, SCOPE);
         }
         __syncthreads();
         if (!*last_sh) return;
@@ -559,11 +611,24 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     for (int b = 0; b < FO; b++) store_rows(ks * FO + b, own[b]);
 }
 
+// x split of one product in the scratch (gemm_tiles_scratch_bytes(m, k)).
+struct XSplit {
+    _Float16 *h, *l;
+    int* e;
+    float* s;  // x' sums of each block, or NULL
+};
+XSplit x_split_at(void* scratch, size_t m, size_t k, bool sums) {
+    const size_t xb = (m * k * 2 + 255) & ~(size_t)255, eb = (m * 4 + 255) & ~(size_t)255;
+    uint8_t* p = reinterpret_cast<uint8_t*>(scratch);
+    return {reinterpret_cast<_Float16*>(p), reinterpret_cast<_Float16*>(p + xb), reinterpret_cast<int*>(p + 2 * xb),
+            sums ? reinterpret_cast<float*>(p + 2 * xb + eb) : nullptr};
+}
+
 // One tile shape: 64 WJ weight rows x 16 FI x rows, KS wave groups sharing
 // each chunk's blocks.
 template <int WF, int FI, int WJ, int KS>
-hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const void* xh, const void* xl, const int* xe, int m,
-                           float* y, int accy, const TilePlan& p, float* part, int* cnt, hipStream_t s) {
+hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const XSplit& x, int m, float* y, int accy,
+                           const TilePlan& p, float* part, int* cnt, hipStream_t s) {
     using C = TileCfg<WF, FI, WJ, KS>;
     static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
     const bool local = p.S > 1 && xcd_round_robin(s);
@@ -576,10 +641,10 @@ hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const void* xh, cons
                                 hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS)};  // once a process
         if (e[local] != hipSuccess) return e[local];
     }
-    unsigned tiles = (unsigned)((n + C::TJ - 1) / C::TJ) * (unsigned)((m + C::TI - 1) / C::TI);
-    if (local) tiles = (tiles + 7) / 8 * 8;
-    launch_kernel(kern, dim3(tiles * (unsigned)p.S), dim3(C::NT), (size_t)C::LDS, s, w, n, nb, xh, xl, xe, m, y, accy,
-                  p.S, p.kbs, part, cnt);
+    unsigned rest = (unsigned)((n + C::TJ - 1) / C::TJ) * (unsigned)((m + C::TI - 1) / C::TI) - (unsigned)p.full;
+    if (local) rest = (rest + 7) / 8 * 8;
+    launch_kernel(kern, dim3((unsigned)p.full + rest * (unsigned)p.S), dim3(C::NT), (size_t)C::LDS, s, w, n, nb, x.h, x.l, x.e, m, y,
+                  accy, p.full, p.S, p.kbs, part, cnt);
     return hipGetLastError();
 }
 
@@ -592,87 +657,103 @@ struct TileShape {
 };
 constexpr TileShape TILE_SHAPES[4] = {{256, 128, 2, 0.90}, {256, 64, 2, 0.50}, {128, 64, 4, 0.29}, {64, 64, 4, 0.26}};
 
-// Tile shape and K slices of a product by estimated time: rounds of
-// workgroups times a slice's blocks, plus, split, the last slice's reading of
-// the others' partials (about 40 KB a us; 2 us for the stores and the
-// counter).  Against sweeps over shapes and slices at 80-2048 rows, n = 1024
-// .. 28672, k = 4096 and 14336 the choice was the best or within 5 % of it:
-// at 128 rows 4096 x 4096 64 tiles of 128 x 64 in 4 slices (25.6 us; unsplit
-// 40.4, 2 slices 28.7, 8 slices 36.2), 14336 x 4096 the same tiles unsplit
-// (44 us; 256 x 128 117, 64 x 64 67), 512 rows 14336 x 4096 256 x 128 (127
-// us; 256 x 64 162).
+// Tile shape and K slices of a product by estimated time.  Whole rounds of
+// one workgroup a CU run unsplit; the tiles past them are split over K, where
+// that is estimated to pay, into up to as many slices as fill a round.  Time:
+// a round's blocks, plus, split, the last slice's reading of the others'
+// partials (about 40 KB a us; 2 us for the stores and the counter).  Against
+// sweeps over shapes and slices at 80-2048 rows, n = 1024 .. 28672, k = 4096
+// and 14336 the choice was the best or within 5 % of it: at 128 rows 4096 x
+// 4096 64 tiles of 128 x 64 in 4 slices (25.6 us; unsplit 40.4, 2 slices 28.7,
+// 8 slices 36.2), 14336 x 4096 the same tiles unsplit (44 us; 256 x 128 117,
+// 64 x 64 67), 512 rows 14336 x 4096 256 x 128 (127 us; 256 x 64 162).
 TilePlan tile_plan(size_t m, size_t n, size_t nb, bool can_split) {
-    const int cus = device_cu_count();
+    const size_t round = std::max(8, device_cu_count() / 8 * 8);
     TilePlan best{};
     double best_us = 1e30;
     for (int c = 0; c < 4; c++) {
         const TileShape& t = TILE_SHAPES[c];
         const size_t tiles = ((n + t.tj - 1) / t.tj) * ((m + t.ti - 1) / t.ti);
         const size_t unit = 2 * (size_t)t.ks;  // the main loop's step: two chunks
-        for (size_t S = 1; S <= 16; S *= 2) {
+        const size_t full = tiles / round * round, rest = tiles - full;
+        const double whole = nb * t.us_block + 6.0;  // us a round of unsplit tiles
+        for (size_t S = 1; S <= 16; S++) {
             const size_t kbs = ((nb + S - 1) / S + unit - 1) / unit * unit;
-            if (S > 1) {
-                if (!can_split || tiles > GEMM_SPLIT_TILES || (S - 1) * kbs >= nb) break;  // (no empty slice)
-                if (tiles * S * t.tj * t.ti * sizeof(float) > GEMM_PART_BYTES) break;
+            double us = (double)(full / round) * whole;
+            if (S == 1) {
+                us += rest ? whole : 0.0;
+            } else {
+                if (!can_split || rest * S > round) break;
+                if ((S - 1) * kbs >= nb) continue;  // (an empty slice)
+                const size_t bytes = S * t.tj * t.ti * sizeof(float);
+                if (rest == 0 || rest * bytes > GEMM_PART_BYTES) break;
+                us += kbs * t.us_block + 6.0 + 2.0 + (double)bytes / 40e3;
             }
-            const size_t rounds = (tiles * S + cus - 1) / cus;
-            const double us = (double)rounds * (kbs * t.us_block + 6.0) +
-                              (S > 1 ? 2.0 + (double)(S * t.tj * t.ti * sizeof(float)) / 40e3 : 0.0);
-            if (us < best_us) best_us = us, best = {c, (int)S, (int)kbs};
+            if (us < best_us) best_us = us, best = {c, (int)(S == 1 ? tiles : full), (int)S, (int)kbs};
         }
     }
     return best;
 }
 
-// x split of one product into the scratch (gemm_split_bytes(m, k)).
-struct XSplit {
-    _Float16 *h, *l;
-    int* e;
-};
-XSplit x_split_at(void* scratch, size_t m, size_t k) {
-    const size_t xb = (m * k * 2 + 255) & ~(size_t)255;
-    uint8_t* p = reinterpret_cast<uint8_t*>(scratch);
-    return {reinterpret_cast<_Float16*>(p), reinterpret_cast<_Float16*>(p + xb), reinterpret_cast<int*>(p + 2 * xb)};
-}
-
 template <int PRO>
-hipError_t launch_split(const float* x, size_t m, size_t k, const float* g, float eps, const XSplit& o, float* xs,
-                        hipStream_t s) {
+hipError_t launch_split(const float* x, size_t m, size_t k, const float* g, float eps, const XSplit& o, hipStream_t s) {
     // 256 threads hold 4096 elements of a row, 1024 threads 16384
     if (k <= 4096)
         launch_kernel(gemm_split_kernel<PRO, 256, 4>, dim3((unsigned)m), dim3(256), 0, s, x, (int)k, g, eps, o.h, o.l,
-                      o.e, xs);
+                      o.e, o.s);
     else
         launch_kernel(gemm_split_kernel<PRO, 1024, 4>, dim3((unsigned)m), dim3(1024), 0, s, x, (int)k, g, eps, o.h,
-                      o.l, o.e, xs);
+                      o.l, o.e, o.s);
     return hipGetLastError();
 }
 
 }  // namespace
 
+// The small-tile kernel of gemm.hip keeps short products over small matrices:
+// its 16 x 32 tiles reach all CUs without a split over K, and its code is
+// smaller (us, here against there: Q4_0 100 x 512 x 992 10.7 / 9.1, 200 x 2048 x
+// 992 13.6 / 12.7, 100 x 2048 x 2048 14.2 / 15.8, 100 x 64 x 4096 13.4 / 17.3;
+// Q8_0 100 x 512 x 992 11.0 / 8.9, 1000 x 512 x 992 17.5 / 16.4, 333 x 4096 x 992
+// 19.5 / 25.7, 17 x 4096 x 4096 17.9 / 17.2, 33 x 4096 x 4096 18.6 / 24.4).
+bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k) {
+    if (k > GEMM_TILE_MAX_K) return false;
+    if (t == WType::Q4_0) return m > GEMM_XTILE_M && !(m <= 256 && k <= 2048 && n * k <= (size_t)1 << 22);
+    if (t != WType::Q8_0 || m < KQ_GEMM_MIN_M) return false;
+    if (k <= 2048 && (m * n <= (size_t)1 << 19 || (m <= 256 && n * k <= (size_t)1 << 23))) return false;
+    return m > 24 || n * k > (size_t)1 << 24;
+}
+
 size_t gemm_part_bytes(size_t m, size_t n, size_t k) {
     const TilePlan p = tile_plan(m, n, k / QK, true);
     const TileShape& t = TILE_SHAPES[p.cfg];
-    return p.S > 1 ? ((n + t.tj - 1) / t.tj) * ((m + t.ti - 1) / t.ti) * p.S * t.tj * t.ti * sizeof(float) : 0;
+    const size_t rest = ((n + t.tj - 1) / t.tj) * ((m + t.ti - 1) / t.ti) - (size_t)p.full;
+    return rest * p.S * t.tj * t.ti * sizeof(float);
+}
+
+template <int WF>
+static hipError_t launch_tile_wf(const uint8_t* w, int n, int nb, const XSplit& x, int m, float* y, int accy,
+                                 float* part, int* cnt, hipStream_t s) {
+    const TilePlan p = tile_plan(m, n, nb, part != nullptr && cnt != nullptr);
+    switch (p.cfg) {
+        case 0: return launch_tile_cfg<WF, 8, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+        case 1: return launch_tile_cfg<WF, 4, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+        case 2: return launch_tile_cfg<WF, 4, 2, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+        default: return launch_tile_cfg<WF, 4, 1, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+    }
 }
 
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
                             hipStream_t s) {
-    if (t != WType::Q4_0 || k == 0 || k > GEMM_TILE_MAX_K) return hipErrorInvalidValue;
-    const XSplit xo = x_split_at(scratch, m, k);
-    hipError_t e = pro == 1   ? launch_split<1>(x, m, k, g, eps, xo, nullptr, s)
-                   : pro == 2 ? launch_split<2>(x, m, k, g, eps, xo, nullptr, s)
-                              : launch_split<0>(x, m, k, g, eps, xo, nullptr, s);
+    if (k == 0 || !gemm_tile_takes(t, m, n, k)) return hipErrorInvalidValue;
+    const XSplit xo = x_split_at(scratch, m, k, false);
+    const hipError_t e = pro == 1   ? launch_split<1>(x, m, k, g, eps, xo, s)
+                         : pro == 2 ? launch_split<2>(x, m, k, g, eps, xo, s)
+                                    : launch_split<0>(x, m, k, g, eps, xo, s);
     if (e != hipSuccess) return e;
     const int ni = (int)n, nb = (int)(k / QK), mi = (int)m, acc = accumulate ? 1 : 0;
-    const TilePlan p = tile_plan(m, n, nb, part != nullptr && cnt != nullptr);
-    switch (p.cfg) {
-        case 0: return launch_tile_cfg<WF_Q4_0, 8, 4, 2>(w, ni, nb, xo.h, xo.l, xo.e, mi, y, acc, p, part, cnt, s);
-        case 1: return launch_tile_cfg<WF_Q4_0, 4, 4, 2>(w, ni, nb, xo.h, xo.l, xo.e, mi, y, acc, p, part, cnt, s);
-        case 2: return launch_tile_cfg<WF_Q4_0, 4, 2, 4>(w, ni, nb, xo.h, xo.l, xo.e, mi, y, acc, p, part, cnt, s);
-        default: return launch_tile_cfg<WF_Q4_0, 4, 1, 4>(w, ni, nb, xo.h, xo.l, xo.e, mi, y, acc, p, part, cnt, s);
-    }
+    return t == WType::Q4_0 ? launch_tile_wf<WF_Q4_0>(w, ni, nb, xo, mi, y, acc, part, cnt, s)
+                            : launch_tile_wf<WF_Q8_0>(w, ni, nb, xo, mi, y, acc, part, cnt, s);
 }
 
 }  // namespace rdl

@@ -203,6 +203,10 @@ constexpr size_t GEMM_TILE_MAX_K = 16384;
 constexpr size_t GEMM_PART_BYTES = 16u << 20;
 constexpr size_t GEMM_SPLIT_TILES = 256;
 size_t gemm_part_bytes(size_t m, size_t n, size_t k);
+// Whether a float-mode product takes the tile GEMM (Q4_0 beyond GEMM_XTILE_M
+// rows, Q8_0 from KQ_GEMM_MIN_M): where it is faster than the small-tile
+// kernel of gemm.hip.
+bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k);
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
                             hipStream_t s);

@@ -13,19 +13,21 @@ pytestmark = pytest.mark.gpu
 # weight tile, odd block counts (blocks 2 bytes past a dword, the matrix ending
 # inside one), K in 16 / 8 / 4 / 2 slices with a ragged last one, 256 x 128 tiles,
 # and rows longer than one workgroup's registers hold (k > 16384)
-SHAPES = [(65, 1, 32), (65, 65, 96), (129, 63, 1056), (128, 1024, 4096), (66, 200, 4128), (80, 4096, 2080),
-          (130, 6000, 544), (200, 14400, 96), (513, 4097, 288), (70, 40, 16416)]
+# (the rows before 257 with k <= 2048 stay on the small-tile kernel)
+SHAPES = [(65, 1, 32), (65, 1, 4096), (65, 65, 2080), (129, 63, 4128), (128, 1024, 4096), (80, 4096, 2080),
+          (257, 130, 96), (257, 6000, 544), (300, 14400, 96), (513, 4097, 288), (2049, 65, 32), (70, 40, 16416)]
 
 
+@pytest.mark.parametrize("kind,dtype", [("q4", 2), ("q8", 8)])
 @pytest.mark.parametrize("m,n,k", SHAPES)
-def test_q4_0_tiles(rq, orc, gpu, m, n, k):
-    print(f"case q4_0 tiles m={m} n={n} k={k}", flush=True)
+def test_tiles(rq, orc, gpu, kind, dtype, m, n, k):
+    print(f"case {kind} tiles m={m} n={n} k={k}", flush=True)
     x = synth.activations(m, k, m + n + k)
-    w = synth.q4_0_weights(n, k, m + n)
-    got = rq.matmul_f32_q4(x, w, m, k, n).reshape(m, n)
+    w = synth.weights(dtype, n, k, m + n)
+    got = getattr(rq, f"matmul_f32_{kind}")(x, w, m, k, n).reshape(m, n)
     rows = np.unique(np.linspace(0, m - 1, 24).astype(int))
-    want = orc.matmul("q4", x[rows], w, len(rows), k, n, threads=16)
-    check_parity(got[rows].reshape(-1), want, exact_f64(orc, "q4", x[rows], w, len(rows), k, n))
+    want = orc.matmul(kind, x[rows], w, len(rows), k, n, threads=16)
+    check_parity(got[rows].reshape(-1), want, exact_f64(orc, kind, x[rows], w, len(rows), k, n))
 
 
 @pytest.mark.parametrize("m,n,k", [(128, 1024, 4096), (100, 4096, 1024)])
