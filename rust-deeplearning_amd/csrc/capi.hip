@@ -206,7 +206,7 @@ size_t scratch_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k)
 
 // The tile GEMM's K-slice partials (beside scratch_bytes).
 size_t part_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
-    return p == Path::Gemm && !native && rdl::gemm_tile_takes(t, m, n, k) ? rdl::gemm_part_bytes(m, n, k) : 0;
+    return p == Path::Gemm && !native && rdl::gemm_tile_takes(t, m, n, k) ? rdl::gemm_part_bytes(t, m, n, k) : 0;
 }
 // Whether the path counts K slices (the Q4_0 x-tile kernel, split tile GEMMs).
 bool wants_counters(WType t, Path p, bool native, size_t m, size_t n, size_t k) {

@@ -60,7 +60,7 @@ template <int PRO, int NT, int NV>
 __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict__ X, int k,
                                                         const float* __restrict__ g, float eps,
                                                         _Float16* __restrict__ XH, _Float16* __restrict__ XL,
-                                                        int* __restrict__ XE, float* __restrict__ XS) {
+                                                        int* __restrict__ XE, uint32_t* __restrict__ XS) {
     __shared__ float red[NT / 64], red2[NT / 64];
     const int row = blockIdx.x;
     const int k4 = k >> 2;  // k % 32 == 0
@@ -158,9 +158,12 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
             _Float16* dst = (upper ? XL : XH) + (size_t)row * k + (size_t)(p >> 3) * 32 + (p & 3) * 8;
             *reinterpret_cast<u32x4*>(dst) = o;
         }
-        if (XS) {  // the block's f32 sum of x'
-            bs = sum8_f32(bs);
-            if ((threadIdx.x & 7) == 0 && p < k4) XS[(size_t)row * (k >> 5) + (p >> 3)] = bs;
+        if (XS) {  // the block's sum of x', over 32, as an f16 hi / lo pair
+            bs = sum8_f32(bs) * 0.03125f;
+            const _Float16 sh = (_Float16)bs;
+            const half2_t sp = {sh, (_Float16)(bs - (float)sh)};
+            if ((threadIdx.x & 7) == 0 && p < k4)
+                XS[(size_t)row * (k >> 5) + (p >> 3)] = __builtin_bit_cast(uint32_t, sp);
         }
     }
 }
@@ -170,8 +173,23 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
 // sc1 (device scope).
 constexpr int CPOL_NT = 2, CPOL_SC1 = 16;
 
-// Weight formats: Q4_0 (d (q - 8)) and Q8_0 (d q, tensor.rs:535-639).
-constexpr int WF_Q4_0 = 0, WF_Q8_0 = 1;
+// Weight formats: Q4_0 (d (q - 8)) and Q8_0 (d q, tensor.rs:535-639), whose
+// blocks have f16 scales of their own; Q4_K ((d sc) q - dmin mn, parser.rs:
+// 549-593) and Q6_K ((d sc) (q - 32), parser.rs:510-547), whose 256-element
+// super-blocks have one f16 scale over small integer ones.  There the integer
+// scale goes into the operand and the MFMAs of a super-block chain in their
+// accumulators, T: acc += d T once a super-block instead of one FMA an output
+// a block.
+//  * Q4_K: (q - 8) sc is exact in f16.  What remains, e_j = 8 d sc_j - dmin
+//    mn_j times S_j, the sum of x' over sub-block j, is one more MFMA a
+//    super-block: eight sub-blocks times the four products of the f16 hi / lo
+//    pairs of e_j 2^-t (t by the row's larger of 8 d, dmin) and of S_j / 32.
+//    (e_j first, in f32: d q sc and dmin mn nearly cancel, and summing them
+//    apart doubled the error against 64 bits.)
+//  * Q6_K: (q - 32) sc has up to 13 bits: hi = f16(.) and the exact rest lo (at
+//    most 1 in 4096), T += x_hi hi + x_lo hi + x_hi lo (x_lo lo < 2^-23 of a
+//    product, below x's own split).
+constexpr int WF_Q4_0 = 0, WF_Q8_0 = 1, WF_Q4_K = 2, WF_Q6_K = 3;
 
 template <int WF, int FI, int WJ, int KS>
 struct TileCfg {
@@ -181,21 +199,32 @@ struct TileCfg {
     static constexpr int CB = KS;                // blocks a chunk: one a K group of waves
     // one block's codes: [wj][g][64 rows] dwords of nibbles, or (Q8_0) that twice,
     // bytes 4g .. 4g+3 and 16+4g .. 16+4g+3
-    static constexpr bool BYTES = WF == WF_Q8_0;
+    static constexpr bool BYTES = WF == WF_Q8_0 || WF == WF_Q6_K;
+    static constexpr bool CHAIN = WF == WF_Q4_K || WF == WF_Q6_K;
+    static_assert(WF != WF_Q6_K || KS == 4, "Q6_K chunks are half super-blocks");
     static constexpr int HALF = WJ * 1024;
     static constexpr int NIB_BLOCK = (BYTES ? 2 : 1) * HALF;
     static constexpr int W_BYTES = CB * NIB_BLOCK;
-    static constexpr int D_BYTES = CB * TJ * 2;    // f16 d: [block][row]
+    // f16 d (Q4_K: sc; Q6_K: the pair of its two 16-element scales): [block][row]
+    static constexpr int D_BYTES = CB * TJ * (WF == WF_Q6_K ? 4 : 2);
     static constexpr int X_PART = 1024;          // one 16-row tile of one block, hi or lo
     static constexpr int X_BYTES = CB * (TI / 16) * 2 * X_PART;
     static constexpr int STAGE = W_BYTES + D_BYTES + X_BYTES;
-    static constexpr int WWORDS = BYTES ? 9 : 5;            // dwords a weight block's loads bring
+    static constexpr int WWORDS = WF == WF_Q6_K ? 11 : WF == WF_Q4_K ? 8 : BYTES ? 9 : 5;  // dwords a unit's loads bring
     static constexpr int WU = (TJ * CB + NT - 1) / NT;      // weight blocks a thread stages
     static constexpr int XU = (TI * CB * 4 + NT - 1) / NT;  // 16-byte pieces a thread stages, hi and lo each
     static constexpr int RED = (KS - 1) * WJ * FI * FJ * 1024;
-    // three stages, or the sums at the end; the x rows' exponents behind them
-    static constexpr int XE_AT = 3 * STAGE > RED ? 3 * STAGE : RED;
-    static constexpr int LDS = XE_AT + TI * 4;
+    // a super-block's own data (CHAIN): d (and Q4_K's t) of each row, Q4_K's e
+    // [row][hi / lo][8] f16 and x sums [tile][hi / lo][16 rows][8] f16
+    static constexpr int SU = WF == WF_Q4_K ? (TI * CB + NT - 1) / NT : 0;  // sum pairs a thread stages
+    static constexpr int MN_AT = TJ * 4, SS_AT = MN_AT + TJ * 32;
+    static constexpr int AUX = !CHAIN ? 0 : WF == WF_Q4_K ? SS_AT + TI * 32 : MN_AT;
+    // three stages and three super-blocks' data, or the sums at the end; the x
+    // rows' exponents behind them
+    static constexpr int AUX_AT = 3 * STAGE, MAIN = 3 * STAGE + 3 * AUX;
+    static constexpr int XE_AT = MAIN > RED ? MAIN : RED;
+    static constexpr int DUMP_AT = XE_AT + TI * 4;  // where threads without a sum pair store
+    static constexpr int LDS = DUMP_AT + (WF == WF_Q4_K ? 272 : 0);
     static constexpr bool W_ALL = TJ * CB % NT == 0;        // no idle threads in the last weight unit
     static_assert(TI * CB * 4 % NT == 0, "whole x pieces a thread");
     static_assert(CB % 2 == 0, "eight consecutive pieces of an x row");
@@ -235,18 +264,47 @@ __device__ __forceinline__ half8_t q8_f16(uint32_t n0, uint32_t n1) {
     return half8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
+// f16 (q - 8) sc of eight Q4_K nibbles (bytes 4g .. in n0, 16+4g .. in n1;
+// mask picks the low or the high ones, whose 0x6400 | 16 q takes mul 1 / 16, off
+// -72 to q - 8 where the low ones take 1 and -1032); exact.
+__device__ __forceinline__ half8_t q4k_f16(uint32_t n0, uint32_t n1, uint32_t mask, uint32_t magic, half2_t mul,
+                                           half2_t off, _Float16 sc) {
+    const half2_t s2 = {sc, sc};
+    const half2_t a = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, (n0 & mask) | magic), mul, off) * s2;
+    const half2_t b = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, (n1 & mask) | magic), mul, off) * s2;
+    const half2_t c = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, ((n0 >> 8) & mask) | magic), mul, off) * s2;
+    const half2_t d = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, ((n1 >> 8) & mask) | magic), mul, off) * s2;
+    return half8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+// hi and lo of (q - 32) sc for eight Q6_K codes (n0: sub-block 0, n1: 1).
+__device__ __forceinline__ void q6k_f16(uint32_t n0, uint32_t n1, uint32_t scales, half8_t& hi, half8_t& lo) {
+    const half2_t off = {(_Float16)1056.0f, (_Float16)1056.0f};
+    const half2_t sp = __builtin_bit_cast(half2_t, scales);
+    const half2_t s0 = {sp[0], sp[0]}, s1 = {sp[1], sp[1]};
+    constexpr uint32_t MAGIC = 0x64646464u;
+    const half2_t q0 = __builtin_bit_cast(half2_t, perm(MAGIC, n0, 0x04020400u)) - off;
+    const half2_t q1 = __builtin_bit_cast(half2_t, perm(MAGIC, n1, 0x04020400u)) - off;
+    const half2_t q2 = __builtin_bit_cast(half2_t, perm(MAGIC, n0, 0x04030401u)) - off;
+    const half2_t q3 = __builtin_bit_cast(half2_t, perm(MAGIC, n1, 0x04030401u)) - off;
+    const half2_t h0 = q0 * s0, h1 = q1 * s1, h2 = q2 * s0, h3 = q3 * s1;
+    const half2_t l0 = __builtin_elementwise_fma(q0, s0, -h0), l1 = __builtin_elementwise_fma(q1, s1, -h1);
+    const half2_t l2 = __builtin_elementwise_fma(q2, s0, -h2), l3 = __builtin_elementwise_fma(q3, s1, -h3);
+    hi = half8_t{h0[0], h0[1], h1[0], h1[1], h2[0], h2[1], h3[0], h3[1]};
+    lo = half8_t{l0[0], l0[1], l1[0], l1[1], l2[0], l2[1], l3[0], l3[1]};
+}
+
 template <int WF, int FI, int WJ, int KS, bool LOCAL>
 __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const uint8_t* __restrict__ W, int n, int nb, const void* __restrict__ XH, const void* __restrict__ XL,
-    const int* __restrict__ XE, int m, float* __restrict__ Y, int accy, int full, int SR, int kbs, float* __restrict__ part,
+    const int* __restrict__ XE, int m, const uint32_t* __restrict__ XS, float* __restrict__ Y, int accy, int full, int SR, int kbs, float* __restrict__ part,
     int* __restrict__ cnt) {
     using C = TileCfg<WF, FI, WJ, KS>;
     constexpr int CB = C::CB, FJ = 4;
-    constexpr bool BYTES = C::BYTES;
-    constexpr uint32_t BB = BYTES ? 34u : 18u;  // bytes a block
+    constexpr bool BYTES = C::BYTES, Q4K = WF == WF_Q4_K, Q6K = WF == WF_Q6_K, CHAIN = C::CHAIN;
+    constexpr uint32_t BB = BYTES ? 34u : 18u;  // bytes a block (not CHAIN)
     static_assert(FI == 4 || FI == 8, "x tiles of a wave");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = C::CHAIN ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
     const int ks = wave % KS, wj = wave / KS;
     const int g = lane >> 4, r = lane & 15;
     // The first `full` tiles (whole rounds of workgroups, or all) are unsplit,
@@ -276,14 +334,20 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const int j0 = (rem / bh) * C::TJ, i0 = (band * GI + rem % bh) * C::TI;
     const int kb0 = slice * kbs, kb1 = S > 1 ? min(nb, kb0 + kbs) : nb;  // this slice's blocks (kb0 a multiple of CB)
 
-    const uint32_t k = (uint32_t)nb * 32u, row_bytes = (uint32_t)nb * BB, wbytes = (uint32_t)n * row_bytes;
+    const uint32_t k = (uint32_t)nb * 32u, row_bytes = Q4K   ? (uint32_t)(nb / 8) * 144u
+                                                             : Q6K ? (uint32_t)(nb / 8) * 210u
+                                                                   : (uint32_t)nb * BB,
+                   wbytes = (uint32_t)n * row_bytes;
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(W, wbytes);
     const __amdgpu_buffer_rsrc_t hrs = make_rsrc(XH, (uint32_t)m * k * 2u);
     const __amdgpu_buffer_rsrc_t lrs = make_rsrc(XL, (uint32_t)m * k * 2u);
     const int nchunks = (kb1 - kb0 + CB - 1) / CB;
 
     struct WRegs { uint32_t w[C::WU][C::WWORDS]; };
-    struct XRegs { u32x4 h[C::XU], l[C::XU]; };
+    struct XRegs {
+        u32x4 h[C::XU], l[C::XU];
+        uint32_t s[Q4K ? C::SU : 1];
+    };
     // unit u of a thread: block b0 + c CB of row j; CB is even, so a Q4_0 or Q8_0
     // block's place within its dword (2 bytes past it when j nb + b is odd) is
     // the same in every chunk.  Rows past n start out of range.
@@ -294,7 +358,10 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         const int idx = tid + u * C::NT, j = j0 + idx / CB;
         wblk[u] = idx % CB;
         const bool ok = (C::W_ALL || idx < C::TJ * CB) && j < n;
-        wbase[u] = ok ? ((uint32_t)j * row_bytes + (uint32_t)(kb0 + wblk[u]) * BB) & ~3u : RSRC_OOB;
+        if constexpr (CHAIN)  // the row's first super-block of the slice (kb0 % 8 == 0)
+            wbase[u] = ok ? (uint32_t)j * row_bytes + (uint32_t)(kb0 / 8) * (Q4K ? 144u : 210u) : RSRC_OOB;
+        else
+            wbase[u] = ok ? ((uint32_t)j * row_bytes + (uint32_t)(kb0 + wblk[u]) * BB) & ~3u : RSRC_OOB;
         wsel[u] = (((uint32_t)j * (uint32_t)nb + (uint32_t)wblk[u]) & 1u) ? 0x07060504u : 0x05040302u;
     }
     // the matrix may end 2 bytes into a window's last dword: that dword is read
@@ -303,6 +370,37 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     auto load_w = [&](int c, WRegs& R) {
 #pragma unroll
         for (int u = 0; u < C::WU; u++) {
+            if constexpr (Q4K) {
+                // sub-block b: the super-block's 16-byte header and the 16 bytes 16 (b %
+                // 8) of its nibbles (half b % 2 of the run that sub-blocks b & ~1, b | 1 share)
+                const uint32_t b = (uint32_t)(c * CB + wblk[u]), sb = (b >> 3) * 144u;
+                const bool ok = kb0 + (int)b < kb1;
+                const u32x4 h = buf_load_b128(wrs, ok ? wbase[u] + sb : RSRC_OOB);
+                const u32x4 q = buf_load_b128(wrs, ok ? wbase[u] + sb + 16u + 16u * (b & 7u) : RSRC_OOB);
+                R.w[u][0] = h.x, R.w[u][1] = h.y, R.w[u][2] = h.z, R.w[u][3] = h.w;
+                R.w[u][4] = q.x, R.w[u][5] = q.y, R.w[u][6] = q.z, R.w[u][7] = q.w;
+                continue;
+            }
+            if constexpr (Q6K) {
+                // chunk c is half hh of a super-block; unit e takes elements 8 e .. 8 e +
+                // 7 of its four groups: 8 bytes of each ql run and of qh (12-byte windows
+                // from the dword below: super-blocks start on even bytes), group e's two
+                // scales and d
+                const uint32_t b = (uint32_t)(c * CB), hh = (b >> 2) & 1u, e = (uint32_t)wblk[u];
+                const uint32_t base = wbase[u] + (b >> 3) * 210u;
+                const bool ok = kb0 + (int)b < kb1 && wbase[u] != RSRC_OOB;
+                const uint32_t q0 = ok ? (base + 64u * hh + 8u * e) & ~3u : RSRC_OOB;
+                const uint32_t qh = ok ? (base + 128u + 32u * hh + 8u * e) & ~3u : RSRC_OOB;
+                const auto v0 = __builtin_amdgcn_raw_buffer_load_b96(wrs, (int)q0, 0, 0);
+                const auto v1 = __builtin_amdgcn_raw_buffer_load_b96(wrs, (int)(ok ? q0 + 32u : RSRC_OOB), 0, 0);
+                const auto v2 = __builtin_amdgcn_raw_buffer_load_b96(wrs, (int)qh, 0, 0);
+                R.w[u][0] = v0[0], R.w[u][1] = v0[1], R.w[u][2] = v0[2];
+                R.w[u][3] = v1[0], R.w[u][4] = v1[1], R.w[u][5] = v1[2];
+                R.w[u][6] = v2[0], R.w[u][7] = v2[1], R.w[u][8] = v2[2];
+                R.w[u][9] = buf_load_b16(wrs, ok ? base + 192u + 8u * hh + 2u * e : RSRC_OOB);
+                R.w[u][10] = buf_load_b16(wrs, ok ? base + 208u : RSRC_OOB);
+                continue;
+            }
             const uint32_t base = kb0 + wblk[u] + c * CB < kb1 ? wbase[u] + (uint32_t)c * (CB * BB) : RSRC_OOB;
             const u32x4 v = buf_load_b128(wrs, base);
             R.w[u][0] = v.x, R.w[u][1] = v.y, R.w[u][2] = v.z, R.w[u][3] = v.w;
@@ -331,15 +429,75 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         if (q & 1) R.l[u] = buf_load_b128(lrs, off);
         else R.h[u] = buf_load_b128(hrs, off);
     };
+    const __amdgpu_buffer_rsrc_t srs = make_rsrc(Q4K ? (const void*)XS : XH, Q4K ? (uint32_t)m * (uint32_t)nb * 4u : 0u);
+    auto load_sums = [&](int c, XRegs& R) {
+        if constexpr (Q4K) {
+#pragma unroll
+            for (int u = 0; u < C::SU; u++) {
+                const int idx = tid + u * C::NT, i = i0 + idx / CB, b = kb0 + c * CB + idx % CB;
+                R.s[u] = buf_load_b32(srs, idx < C::TI * CB && i < m && b < kb1
+                                               ? ((uint32_t)i * (uint32_t)nb + (uint32_t)b) * 4u
+                                               : RSRC_OOB);
+            }
+        }
+    };
     auto load_x = [&](int c, XRegs& R) {
 #pragma unroll
         for (int q = 0; q < 2 * C::XU; q++) load_x_part(c, R, q);
+        load_sums(c, R);
     };
-    auto store_w = [&](int c, uint8_t* st, const WRegs& R) {
+    // aux: the super-block's own data (CHAIN)
+    auto store_w = [&](int c, uint8_t* st, uint8_t* aux, const WRegs& R) {
 #pragma unroll
         for (int u = 0; u < C::WU; u++) {
             const int idx = tid + u * C::NT, jl = idx / CB, bl = idx % CB;
             if (!C::W_ALL && idx >= C::TJ * CB) continue;
+            if constexpr (Q4K) {
+                uint32_t* dst = reinterpret_cast<uint32_t*>(st + bl * C::NIB_BLOCK + (jl >> 6) * 1024) + (jl & 63);
+#pragma unroll
+                for (int q = 0; q < 4; q++) dst[q * 64] = R.w[u][4 + q];
+                // every dword of the header stays live to here: a load whose last one
+                // is known dead (sub-blocks 0-3 do not use s[8..11]) has its register
+                // reused at once, behind a wait for the load
+                asm volatile("" ::"v"(R.w[u][0]), "v"(R.w[u][1]), "v"(R.w[u][2]), "v"(R.w[u][3]));
+                // sub-block j's 6-bit scale and min (parser.rs:562-569)
+                const uint32_t j = (uint32_t)(c * CB + bl) & 7u, sh = 8u * (j & 3u);
+                const uint32_t si = R.w[u][1] >> sh, ti = R.w[u][2] >> sh, ui = R.w[u][3] >> sh;
+                const uint32_t sc = j < 4 ? si & 63u : ((si >> 6) & 3u) | ((ui & 15u) << 2);
+                const uint32_t mn = j < 4 ? ti & 63u : ((ti >> 6) & 3u) | ((ui >> 2) & 60u);
+                reinterpret_cast<_Float16*>(st + C::W_BYTES)[bl * C::TJ + jl] = (_Float16)(float)sc;
+                const float d8 = 8.0f * h2f(R.w[u][0] & 0xFFFFu), dm = h2f(R.w[u][0] >> 16);
+                // t by the exponent bits of the larger: |e 2^-t| < 2^15
+                const int t = (int)(max(abs_bits(d8), abs_bits(dm)) >> 23) - 134;
+                const float e = ldexpf(d8 * (float)sc - dm * (float)mn, -t);
+                const _Float16 eh = (_Float16)e;
+                _Float16* em = reinterpret_cast<_Float16*>(aux + C::MN_AT) + jl * 16 + j;
+                em[0] = eh;
+                em[8] = (_Float16)(e - (float)eh);
+                reinterpret_cast<uint32_t*>(aux)[jl] = (R.w[u][0] & 0xFFFFu) | ((uint32_t)t << 16);  // d, t
+                continue;
+            }
+            if constexpr (Q6K) {
+                const uint32_t b = (uint32_t)(c * CB);
+                const uint32_t sel = ((wbase[u] + (b >> 3) * 210u) & 2u) ? 0x05040302u : 0x03020100u;
+                uint8_t* dst0 = st + (jl >> 6) * 1024 + (jl & 63) * 4;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const uint32_t A = perm(R.w[u][i + 1], R.w[u][i], sel), B = perm(R.w[u][i + 4], R.w[u][i + 3], sel);
+                    const uint32_t H = perm(R.w[u][i + 7], R.w[u][i + 6], sel);
+                    const int dq = 2 * bl + i;  // dword of the group's 32 codes
+                    uint8_t* dst = dst0 + (dq >> 2) * C::HALF + (dq & 3) * 256;
+                    constexpr uint32_t LO = 0x0F0F0F0Fu, TWO = 0x30303030u;
+                    *reinterpret_cast<uint32_t*>(dst) = (A & LO) | ((H << 4) & TWO);
+                    *reinterpret_cast<uint32_t*>(dst + C::NIB_BLOCK) = (B & LO) | ((H << 2) & TWO);
+                    *reinterpret_cast<uint32_t*>(dst + 2 * C::NIB_BLOCK) = ((A >> 4) & LO) | (H & TWO);
+                    *reinterpret_cast<uint32_t*>(dst + 3 * C::NIB_BLOCK) = ((B >> 4) & LO) | ((H >> 2) & TWO);
+                }
+                const half2_t sp = {(_Float16)(float)(int8_t)(R.w[u][9] & 0xFFu), (_Float16)(float)(int8_t)(R.w[u][9] >> 8)};
+                reinterpret_cast<uint32_t*>(st + C::W_BYTES)[bl * C::TJ + jl] = __builtin_bit_cast(uint32_t, sp);
+                reinterpret_cast<uint32_t*>(aux)[jl] = R.w[u][10];
+                continue;
+            }
             const uint32_t end = wbase[u] + (uint32_t)c * (CB * BB) + (BYTES ? 32u : 16u);
             const uint32_t tail = R.w[u][C::WWORDS - 1];
             const uint32_t wt = end > wlast ? tail >> 16 : tail;
@@ -360,7 +518,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // x piece (row il, block bl, group gq) at slot 16 gq + (row ^ (4 (bl % 2) + gq)) of its tile's
     // part: eight consecutive threads (one row's pieces) and eight consecutive
     // lanes of a fragment read (one group's rows) each touch all LDS banks once
-    auto store_x = [&](uint8_t* st, const XRegs& R) {
+    auto store_x = [&](int c, uint8_t* st, uint8_t* aux, const XRegs& R) {
         uint8_t* xs = st + C::W_BYTES + C::D_BYTES;
 #pragma unroll
         for (int u = 0; u < C::XU; u++) {
@@ -369,6 +527,17 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
             uint8_t* p = xs + (((q >> 2) * (C::TI / 16) + (il >> 4)) * 2) * C::X_PART + slot * 16;
             *reinterpret_cast<u32x4*>(p) = R.h[u];
             *reinterpret_cast<u32x4*>(p + C::X_PART) = R.l[u];
+        }
+        if constexpr (Q4K) {
+#pragma unroll
+            for (int u = 0; u < C::SU; u++) {
+                const int idx = tid + u * C::NT, il = idx / CB, j = (c * CB + idx % CB) & 7;
+                // (no branch in the loop body: what follows it would sink past it)
+                uint16_t* ss = reinterpret_cast<uint16_t*>(
+                    idx < C::TI * CB ? aux + C::SS_AT + (il >> 4) * 512 + (il & 15) * 16 + j * 2 : lds + C::DUMP_AT);
+                ss[0] = (uint16_t)R.s[u];
+                ss[128] = (uint16_t)(R.s[u] >> 16);
+            }
         }
     };
 
@@ -387,17 +556,34 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // Past the end every load reads zeros (x 0, d 0).
     constexpr int RB = FI / 2;
     const Q4Consts qc = q4_consts();
-    u32x4 nv, nv2;    // codes of the next block (nv2: Q8_0's second half)
-    uint2 dd;
-    half8_t wq[2][4];
+    constexpr bool ONE = Q6K;  // no registers for two sets of operands: converted between the chunks
+    u32x4 nv, nv2;  // codes of the next block (nv2: bytes 16+4g .., Q8_0 and the super-block formats)
+    uint32_t dd[Q6K ? 4 : 2];
+    half8_t wq[ONE ? 1 : 2][4], wl[Q6K ? 4 : 1];
     float dv[2][4];
     half8_t xh[2], xl[2];
-    f32x4 p[2][FJ];
+    f32x4 p[CHAIN ? 1 : 2][FJ], T[CHAIN ? FI : 1][FJ];
+    // Q4_K: even sub-blocks are low nibbles, odd ones high; this wave's are all alike
+    const uint32_t kmask = ks & 1 ? qc.hi : qc.lo;
+    const uint32_t kmul = ks & 1 ? 0x2C002C00u : 0x3C003C00u;  // f16 1 / 16, 1
+    const uint32_t koff = ks & 1 ? 0xD480D480u : 0xE408E408u;  // f16 -72, -1032
     auto read_w = [&](const uint8_t* st) {
-        nv = *reinterpret_cast<const u32x4*>(st + ks * C::NIB_BLOCK + wj * 1024 + g * 256 + r * 16);
-        if constexpr (BYTES)
-            nv2 = *reinterpret_cast<const u32x4*>(st + ks * C::NIB_BLOCK + C::HALF + wj * 1024 + g * 256 + r * 16);
-        dd = *reinterpret_cast<const uint2*>(st + C::W_BYTES + (ks * C::TJ + wj * 64 + r * 4) * 2);
+        const int lo = wj * 1024 + g * 256 + r * 16;
+        if constexpr (Q4K) {  // both halves of the run of sub-blocks ks & ~1, ks | 1
+            nv = *reinterpret_cast<const u32x4*>(st + (ks & ~1) * C::NIB_BLOCK + lo);
+            nv2 = *reinterpret_cast<const u32x4*>(st + (ks | 1) * C::NIB_BLOCK + lo);
+        } else {
+            nv = *reinterpret_cast<const u32x4*>(st + ks * C::NIB_BLOCK + lo);
+            if constexpr (BYTES) nv2 = *reinterpret_cast<const u32x4*>(st + ks * C::NIB_BLOCK + C::HALF + lo);
+        }
+        const uint8_t* dp = st + C::W_BYTES + (ks * C::TJ + wj * 64 + r * 4) * (Q6K ? 4 : 2);
+        if constexpr (Q6K) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(dp);
+            dd[0] = v.x, dd[1] = v.y, dd[2] = v.z, dd[3] = v.w;
+        } else {
+            const uint2 v = *reinterpret_cast<const uint2*>(dp);
+            dd[0] = v.x, dd[1] = v.y;
+        }
     };
     auto read_x = [&](const uint8_t* st, int s) {
         const uint8_t* xb = st + C::W_BYTES + C::D_BYTES + (ks * FI + s) * 2 * C::X_PART +
@@ -407,13 +593,21 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     };
     auto conv = [&](int o, int a) {
         const uint32_t n0 = a == 0 ? nv.x : a == 1 ? nv.y : a == 2 ? nv.z : nv.w;
-        if constexpr (BYTES) {
-            const uint32_t n1 = a == 0 ? nv2.x : a == 1 ? nv2.y : a == 2 ? nv2.z : nv2.w;
-            wq[o][a] = q8_f16(n0, n1);
-        } else {
-            wq[o][a] = q4_f16(n0, qc);
+        const uint32_t n1 = a == 0 ? nv2.x : a == 1 ? nv2.y : a == 2 ? nv2.z : nv2.w;
+        if constexpr (Q6K) {
+            q6k_f16(n0, n1, dd[a], wq[0][a], wl[a]);
+            return;
         }
-        dv[o][a] = h2f(a == 0 ? dd.x & 0xFFFFu : a == 1 ? dd.x >> 16 : a == 2 ? dd.y & 0xFFFFu : dd.y >> 16);
+        const uint32_t d16 = a & 1 ? dd[a >> 1] >> 16 : dd[a >> 1] & 0xFFFFu;
+        if constexpr (Q4K) {
+            const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)d16);
+            wq[ONE ? 0 : o][a] = q4k_f16(n0, n1, kmask, qc.magic, __builtin_bit_cast(half2_t, kmul),
+                                              __builtin_bit_cast(half2_t, koff), sc);
+            return;
+        }
+        if constexpr (BYTES) wq[o][a] = q8_f16(n0, n1);
+        else wq[o][a] = q4_f16(n0, qc);
+        dv[o][a] = h2f(d16);
         // f32 here once a block: left to itself the compiler folds the conversion
         // into every scale FMA (v_fma_mix_f32: 1,240 against 546 us, 2048 x 14336 x 4096)
         asm volatile("" : "+v"(dv[o][a]));
@@ -424,81 +618,193 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
 #pragma unroll
             for (int u = 0; u < 4; u++) acc[b][a][u] = fmaf(dv[o][a], p[ps][a][u], acc[b][a][u]);
     };
-    // chunks the loads run ahead (FI 8: no registers for more)
-    constexpr int DX = FI == 8 ? 1 : 2, DW = FI == 8 && BYTES ? 1 : 2;
+    // CHAIN: a finished super-block (its own data at aux) goes into the sums in
+    // the FI steps of the next chunk: step b adds x tile b, and Q4_K's remainder
+    // of weight column b for the FO tiles ks FO .. that this K group ends with
+    // (um, so that the KS groups share them).  K elements 8 g .. of that MFMA:
+    // S hi, lo, hi, lo times e hi, hi, lo, lo.
+    constexpr int FO = FI / KS;
+    static_assert(!CHAIN || FI == FJ, "a weight column a step");
+    f32x4 um[Q4K ? FO : 1][FJ];
+    u32x4 fd;                       // d (and t) of the lane's four columns
+    half8_t fs[Q4K ? FO : 1], fe;   // S of the tiles, e of the step's column
+    auto flush_e = [&](int a, const uint8_t* aux) {
+        if constexpr (Q4K)
+            fe = *reinterpret_cast<const half8_t*>(aux + C::MN_AT + (wj * 64 + r * 4 + a) * 32 + (g >> 1) * 16);
+    };
+    auto flush_begin = [&](const uint8_t* aux) {
+        fd = *reinterpret_cast<const u32x4*>(aux + (wj * 64 + r * 4) * 4);
+        if constexpr (Q4K) {
+#pragma unroll
+            for (int b = 0; b < FO; b++)
+                fs[b] = *reinterpret_cast<const half8_t*>(aux + C::SS_AT + (ks * FO + b) * 512 + (g & 1) * 256 + r * 16);
+        }
+        flush_e(0, aux);
+    };
+    auto flush = [&](int b, const uint8_t* aux) {
+        const uint32_t db[4] = {fd.x, fd.y, fd.z, fd.w};
+        f32x4 u4[Q4K ? FO : 1];
+        if constexpr (Q4K) {
+            const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int o = 0; o < FO; o++) u4[o] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fs[o], fe, z, 0, 0, 0);
+            if (b + 1 < FJ) flush_e(b + 1, aux);
+        }
+#pragma unroll
+        for (int a = 0; a < FJ; a++) {
+            const float d = h2f(db[a] & 0xFFFFu);
+#pragma unroll
+            for (int u = 0; u < 4; u++) acc[b][a][u] = fmaf(d, T[b][a][u], acc[b][a][u]);
+        }
+        if constexpr (Q4K) {
+            const float dm = ldexpf(32.0f, (int)db[b] >> 16);
+#pragma unroll
+            for (int o = 0; o < FO; o++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) um[o][b][u] = fmaf(dm, u4[o][u], um[o][b][u]);
+        }
+    };
+    // chunks the loads run ahead (no registers for more)
+    constexpr int DX = FI == 8 || CHAIN ? 1 : 2, DW = (FI == 8 && BYTES) || CHAIN ? 1 : 2;
+    constexpr int UN = CHAIN ? 8 / CB : 2;  // chunks a turn of the loop: a super-block, or two
     WRegs w[DW];
     XRegs x1[DX];
     uint8_t *bc = lds, *bn = lds + C::STAGE, *bf = lds + 2 * C::STAGE;  // chunk c, c + 1, free
-    // chunk c; H = c % 2 (register sets by parity)
+    // super-block being multiplied, the next one, the previous one
+    uint8_t *ac = lds + C::AUX_AT, *an = ac + C::AUX, *ap = an + C::AUX;
+    // chunk c = U modulo UN (register sets by parity)
     auto chunk = [&](int c, auto u_tag) {
-        constexpr int U = decltype(u_tag)::value, H = U & 1, WS = (U + 1) % DW, XS = (U + 1) % DX;
+        constexpr int U = decltype(u_tag)::value, H = U & 1, WS = (U + 1) % DW, XS1 = (U + 1) % DX;
+        uint8_t* const as = CHAIN && U == UN - 1 ? an : ac;  // chunk c + 1's super-block
 #pragma unroll
         for (int s = 0; s < FI; s++) {
             if (s + 1 < FI) read_x(bc, s + 1);
             else read_x(bn, 0);
-            if (s == RB) read_w(bn);
+            if (s == RB && !ONE) read_w(bn);
             const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (CHAIN) {
+                if (U == 0) {
+                    flush(s, ap);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // Q6_K: one operand at a time, four independent MFMAs between
+                // dependent ones (2 % faster); Q4_K: a column at a time (3 %)
+                auto mul = [&](int a, const half8_t& xv, const half8_t& wv, bool first) {
+                    T[s][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, wv, U == 0 && first ? z : T[s][a], 0, 0, 0);
+                };
+                if constexpr (Q6K) {
 #pragma unroll
-            for (int a = 0; a < FJ; a++) {
-                p[s & 1][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[s & 1], wq[H][a], z, 0, 0, 0);
-                p[s & 1][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[s & 1], wq[H][a], p[s & 1][a], 0, 0, 0);
+                    for (int a = 0; a < FJ; a++) mul(a, xh[s & 1], wq[0][a], true);
+#pragma unroll
+                    for (int a = 0; a < FJ; a++) mul(a, xl[s & 1], wq[0][a], false);
+#pragma unroll
+                    for (int a = 0; a < FJ; a++) mul(a, xh[s & 1], wl[a], false);
+                } else {
+#pragma unroll
+                    for (int a = 0; a < FJ; a++) {
+                        mul(a, xh[s & 1], wq[H][a], true);
+                        mul(a, xl[s & 1], wq[H][a], false);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int a = 0; a < FJ; a++) {
+                    p[s & 1][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[s & 1], wq[H][a], z, 0, 0, 0);
+                    p[s & 1][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[s & 1], wq[H][a], p[s & 1][a], 0, 0, 0);
+                }
+                add(s == 0 ? FI - 1 : s - 1, s == 0 ? H ^ 1 : H, (s & 1) ^ 1);
             }
-            add(s == 0 ? FI - 1 : s - 1, s == 0 ? H ^ 1 : H, (s & 1) ^ 1);
-            if (s > RB) {
+            if (s > RB && !ONE) {
 #pragma unroll
                 for (int a = 0; a < FJ; a++)
                     if (a * (FI - 1 - RB) / FJ == s - 1 - RB) conv(H ^ 1, a);
             }
-            if (s == 0) store_w(c + 1, bn, w[WS]);
-            if (s == 1) store_x(bn, x1[XS]);
+            if (s == 0) {
+                store_w(c + 1, bn, as, w[WS]);
+                if (DW == 1) load_w(c + 2, w[0]);
+            }
+            if (s == 1) store_x(c + 1, bn, as, x1[XS1]);
             // the loads into the freed registers, spread over the later steps (a
             // burst of them stalls the waves at issue)
-            if (s == FI - 1) load_w(c + 1 + DW, w[WS]);
+            if (DW == 2 && s == FI - 1) load_w(c + 3, w[WS]);
             if (s >= 2) {
 #pragma unroll
                 for (int q = 0; q < 2 * C::XU; q++)
-                    if (2 + q * (FI - 2) / (2 * C::XU) == s) load_x_part(c + 1 + DX, x1[XS], q);
+                    if (2 + q * (FI - 2) / (2 * C::XU) == s) load_x_part(c + 1 + DX, x1[XS1], q);
+                if (s == FI - 1) load_sums(c + 1 + DX, x1[XS1]);
             }
+            if constexpr (!Q6K) {
 #pragma unroll
-            for (int a = 0; a < FJ; a++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                for (int a = 0; a < FJ; a++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
             if (s == RB - 1) __syncthreads();
+        }
+        if (CHAIN && U == UN - 1) flush_begin(ac);
+        if constexpr (ONE) {
+            read_w(bn);
+#pragma unroll
+            for (int a = 0; a < FJ; a++) conv(0, a);
         }
         uint8_t* t3 = bc;
         bc = bn;
         bn = bf;
         bf = t3;
+        if (CHAIN && U == UN - 1) {
+            uint8_t* t4 = ap;
+            ap = ac;
+            ac = an;
+            an = t4;
+        }
     };
     // chunks 0 .. DW - 1 of W and 0 .. DX - 1 of x first, then on to DW / DX
     // once chunk 0 is stored
 #pragma unroll
-    for (int q = 0; q < DW; q++) {
-        load_w(q, w[q]);
-    }
+    for (int q = 0; q < DW; q++) load_w(q, w[q]);
 #pragma unroll
     for (int q = 0; q < DX; q++) load_x(q, x1[q]);
-    store_w(0, bc, w[0]);
-    store_x(bc, x1[0]);
+    if constexpr (CHAIN)  // nothing to flush before the first super-block: zeros
+        for (int q = tid; q < C::AUX / 4; q += C::NT) reinterpret_cast<uint32_t*>(ap)[q] = 0;
+    store_w(0, bc, ac, w[0]);
+    store_x(0, bc, ac, x1[0]);
     load_w(DW, w[0]);
     load_x(DX, x1[0]);
     __syncthreads();
     read_w(bc);
     read_x(bc, 0);
+    if constexpr (CHAIN) flush_begin(ap);
 #pragma unroll
     for (int a = 0; a < FJ; a++) {
         conv(0, a);
-        dv[1][a] = 0.0f;
-        p[1][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (!CHAIN) {
+            dv[1][a] = 0.0f;
+            p[1][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        } else {
+#pragma unroll
+            for (int b = 0; b < FI; b++) T[b][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (Q4K)
+#pragma unroll
+                for (int b = 0; b < FO; b++) um[b][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
     }
     // (chunks past the slice's end: zeros; no branch, so that the waits stay exact)
-    for (int c = 0; c < nchunks; c += 2) {
+    for (int c = 0; c < nchunks; c += UN) {
         chunk(c, std::integral_constant<int, 0>{});
         chunk(c + 1, std::integral_constant<int, 1>{});
+        if constexpr (UN == 4) {
+            chunk(c + 2, std::integral_constant<int, 2>{});
+            chunk(c + 3, std::integral_constant<int, 3>{});
+        }
     }
-    add(FI - 1, 1, 1);
+    if constexpr (CHAIN) {
+#pragma unroll
+        for (int b = 0; b < FI; b++) flush(b, ap);  // (begun at the end of the last chunk)
+    } else {
+        add(FI - 1, 1, 1);
+    }
 
     // lane (g, r) holds y[i = 4 g + u][j = 4 r .. 4 r + 3] of 16-row tile b
     auto store_rows = [&](int b, const f32x4 (&v4)[FJ]) {
@@ -524,7 +830,6 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // The KS waves of a column group share its 16-row tiles: wave ks ends with
     // the sums of tiles ks FO .. ks FO + FO - 1.  Each wave hands the tiles of
     // the others through LDS (the stages are free once every wave is here).
-    constexpr int FO = FI / KS;
     __syncthreads();
     if constexpr (KS > 1) {
         f32x4* red = reinterpret_cast<f32x4*>(lds) + wj * (KS * (KS - 1) * FO * FJ * 64) + lane;
@@ -557,6 +862,12 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
 #pragma unroll
                 for (int a = 0; a < FJ; a++) own[b][a] += red[(((ks * (KS - 1) + q) * FO + b) * FJ + a) * 64];
     }
+
+    if constexpr (Q4K)
+#pragma unroll
+        for (int b = 0; b < FO; b++)
+#pragma unroll
+            for (int a = 0; a < FJ; a++) own[b][a] += um[b][a];
 
     // ---- slices of the tile: partials, counter, the last one adds them in slice order
     if (S > 1) {
@@ -615,13 +926,13 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
 struct XSplit {
     _Float16 *h, *l;
     int* e;
-    float* s;  // x' sums of each block, or NULL
+    uint32_t* s;  // x' sums of each block (hi / lo pairs), or NULL
 };
 XSplit x_split_at(void* scratch, size_t m, size_t k, bool sums) {
     const size_t xb = (m * k * 2 + 255) & ~(size_t)255, eb = (m * 4 + 255) & ~(size_t)255;
     uint8_t* p = reinterpret_cast<uint8_t*>(scratch);
     return {reinterpret_cast<_Float16*>(p), reinterpret_cast<_Float16*>(p + xb), reinterpret_cast<int*>(p + 2 * xb),
-            sums ? reinterpret_cast<float*>(p + 2 * xb + eb) : nullptr};
+            sums ? reinterpret_cast<uint32_t*>(p + 2 * xb + eb) : nullptr};
 }
 
 // One tile shape: 64 WJ weight rows x 16 FI x rows, KS wave groups sharing
@@ -643,7 +954,7 @@ hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const XSplit& x, int
     }
     unsigned rest = (unsigned)((n + C::TJ - 1) / C::TJ) * (unsigned)((m + C::TI - 1) / C::TI) - (unsigned)p.full;
     if (local) rest = (rest + 7) / 8 * 8;
-    launch_kernel(kern, dim3((unsigned)p.full + rest * (unsigned)p.S), dim3(C::NT), (size_t)C::LDS, s, w, n, nb, x.h, x.l, x.e, m, y,
+    launch_kernel(kern, dim3((unsigned)p.full + rest * (unsigned)p.S), dim3(C::NT), (size_t)C::LDS, s, w, n, nb, x.h, x.l, x.e, m, x.s, y,
                   accy, p.full, p.S, p.kbs, part, cnt);
     return hipGetLastError();
 }
@@ -656,6 +967,11 @@ struct TileShape {
     double us_block;
 };
 constexpr TileShape TILE_SHAPES[4] = {{256, 128, 2, 0.90}, {256, 64, 2, 0.50}, {128, 64, 4, 0.29}, {64, 64, 4, 0.26}};
+// The super-block formats run on one shape: their sums take the registers of
+// the larger ones (Q4_K in 256 x 64 tiles spills: 211 x 14336 x 4096 115 us there, 114 here),
+// and 64 x 64 tiles spill too (72 us against 58 at 128 x 4096 x 4096).
+constexpr int SUPER_SHAPE = 2;
+constexpr double SUPER_US_BLOCK = 0.43;
 
 // Tile shape and K slices of a product by estimated time.  Whole rounds of
 // one workgroup a CU run unsplit; the tiles past them are split over K, where
@@ -667,16 +983,19 @@ constexpr TileShape TILE_SHAPES[4] = {{256, 128, 2, 0.90}, {256, 64, 2, 0.50}, {
 // 4096 64 tiles of 128 x 64 in 4 slices (25.6 us; unsplit 40.4, 2 slices 28.7,
 // 8 slices 36.2), 14336 x 4096 the same tiles unsplit (44 us; 256 x 128 117,
 // 64 x 64 67), 512 rows 14336 x 4096 256 x 128 (127 us; 256 x 64 162).
-TilePlan tile_plan(size_t m, size_t n, size_t nb, bool can_split) {
+TilePlan tile_plan(WType t, size_t m, size_t n, size_t nb, bool can_split) {
+    const bool super = t == WType::Q4_K || t == WType::Q6_K;
     const size_t round = std::max(8, device_cu_count() / 8 * 8);
     TilePlan best{};
     double best_us = 1e30;
     for (int c = 0; c < 4; c++) {
-        const TileShape& t = TILE_SHAPES[c];
-        const size_t tiles = ((n + t.tj - 1) / t.tj) * ((m + t.ti - 1) / t.ti);
-        const size_t unit = 2 * (size_t)t.ks;  // the main loop's step: two chunks
+        if (super && c != SUPER_SHAPE) continue;
+        const TileShape& sh = TILE_SHAPES[c];
+        const double us_block = super ? SUPER_US_BLOCK : sh.us_block;
+        const size_t tiles = ((n + sh.tj - 1) / sh.tj) * ((m + sh.ti - 1) / sh.ti);
+        const size_t unit = super ? 8 : 2 * (size_t)sh.ks;  // a turn of the main loop: two chunks, or a super-block
         const size_t full = tiles / round * round, rest = tiles - full;
-        const double whole = nb * t.us_block + 6.0;  // us a round of unsplit tiles
+        const double whole = nb * us_block + 6.0;  // us a round of unsplit tiles
         for (size_t S = 1; S <= 16; S++) {
             const size_t kbs = ((nb + S - 1) / S + unit - 1) / unit * unit;
             double us = (double)(full / round) * whole;
@@ -685,9 +1004,9 @@ TilePlan tile_plan(size_t m, size_t n, size_t nb, bool can_split) {
             } else {
                 if (!can_split || rest * S > round) break;
                 if ((S - 1) * kbs >= nb) continue;  // (an empty slice)
-                const size_t bytes = S * t.tj * t.ti * sizeof(float);
+                const size_t bytes = S * sh.tj * sh.ti * sizeof(float);
                 if (rest == 0 || rest * bytes > GEMM_PART_BYTES) break;
-                us += kbs * t.us_block + 6.0 + 2.0 + (double)bytes / 40e3;
+                us += kbs * us_block + 6.0 + 2.0 + (double)bytes / 40e3;
             }
             if (us < best_us) best_us = us, best = {c, (int)(S == 1 ? tiles : full), (int)S, (int)kbs};
         }
@@ -714,46 +1033,58 @@ hipError_t launch_split(const float* x, size_t m, size_t k, const float* g, floa
 // smaller (us, here against there: Q4_0 100 x 512 x 992 10.7 / 9.1, 200 x 2048 x
 // 992 13.6 / 12.7, 100 x 2048 x 2048 14.2 / 15.8, 100 x 64 x 4096 13.4 / 17.3;
 // Q8_0 100 x 512 x 992 11.0 / 8.9, 1000 x 512 x 992 17.5 / 16.4, 333 x 4096 x 992
-// 19.5 / 25.7, 17 x 4096 x 4096 17.9 / 17.2, 33 x 4096 x 4096 18.6 / 24.4).
+// 19.5 / 25.7, 17 x 4096 x 4096 17.9 / 17.2, 33 x 4096 x 4096 18.6 / 24.4; Q4_K 64 x
+// 2048 x 2048 16.5 / 14.7, 128 x 2048 x 2048 18.5 / 19.1, 32 x 512 x 4096 17.3 / 22.3, 16 x
+// 4096 x 4096 19.5 / 17.3, 16 x 14336 x 1024 17.6 / 24.1, 500 x 4096 x 1024 23.4 / 26.8,
+// 211 x 4096 x 1024 19.7 / 17.4; Q6_K alike).
 bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k) {
     if (k > GEMM_TILE_MAX_K) return false;
     if (t == WType::Q4_0) return m > GEMM_XTILE_M && !(m <= 256 && k <= 2048 && n * k <= (size_t)1 << 22);
+    if (t == WType::Q4_K || t == WType::Q6_K) {
+        if (n >= 8192) return m >= KQ_GEMM_MIN_M;
+        return m >= 32 && (k >= 4096 || (m >= 128 && k >= 2048 && n >= 2048) || m * n >= (size_t)3 << 19);
+    }
     if (t != WType::Q8_0 || m < KQ_GEMM_MIN_M) return false;
     if (k <= 2048 && (m * n <= (size_t)1 << 19 || (m <= 256 && n * k <= (size_t)1 << 23))) return false;
     return m > 24 || n * k > (size_t)1 << 24;
 }
 
-size_t gemm_part_bytes(size_t m, size_t n, size_t k) {
-    const TilePlan p = tile_plan(m, n, k / QK, true);
-    const TileShape& t = TILE_SHAPES[p.cfg];
-    const size_t rest = ((n + t.tj - 1) / t.tj) * ((m + t.ti - 1) / t.ti) - (size_t)p.full;
-    return rest * p.S * t.tj * t.ti * sizeof(float);
+size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k) {
+    const TilePlan p = tile_plan(t, m, n, k / QK, true);
+    const TileShape& sh = TILE_SHAPES[p.cfg];
+    const size_t rest = ((n + sh.tj - 1) / sh.tj) * ((m + sh.ti - 1) / sh.ti) - (size_t)p.full;
+    return rest * p.S * sh.tj * sh.ti * sizeof(float);
 }
 
 template <int WF>
-static hipError_t launch_tile_wf(const uint8_t* w, int n, int nb, const XSplit& x, int m, float* y, int accy,
+static hipError_t launch_tile_wf(WType t, const uint8_t* w, int n, int nb, const XSplit& x, int m, float* y, int accy,
                                  float* part, int* cnt, hipStream_t s) {
-    const TilePlan p = tile_plan(m, n, nb, part != nullptr && cnt != nullptr);
-    switch (p.cfg) {
-        case 0: return launch_tile_cfg<WF, 8, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
-        case 1: return launch_tile_cfg<WF, 4, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
-        case 2: return launch_tile_cfg<WF, 4, 2, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
-        default: return launch_tile_cfg<WF, 4, 1, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
-    }
+    const TilePlan p = tile_plan(t, m, n, nb, part != nullptr && cnt != nullptr);
+    if constexpr (WF == WF_Q4_0 || WF == WF_Q8_0)
+        if (p.cfg == 0) return launch_tile_cfg<WF, 8, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+    if constexpr (WF == WF_Q4_0 || WF == WF_Q8_0)
+        if (p.cfg == 1) return launch_tile_cfg<WF, 4, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+    if constexpr (WF == WF_Q4_0 || WF == WF_Q8_0)
+        if (p.cfg == 3) return launch_tile_cfg<WF, 4, 1, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+    return launch_tile_cfg<WF, 4, 2, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
 }
 
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
                             hipStream_t s) {
     if (k == 0 || !gemm_tile_takes(t, m, n, k)) return hipErrorInvalidValue;
-    const XSplit xo = x_split_at(scratch, m, k, false);
+    const XSplit xo = x_split_at(scratch, m, k, t == WType::Q4_K);
     const hipError_t e = pro == 1   ? launch_split<1>(x, m, k, g, eps, xo, s)
                          : pro == 2 ? launch_split<2>(x, m, k, g, eps, xo, s)
                                     : launch_split<0>(x, m, k, g, eps, xo, s);
     if (e != hipSuccess) return e;
     const int ni = (int)n, nb = (int)(k / QK), mi = (int)m, acc = accumulate ? 1 : 0;
-    return t == WType::Q4_0 ? launch_tile_wf<WF_Q4_0>(w, ni, nb, xo, mi, y, acc, part, cnt, s)
-                            : launch_tile_wf<WF_Q8_0>(w, ni, nb, xo, mi, y, acc, part, cnt, s);
+    switch (t) {
+        case WType::Q4_0: return launch_tile_wf<WF_Q4_0>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
+        case WType::Q8_0: return launch_tile_wf<WF_Q8_0>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
+        case WType::Q4_K: return launch_tile_wf<WF_Q4_K>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
+        default: return launch_tile_wf<WF_Q6_K>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
+    }
 }
 
 }  // namespace rdl

@@ -189,7 +189,7 @@ bool combine_is_coherent();
 // True when the current device's next combine runs XCD-local (placement
 // probed and a rotation, switch off); does not probe.
 bool combine_local_now();
-// part: gemm_part_bytes(m, n, k) bytes for the K-slice partials of the tile
+// part: gemm_part_bytes(Q4_0, m, n, k) bytes for the K-slice partials of the tile
 // GEMM (m > GEMM_XTILE_M); NULL (or no counters): that GEMM runs unsplit.
 hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* counters, hipStream_t s);
@@ -197,12 +197,12 @@ hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x
 // device (gemm.hip).
 bool xcd_round_robin(hipStream_t s);
 // The tile GEMM (gemm_tiles.hip; arguments as launch_gemm_tiles_ex, k <=
-// GEMM_TILE_MAX_K): its K-slice partials take gemm_part_bytes(m, n, k), at
+// GEMM_TILE_MAX_K): its K-slice partials take gemm_part_bytes(t, m, n, k), at
 // most GEMM_PART_BYTES, and one counter a tile of at most GEMM_SPLIT_TILES.
 constexpr size_t GEMM_TILE_MAX_K = 16384;
 constexpr size_t GEMM_PART_BYTES = 16u << 20;
 constexpr size_t GEMM_SPLIT_TILES = 256;
-size_t gemm_part_bytes(size_t m, size_t n, size_t k);
+size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k);
 // Whether a float-mode product takes the tile GEMM (Q4_0 beyond GEMM_XTILE_M
 // rows, Q8_0 from KQ_GEMM_MIN_M): where it is faster than the small-tile
 // kernel of gemm.hip.

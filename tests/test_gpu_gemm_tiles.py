@@ -4,7 +4,7 @@ unsplit, on both combines and under graph replay."""
 import numpy as np
 import pytest
 
-from parity import check_parity, exact_f64
+from parity import check_parity, exact_f64, exact_f64_cond
 from rdlquant import synth
 
 pytestmark = pytest.mark.gpu
@@ -28,6 +28,46 @@ def test_tiles(rq, orc, gpu, kind, dtype, m, n, k):
     rows = np.unique(np.linspace(0, m - 1, 24).astype(int))
     want = orc.matmul(kind, x[rows], w, len(rows), k, n, threads=16)
     check_parity(got[rows].reshape(-1), want, exact_f64(orc, kind, x[rows], w, len(rows), k, n))
+
+
+# one 16-row x tile and just past one, both sides of the 128-row weight tiles,
+# one super-block a row and 17 (the last slice shorter), odd super-block counts
+# (Q6_K rows starting 2 bytes past a dword), the K split, a partial last round
+@pytest.mark.parametrize("kind,dtype", [("q4k", 12), ("q6k", 14)])
+@pytest.mark.parametrize("m,n,k", [(16, 8192, 256), (32, 1, 4096), (33, 127, 4352), (65, 129, 4096), (128, 2048, 2048),
+                                   (130, 8200, 768), (400, 4096, 256)])
+def test_super_block_tiles(rq, orc, gpu, kind, dtype, m, n, k):
+    print(f"case {kind} tiles m={m} n={n} k={k}", flush=True)
+    x = synth.activations(m, k, m + n + k)
+    w = synth.weights(dtype, n, k, m + n)
+    got = getattr(rq, "matmul_f32_q4_k" if dtype == 12 else "matmul_f32_q6_k")(x, w, m, k, n).reshape(m, n)
+    rows = np.unique(np.linspace(0, m - 1, 20).astype(int))
+    want = orc.matmul(kind, x[rows], w, len(rows), k, n, threads=16)
+    exact, cond = exact_f64_cond(orc, kind, x[rows], w, len(rows), k, n)
+    check_parity(got[rows].reshape(-1), want, exact, cond=cond)
+
+
+@pytest.mark.parametrize("kind,dtype", [("q4k", 12), ("q6k", 14)])
+def test_super_block_tiles_extreme_scales(rq, orc, gpu, kind, dtype):
+    # d (and dmin) from 2^-24 to 2^10 within a row, scale bytes at both ends.  Each
+    # output within 1e-6 sum |w x|: 2^-23 for the x split, as much for Q6_K's
+    # dropped lo lo and Q4_K's f16 pairs, and f32 sums of 16 super-blocks
+    m, n, k = 40, 130, 4096
+    r = np.random.default_rng(7)
+    ns = k // 256
+    w = synth.weights(dtype, n, k, 8).reshape(n, ns, -1).copy()
+    half = lambda: synth.f16_bits(2.0 ** r.integers(-24, 11, size=(n, ns)))[..., None].view(np.uint8).reshape(n, ns, 2)
+    if dtype == 12:
+        w[..., 0:2], w[..., 2:4] = half(), half()
+        w[0, :, 4:16], w[1, :, 4:16] = 0xFF, 0x00
+    else:
+        w[..., 208:210] = half()
+        w[0, :, 192:208], w[1, :, 192:208] = 0x80, 0x00
+    x = synth.activations(m, k, 9) * (10.0 ** r.uniform(-6, 4, size=(m, 1))).astype(np.float32)
+    got = getattr(rq, "matmul_f32_q4_k" if dtype == 12 else "matmul_f32_q6_k")(x, w.reshape(-1), m, k, n)
+    exact, cond = exact_f64_cond(orc, kind, x, w.reshape(-1), m, k, n)
+    assert np.all(np.abs(got - exact) <= 1e-6 * cond)
+    assert np.all(got.reshape(m, n)[:, 1] == 0.0)
 
 
 @pytest.mark.parametrize("m,n,k", [(128, 1024, 4096), (100, 4096, 1024)])
