@@ -48,43 +48,6 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ---- x preparation: per-row power-of-two scale, f16 hi / lo split ---------------
-constexpr int XPREP_THREADS = 256;
-
-__global__ __launch_bounds__(XPREP_THREADS) void gemm_xprep_kernel(const float* __restrict__ X, int k,
-                                                                   _Float16* __restrict__ XH,
-                                                                   _Float16* __restrict__ XL,
-                                                                   int* __restrict__ XE) {
-    __shared__ float red[XPREP_THREADS / 64];
-    const int row = blockIdx.x;
-    const float* x = X + (size_t)row * k;
-    float amax = 0.0f;
-    bool bad = false;
-    for (int c = threadIdx.x; c < k; c += XPREP_THREADS) {
-        const float v = x[c];
-        bad |= !isfinite(v);
-        amax = fmaxf(amax, fabsf(v));
-    }
-    if (bad) amax = __builtin_inff();
-    // wave max, then across the four waves
-    amax = max8_f32(amax);
-    amax = fmaxf(amax, dpp_f32<DPP_ROW_MIRROR>(amax));
-    amax = fmaxf(amax, __shfl_xor(amax, 16));
-    amax = fmaxf(amax, __shfl_xor(amax, 32));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
-    __syncthreads();
-    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    // e: amax * 2^-e in [2^14, 2^15); non-finite or zero rows keep e = 0
-    int e = 0;
-    if (amax > 0.0f && isfinite(amax)) e = ilogbf(amax) - 14;
-    if (threadIdx.x == 0) XE[row] = e;
-    for (int c = threadIdx.x; c < k; c += XPREP_THREADS) {
-        const float v = ldexpf(x[c], -e);
-        const _Float16 h = (_Float16)v;
-        XH[(size_t)row * k + c] = h;
-        XL[(size_t)row * k + c] = (_Float16)(v - (float)h);
-    }
-}
-
 // The split of a row held in registers (thread t: elements 4 (t + j NT) ..
 // +3 of v[j], zeros past k): x' = x 2^-e, x_hi = f16(x'), x_lo = f16(x' -
 // x_hi); XS (if not null): the f32 sum of x' over each 32-element block
@@ -299,13 +262,8 @@ struct GemmCfg {
     static constexpr int TJ = WJ * FJ * 16;
     static constexpr int TI = WI * FI * 16;
     static constexpr int CB = KB * KS;                      // blocks per chunk
-    // Q4_0 float mode, 128 x 128 tile: the weights staged as the MFMA's f16
-    // (q - 8) operands, converted once a chunk by the staging threads rather
-    // than by each of the WI waves that read a weight tile
-    static constexpr bool AF16 = !NATIVE && WF == WF_Q4_0 && FJ * FI == 16;
-    // weight rows: 16 nibble bytes a block (Q6_K, Q8_0: 32 codes as bytes;
-    // AF16: 32 f16 operands, the x rows' stride), padded
-    static constexpr int WNS = AF16 ? Lds<CB>::X_STRIDE : wf_bytes(WF) ? CB * 32 + 8 : Lds<CB>::WN_STRIDE;
+    // weight rows: 16 nibble bytes a block (Q6_K, Q8_0: 32 codes as bytes), padded
+    static constexpr int WNS = wf_bytes(WF) ? CB * 32 + 8 : Lds<CB>::WN_STRIDE;
     static constexpr int WN_BYTES = TJ * WNS;
     // Q4_0, Q8_0: the f16 d of each (row, block); Q4_K: f32 pairs {d sc,
     // 8 d sc - dmin mn}; Q6_K: {d sc0, d sc1} of the block's two sub-blocks;
@@ -647,21 +605,9 @@ __global__ __launch_bounds__(WJ * WI * KS * 64) void gemm_q4_0_kernel(
                 lo.y = perm(r.w[u][2], r.w[u][1], sel);
                 hi.x = perm(r.w[u][3], r.w[u][2], sel);
                 hi.y = perm(w4, r.w[u][3], sel);
-                if constexpr (C::AF16) {
-                    // elements 8 g .. 8 g + 7 at 16 g: the low nibbles of bytes
-                    // 0-7, 8-15, then the high ones (rows or blocks past the
-                    // matrix: codes -8 with d = 0)
-                    constexpr uint32_t NIB = 0x0F0F0F0Fu;
-                    half8_t* dst = reinterpret_cast<half8_t*>(wn + jl * C::WNS + bl * 64);
-                    dst[0] = q_f16(lo.x & NIB, lo.y & NIB);
-                    dst[1] = q_f16(hi.x & NIB, hi.y & NIB);
-                    dst[2] = q_f16((lo.x >> 4) & NIB, (lo.y >> 4) & NIB);
-                    dst[3] = q_f16((hi.x >> 4) & NIB, (hi.y >> 4) & NIB);
-                } else {
-                    uint2* dst = reinterpret_cast<uint2*>(wn + jl * Lds<CB>::WN_STRIDE + bl * 16);
-                    dst[0] = lo;
-                    dst[1] = hi;
-                }
+                uint2* dst = reinterpret_cast<uint2*>(wn + jl * Lds<CB>::WN_STRIDE + bl * 16);
+                dst[0] = lo;
+                dst[1] = hi;
                 wd[bl * C::TJ + jl] = (uint16_t)dbits;  // block-major: a lane's four rows are adjacent
             }
         }
@@ -726,8 +672,6 @@ __global__ __launch_bounds__(WJ * WI * KS * 64) void gemm_q4_0_kernel(
                     // lane group g: codes (+ 128) of elements 8 g .. 8 g + 7
                     const uint2 c8 = *reinterpret_cast<const uint2*>(wn + (jt + r16) * C::WNS + bl * 32 + 8 * g);
                     aq[a] = q_f16<128>(c8.x, c8.y);
-                } else if constexpr (C::AF16) {
-                    aq[a] = *reinterpret_cast<const half8_t*>(wn + (jt + r16) * C::WNS + bl * 64 + 16 * g);
                 } else {
                     const uint2 nb8 = *reinterpret_cast<const uint2*>(wn + (jt + r16) * C::WNS + bl * 16 + 8 * (g & 1));
                     const uint32_t sh = (g >> 1) * 4;  // groups 2, 3: high nibbles
@@ -795,19 +739,6 @@ __global__ __launch_bounds__(WJ * WI * KS * 64) void gemm_q4_0_kernel(
                             for (int u = 0; u < 4; u++) acc[a][b][u] = fmaf(dv[a][u], t[u], acc[a][b][u]);
                         }
                     }
-                }
-            }
-            if constexpr (!NATIVE && !SUMS && !Q6 && FI * FJ == 16 && KB == 1) {
-                // the 128 x 128 tile: each tile's two MFMAs followed by four
-                // VALU instructions (the previous tile's scale FMAs).  The
-                // scheduler otherwise issues all 32 of a block's MFMAs first,
-                // keeping every product live at once, and spills (256 -> 230
-                // VGPRs, no scratch; M = 2048 309-313 -> 323-326 TFLOP/s; the
-                // 128 x 64 tile measured 1-2 % slower with it)
-#pragma unroll
-                for (int p = 0; p < FI * FJ; p++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
                 }
             }
         }
@@ -1713,13 +1644,11 @@ hipError_t launch_cfg(const uint8_t* w, int n, int nb, const void* x0, const voi
 }
 
 // Tile choice: enough workgroups for the CUs, then the largest tile (fewest
-// re-reads of x and W from L2).  M >= 256: swept on MI355X at M = 512 and
-// 2048 over tile shapes, waves and chunk sizes, per mode (the native kernel
-// stages half the x bytes and keeps fewer registers).
-// WF_Q4_K: the float shapes, 128 x 64 tiles of one block a wave (or 64 x 64)
-// in place of the 128-row ones; xs the x' block sums.  WF_Q6_K: shapes of at
-// most 64 x 64.  (Their staged headers or codes, scale pairs and masked
-// operands hold more registers: the larger tiles spill.)
+// re-reads of x and W from L2).  Float-mode Q4_0, Q8_0 and the K-quants come
+// here only for short products (gemm_tile_takes); native mode: swept at 512
+// and 2048 rows over tile shapes, waves and chunk sizes.  xs: the x' block
+// sums (Q4_K, Q4_1).  WF_Q6_K: shapes of at most 64 x 64 (its codes, scale pairs
+// and masked operands hold more registers: larger tiles spill).
 template <bool NATIVE, bool DUMP, int WF = WF_Q4_0>
 hipError_t launch_tiles(const uint8_t* w, int n, int nb, const void* x0, const void* x1, const int* xe, int m,
                         float* y, int32_t* p, hipStream_t s, int accy = 0, const float* xs = nullptr) {
@@ -1749,17 +1678,6 @@ hipError_t launch_tiles(const uint8_t* w, int n, int nb, const void* x0, const v
         if constexpr (NATIVE) {
             if (m >= 1024) return launch_cfg<NATIVE, DUMP, WF, 2, 2, 2, 2, 2, 2>(w, n, nb, x0, x1, xe, m, y, p, s, accy, xs);
             if (m >= 256) return launch_cfg<NATIVE, DUMP, WF, 2, 4, 2, 2, 2, 2>(w, n, nb, x0, x1, xe, m, y, p, s, accy, xs);
-        } else if constexpr (WF == WF_Q4_0) {
-            if (m >= 1024) return launch_cfg<NATIVE, DUMP, WF, 4, 4, 2, 2, 2, 1>(w, n, nb, x0, x1, xe, m, y, p, s, accy, xs);
-            // 128 x 128 tiles from m = 128 where they fill three quarters of
-            // the CUs (the 7B prefill's 28672-row gate/up GEMM at 128 rows: 224
-            // tiles, 110 us against 119 us in 128 x 64 tiles); 128 x 64 tiles from
-            // m = 256, and from m = 128 where they alone fill the CUs (prefill
-            // 15.7 -> 12.3 ms; taken for every matrix: 14.9 ms)
-            if (m >= 128 && m < 256 && 4 * (size_t)((n + 127) / 128) * ((m + 127) / 128) >= 3 * (size_t)cus)
-                return launch_cfg<NATIVE, DUMP, WF, 4, 4, 2, 2, 2, 1>(w, n, nb, x0, x1, xe, m, y, p, s, accy, xs);
-            if (m >= 256 || (m >= 128 && (size_t)((n + 127) / 128) * ((m + 63) / 64) >= (size_t)cus))
-                return launch_cfg<NATIVE, DUMP, WF, 4, 2, 2, 2, 2, 2>(w, n, nb, x0, x1, xe, m, y, p, s, accy, xs);
         }
         const size_t t32 = (size_t)((n + 31) / 32) * ((m + 63) / 64);  // 32 x 64 tiles
         if (m >= 48 && t32 >= (size_t)cus) {
@@ -1857,11 +1775,8 @@ hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x
     _Float16* xh = reinterpret_cast<_Float16*>(scratch);
     _Float16* xl = reinterpret_cast<_Float16*>(reinterpret_cast<uint8_t*>(scratch) + xb);
     int* xe = reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(scratch) + 2 * xb);
-    if (k <= (size_t)16 * XPREP_FAST_THREADS)
-        launch_kernel(gemm_xprep_fast_kernel, dim3((unsigned)m), dim3(XPREP_FAST_THREADS), 0, s, x, (int)k, xh, xl,
-                      xe, (float*)nullptr);
-    else
-        launch_kernel(gemm_xprep_kernel, dim3((unsigned)m), dim3(XPREP_THREADS), 0, s, x, (int)k, xh, xl, xe);
+    launch_kernel(gemm_xprep_fast_kernel, dim3((unsigned)m), dim3(XPREP_FAST_THREADS), 0, s, x, (int)k, xh, xl, xe,
+                  (float*)nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return launch_tiles<false, false>(w, (int)n, (int)(k / QK), xh, xl, xe, (int)m, y, nullptr, s);
@@ -1899,10 +1814,8 @@ hipError_t launch_gemm_tiles_ex(WType t, const uint8_t* w, size_t n, size_t k, c
     else if (pro == 2)
         launch_kernel(gemm_xprep_pro_kernel<2>, grid, dim3(XPREP_FAST_THREADS), 0, s, x, (int)k, g, eps, xh, xl, xe,
                       xs);
-    else if (k <= (size_t)16 * XPREP_FAST_THREADS)
-        launch_kernel(gemm_xprep_fast_kernel, grid, dim3(XPREP_FAST_THREADS), 0, s, x, (int)k, xh, xl, xe, xs);
     else
-        launch_kernel(gemm_xprep_kernel, grid, dim3(XPREP_THREADS), 0, s, x, (int)k, xh, xl, xe);
+        launch_kernel(gemm_xprep_fast_kernel, grid, dim3(XPREP_FAST_THREADS), 0, s, x, (int)k, xh, xl, xe, xs);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int accy = accumulate ? 1 : 0;

@@ -53,6 +53,55 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ---- x preparation ---------------------------------------------------------
+// The row exponent e (amax 2^-e in [2^14, 2^15); 0 for a zero or non-finite
+// row) from each thread's maximum of |x| bits.
+template <int NT>
+__device__ __forceinline__ int split_exponent(uint32_t am, uint32_t* red) {
+    am = max8_u32(am);
+    am = max(am, (uint32_t)dpp_i32<DPP_ROW_MIRROR>((int)am));
+    am = max(am, (uint32_t)__shfl_xor((int)am, 16));
+    am = max(am, (uint32_t)__shfl_xor((int)am, 32));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = am;
+    __syncthreads();
+    am = red[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; w++) am = max(am, red[w]);
+    return am != 0 && am < 0x7F800000u ? ilogbf(__builtin_bit_cast(float, am)) - 14 : 0;
+}
+
+// The split of elements 4 p .. 4 p + 3 of a row (p = t modulo 8).  Thread c = t %
+// 8 of a block's eight holds elements 4c .. 4c+3.  Threads c and c ^ 4 trade
+// halves: c < 4 ends with the block's x_hi piece g = c (elements of 4c and 16 +
+// 4c in K order), c >= 4 with the x_lo piece c - 4.  Every thread of a group of
+// eight takes part; p >= k4 stores nothing.
+__device__ __forceinline__ void split_piece(const f32x4& v, int e, int p, int k4, _Float16* xh, _Float16* xl,
+                                            uint32_t* xs) {
+    const bool upper = (threadIdx.x & 4) != 0;
+    _Float16 h[4], l[4];
+    float bs = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const float s = ldexpf(v[t], -e);
+        h[t] = (_Float16)s;
+        l[t] = (_Float16)(s - (float)h[t]);
+        bs += s;
+    }
+    const uint32_t h02 = __builtin_bit_cast(uint32_t, half2_t{h[0], h[2]});
+    const uint32_t h13 = __builtin_bit_cast(uint32_t, half2_t{h[1], h[3]});
+    const uint32_t l02 = __builtin_bit_cast(uint32_t, half2_t{l[0], l[2]});
+    const uint32_t l13 = __builtin_bit_cast(uint32_t, half2_t{l[1], l[3]});
+    const uint32_t r0 = (uint32_t)__shfl_xor((int)(upper ? h02 : l02), 4);
+    const uint32_t r1 = (uint32_t)__shfl_xor((int)(upper ? h13 : l13), 4);
+    const u32x4 o = upper ? u32x4{r0, l02, r1, l13} : u32x4{h02, r0, h13, r1};
+    if (p < k4) *reinterpret_cast<u32x4*>((upper ? xl : xh) + (size_t)(p >> 3) * 32 + (p & 3) * 8) = o;
+    if (xs) {  // the block's sum of x', over 32, as an f16 hi / lo pair
+        bs = sum8_f32(bs) * 0.03125f;
+        const _Float16 sh = (_Float16)bs;
+        const half2_t sp = {sh, (_Float16)(bs - (float)sh)};
+        if ((threadIdx.x & 7) == 0 && p < k4) xs[p >> 3] = __builtin_bit_cast(uint32_t, sp);
+    }
+}
+
 // One workgroup a row: thread t holds elements 4 (t + j NT) .. +3 (k <= 4 NV
 // NT), so x is read once.  PRO 1: RMSNorm first; PRO 2: SwiGLU of rows of 2k
 // interleaved (gate_j, up_j) values.
@@ -61,7 +110,8 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
                                                         const float* __restrict__ g, float eps,
                                                         _Float16* __restrict__ XH, _Float16* __restrict__ XL,
                                                         int* __restrict__ XE, uint32_t* __restrict__ XS) {
-    __shared__ float red[NT / 64], red2[NT / 64];
+    __shared__ uint32_t red[NT / 64];
+    __shared__ float red2[NT / 64];
     const int row = blockIdx.x;
     const int k4 = k >> 2;  // k % 32 == 0
     f32x4 v[NV];
@@ -117,55 +167,32 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
     for (int j = 0; j < NV; j++)
 #pragma unroll
         for (int t = 0; t < 4; t++) am = max(am, abs_bits(v[j][t]));
-    am = max8_u32(am);
-    am = max(am, (uint32_t)dpp_i32<DPP_ROW_MIRROR>((int)am));
-    am = max(am, (uint32_t)__shfl_xor((int)am, 16));
-    am = max(am, (uint32_t)__shfl_xor((int)am, 32));
-    uint32_t* redu = reinterpret_cast<uint32_t*>(red);
-    if ((threadIdx.x & 63) == 0) redu[threadIdx.x >> 6] = am;
-    __syncthreads();
-    am = redu[0];
-#pragma unroll
-    for (int w = 1; w < NT / 64; w++) am = max(am, redu[w]);
-    // e: amax * 2^-e in [2^14, 2^15); non-finite or zero rows keep e = 0
-    int e = 0;
-    if (am != 0 && am < 0x7F800000u) e = ilogbf(__builtin_bit_cast(float, am)) - 14;
+    const int e = split_exponent<NT>(am, red);
     if (threadIdx.x == 0) XE[row] = e;
-    // Thread c = t % 8 of a block's eight holds elements 4c .. 4c+3.  Threads c
-    // and c ^ 4 trade halves: c < 4 ends with the block's x_hi piece g = c
-    // (elements of 4c and 16 + 4c in K order), c >= 4 with the x_lo piece c - 4.
-    const bool upper = (threadIdx.x & 4) != 0;
 #pragma unroll
-    for (int j = 0; j < NV; j++) {
-        const int p = threadIdx.x + j * NT;
-        _Float16 h[4], l[4];
-        float bs = 0.0f;
+    for (int j = 0; j < NV; j++)
+        split_piece(v[j], e, threadIdx.x + j * NT, k4, XH + (size_t)row * k, XL + (size_t)row * k,
+                    XS ? XS + (size_t)row * (k >> 5) : nullptr);
+}
+
+// The split of rows longer than a workgroup's registers hold: two reads of x.
+__global__ __launch_bounds__(1024) void gemm_split_long_kernel(const float* __restrict__ X, int k,
+                                                               _Float16* __restrict__ XH, _Float16* __restrict__ XL,
+                                                               int* __restrict__ XE) {
+    __shared__ uint32_t red[1024 / 64];
+    const int row = blockIdx.x, k4 = k >> 2;
+    const f32x4* x = reinterpret_cast<const f32x4*>(X + (size_t)row * k);
+    uint32_t am = 0;
+    for (int p = threadIdx.x; p < k4; p += 1024) {
+        const f32x4 v = x[p];
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const float s = ldexpf(v[j][t], -e);
-            h[t] = (_Float16)s;
-            l[t] = (_Float16)(s - (float)h[t]);
-            bs += s;
-        }
-        const uint32_t h02 = __builtin_bit_cast(uint32_t, half2_t{h[0], h[2]});
-        const uint32_t h13 = __builtin_bit_cast(uint32_t, half2_t{h[1], h[3]});
-        const uint32_t l02 = __builtin_bit_cast(uint32_t, half2_t{l[0], l[2]});
-        const uint32_t l13 = __builtin_bit_cast(uint32_t, half2_t{l[1], l[3]});
-        const uint32_t r0 = (uint32_t)__shfl_xor((int)(upper ? h02 : l02), 4);
-        const uint32_t r1 = (uint32_t)__shfl_xor((int)(upper ? h13 : l13), 4);
-        const u32x4 o = upper ? u32x4{r0, l02, r1, l13} : u32x4{h02, r0, h13, r1};
-        if (p < k4) {
-            _Float16* dst = (upper ? XL : XH) + (size_t)row * k + (size_t)(p >> 3) * 32 + (p & 3) * 8;
-            *reinterpret_cast<u32x4*>(dst) = o;
-        }
-        if (XS) {  // the block's sum of x', over 32, as an f16 hi / lo pair
-            bs = sum8_f32(bs) * 0.03125f;
-            const _Float16 sh = (_Float16)bs;
-            const half2_t sp = {sh, (_Float16)(bs - (float)sh)};
-            if ((threadIdx.x & 7) == 0 && p < k4)
-                XS[(size_t)row * (k >> 5) + (p >> 3)] = __builtin_bit_cast(uint32_t, sp);
-        }
+        for (int t = 0; t < 4; t++) am = max(am, abs_bits(v[t]));
     }
+    const int e = split_exponent<1024>(am, red);
+    if (threadIdx.x == 0) XE[row] = e;
+    for (int p = threadIdx.x; p - (int)threadIdx.x < k4; p += 1024)
+        split_piece(p < k4 ? x[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f}, e, p, k4, XH + (size_t)row * k,
+                    XL + (size_t)row * k, nullptr);
 }
 
 // ---- GEMM --------------------------------------------------------------------
@@ -1016,7 +1043,12 @@ TilePlan tile_plan(WType t, size_t m, size_t n, size_t nb, bool can_split) {
 
 template <int PRO>
 hipError_t launch_split(const float* x, size_t m, size_t k, const float* g, float eps, const XSplit& o, hipStream_t s) {
-    // 256 threads hold 4096 elements of a row, 1024 threads 16384
+    // 256 threads hold 4096 elements of a row, 1024 threads GEMM_SPLIT_MAX_K
+    if (k > GEMM_SPLIT_MAX_K) {
+        if (PRO != 0 || o.s) return hipErrorInvalidValue;
+        launch_kernel(gemm_split_long_kernel, dim3((unsigned)m), dim3(1024), 0, s, x, (int)k, o.h, o.l, o.e);
+        return hipGetLastError();
+    }
     if (k <= 4096)
         launch_kernel(gemm_split_kernel<PRO, 256, 4>, dim3((unsigned)m), dim3(256), 0, s, x, (int)k, g, eps, o.h, o.l,
                       o.e, o.s);
@@ -1038,8 +1070,8 @@ hipError_t launch_split(const float* x, size_t m, size_t k, const float* g, floa
 // 4096 x 4096 19.5 / 17.3, 16 x 14336 x 1024 17.6 / 24.1, 500 x 4096 x 1024 23.4 / 26.8,
 // 211 x 4096 x 1024 19.7 / 17.4; Q6_K alike).
 bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k) {
-    if (k > GEMM_TILE_MAX_K) return false;
-    if (t == WType::Q4_0) return m > GEMM_XTILE_M && !(m <= 256 && k <= 2048 && n * k <= (size_t)1 << 22);
+    if (t == WType::Q4_0) return m > GEMM_XTILE_M && !(m < 256 && n <= 4096 && k <= 2048 && n * k <= (size_t)1 << 22);
+    if (k > GEMM_SPLIT_MAX_K) return false;
     if (t == WType::Q4_K || t == WType::Q6_K) {
         if (n >= 8192) return m >= KQ_GEMM_MIN_M;
         return m >= 32 && (k >= 4096 || (m >= 128 && k >= 2048 && n >= 2048) || m * n >= (size_t)3 << 19);
@@ -1072,7 +1104,7 @@ static hipError_t launch_tile_wf(WType t, const uint8_t* w, int n, int nb, const
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
                             hipStream_t s) {
-    if (k == 0 || !gemm_tile_takes(t, m, n, k)) return hipErrorInvalidValue;
+    if (k == 0 || !gemm_tile_takes(t, m, n, k) || (pro != 0 && k > GEMM_SPLIT_MAX_K)) return hipErrorInvalidValue;
     const XSplit xo = x_split_at(scratch, m, k, t == WType::Q4_K);
     const hipError_t e = pro == 1   ? launch_split<1>(x, m, k, g, eps, xo, s)
                          : pro == 2 ? launch_split<2>(x, m, k, g, eps, xo, s)

@@ -196,10 +196,10 @@ hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x
 // True when workgroup b of a launch runs on XCD (b + o) % 8 on the current
 // device (gemm.hip).
 bool xcd_round_robin(hipStream_t s);
-// The tile GEMM (gemm_tiles.hip; arguments as launch_gemm_tiles_ex, k <=
-// GEMM_TILE_MAX_K): its K-slice partials take gemm_part_bytes(t, m, n, k), at
+// The tile GEMM (gemm_tiles.hip; arguments as launch_gemm_tiles_ex; rows
+// past GEMM_SPLIT_MAX_K: Q4_0 without a prologue): its K-slice partials take gemm_part_bytes(t, m, n, k), at
 // most GEMM_PART_BYTES, and one counter a tile of at most GEMM_SPLIT_TILES.
-constexpr size_t GEMM_TILE_MAX_K = 16384;
+constexpr size_t GEMM_SPLIT_MAX_K = 16384;
 constexpr size_t GEMM_PART_BYTES = 16u << 20;
 constexpr size_t GEMM_SPLIT_TILES = 256;
 size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k);
