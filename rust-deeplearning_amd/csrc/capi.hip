@@ -171,10 +171,11 @@ bool use_fused(WType t, size_t m, size_t n, size_t k, const float* x_dev) {
 }
 
 // How a product runs: one fused GEMV launch (m <= 4), the matrix-core GEMM
-// (Q4_0, more rows: f16 MFMA in float mode, int8 MFMA in native mode; Q4_K,
+// (Q4_0, more rows: f16 MFMA in float mode, int8 MFMA in native mode, or f16
+// MFMA on what the Q8_0 codes and scales give (NativeTile); Q4_K,
 // Q6_K, Q8_0 and float-mode Q4_1 from KQ_GEMM_MIN_M rows), or activation
 // records + the records GEMV.
-enum class Path { Fused, Gemm, Records };
+enum class Path { Fused, Gemm, NativeTile, Records };
 
 // The GEMM addresses x and W with 32-bit offsets; the x prep of the other
 // types holds a row in registers (k <= 16384).
@@ -190,8 +191,8 @@ bool gemm_fits(WType t, bool native, size_t m, size_t n, size_t k) {
 
 Path pick_path(WType t, bool native, size_t m, size_t n, size_t k, const float* x_dev) {
     if (use_fused(t, m, n, k, x_dev)) return Path::Fused;
-    if (gemm_fits(t, native, m, n, k)) return Path::Gemm;
-    return Path::Records;
+    if (!gemm_fits(t, native, m, n, k)) return Path::Records;
+    return native && rdl::gemm_native_tile_takes(m, n, k) ? Path::NativeTile : Path::Gemm;
 }
 
 size_t scratch_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
@@ -199,6 +200,7 @@ size_t scratch_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k)
         case Path::Fused: return 0;
         case Path::Gemm:
             return t == WType::Q4_0 ? rdl::gemm_scratch_bytes(m, n, k, native) : rdl::gemm_tiles_scratch_bytes(m, k);
+        case Path::NativeTile: return rdl::gemm_scratch_bytes(m, n, k, false);
         case Path::Records: return rec_bytes(native, m, k);
     }
     return 0;
@@ -206,7 +208,8 @@ size_t scratch_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k)
 
 // The tile GEMM's K-slice partials (beside scratch_bytes).
 size_t part_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
-    return p == Path::Gemm && !native && rdl::gemm_tile_takes(t, m, n, k) ? rdl::gemm_part_bytes(t, m, n, k) : 0;
+    const bool tile = p == Path::NativeTile || (p == Path::Gemm && !native && rdl::gemm_tile_takes(t, m, n, k));
+    return tile ? rdl::gemm_part_bytes(t, m, n, k) : 0;
 }
 // Whether the path counts K slices (the Q4_0 x-tile kernel, split tile GEMMs).
 bool wants_counters(WType t, Path p, bool native, size_t m, size_t n, size_t k) {
@@ -227,6 +230,11 @@ rdl_status run_linear(WType t, bool native, const uint8_t* w_dev, size_t n, size
     }
     if (path == Path::Fused) {
         HIP_TRY(rdl::launch_gemv_fused(t, native, w_dev, n, k, x_dev, m, y_dev, s));
+        return RDL_OK;
+    }
+    if (path == Path::NativeTile) {
+        HIP_TRY(rdl::launch_gemm_tile(t, w_dev, n, k, x_dev, m, y_dev, work, part, counters, 3, nullptr, 0.0f, false,
+                                      s));
         return RDL_OK;
     }
     if (path == Path::Gemm) {
@@ -689,8 +697,12 @@ rdl_status rdl_linear_forward_dev_noalloc(const rdl_weight* w, const float* x_de
     if (m == 0 || w->n == 0) return ok();
     if (!x_dev || !y_dev) return fail(RDL_ERR_NULL_POINTER, "NULL activation pointer");
     const bool native = mode == RDL_MODE_NATIVE && (w->type == WType::Q4_0 || w->type == WType::Q4_1);
-    const Path path = pick_path(w->type, native, m, w->n, w->k, x_dev);
-    const size_t rb = scratch_bytes(w->type, path, native, m, w->n, w->k);
+    Path path = pick_path(w->type, native, m, w->n, w->k, x_dev);
+    size_t rb = scratch_bytes(w->type, path, native, m, w->n, w->k);
+    if (path == Path::NativeTile && rb > NOALLOC_DATA_BYTES) {  // int8 codes take a quarter of its x split
+        path = Path::Gemm;
+        rb = scratch_bytes(w->type, path, native, m, w->n, w->k);
+    }
     if (rb > NOALLOC_DATA_BYTES)
         return fail(RDL_ERR_UNSUPPORTED,
                     "m=%zu rows of in_features %zu need %zu scratch bytes; the static scratch holds %zu",

@@ -51,6 +51,7 @@ struct TilePlan {
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // x rows start on any float
 
 // ---- x preparation ---------------------------------------------------------
 // The row exponent e (amax 2^-e in [2^14, 2^15); 0 for a zero or non-finite
@@ -104,7 +105,8 @@ __device__ __forceinline__ void split_piece(const f32x4& v, int e, int p, int k4
 
 // One workgroup a row: thread t holds elements 4 (t + j NT) .. +3 (k <= 4 NV
 // NT), so x is read once.  PRO 1: RMSNorm first; PRO 2: SwiGLU of rows of 2k
-// interleaved (gate_j, up_j) values.
+// interleaved (gate_j, up_j) values; PRO 3: x as its Q8_0 blocks hold it
+// (quantize_row_q8_0, quantize.rs:164-193).
 template <int PRO, int NT, int NV>
 __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict__ X, int k,
                                                         const float* __restrict__ g, float eps,
@@ -116,7 +118,7 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
     const int k4 = k >> 2;  // k % 32 == 0
     f32x4 v[NV];
     if constexpr (PRO == 2) {
-        const f32x4* x = reinterpret_cast<const f32x4*>(X + (size_t)row * 2 * k);
+        const f32x4u* x = reinterpret_cast<const f32x4u*>(X + (size_t)row * 2 * k);
         auto silu_mul = [](float gv, float uv) {
             const float sig = 1.0f / (1.0f + expf(-gv));
             return (gv * sig) * uv;
@@ -132,11 +134,30 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
             }
         }
     } else {
-        const f32x4* x = reinterpret_cast<const f32x4*>(X + (size_t)row * k);
+        const f32x4u* x = reinterpret_cast<const f32x4u*>(X + (size_t)row * k);
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             const int p = threadIdx.x + j * NT;
-            v[j] = p < k4 ? x[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            v[j] = p < k4 ? (f32x4)x[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    if constexpr (PRO == 3) {
+        // code times scale, 7 + 11 bits: exact in f32, and in the hi / lo pair of a
+        // block within 2^-21 of the row's largest; a NaN scores as 0 in the block
+        // maximum and as code 0, an overflowing scale makes the block NaN
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            float am = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 4; t++) am = fmaxf(am, fabsf(v[j][t]));
+            am = max8_f32(am);
+            const float rt = h2f(f2h_rne(am == 0.0f ? 0.0f : am / 127.0f));
+            const float inv = rt == 0.0f ? 0.0f : 1.0f / rt;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float q = roundf(v[j][t] * inv);
+                v[j][t] = (q != q ? 0.0f : fminf(fmaxf(q, -128.0f), 127.0f)) * rt;
+            }
         }
     }
     if constexpr (PRO == 1) {
@@ -181,17 +202,17 @@ __global__ __launch_bounds__(1024) void gemm_split_long_kernel(const float* __re
                                                                int* __restrict__ XE) {
     __shared__ uint32_t red[1024 / 64];
     const int row = blockIdx.x, k4 = k >> 2;
-    const f32x4* x = reinterpret_cast<const f32x4*>(X + (size_t)row * k);
+    const f32x4u* x = reinterpret_cast<const f32x4u*>(X + (size_t)row * k);
     uint32_t am = 0;
     for (int p = threadIdx.x; p < k4; p += 1024) {
-        const f32x4 v = x[p];
+        const f32x4 v = (f32x4)x[p];
 #pragma unroll
         for (int t = 0; t < 4; t++) am = max(am, abs_bits(v[t]));
     }
     const int e = split_exponent<1024>(am, red);
     if (threadIdx.x == 0) XE[row] = e;
     for (int p = threadIdx.x; p - (int)threadIdx.x < k4; p += 1024)
-        split_piece(p < k4 ? x[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f}, e, p, k4, XH + (size_t)row * k,
+        split_piece(p < k4 ? (f32x4)x[p] : f32x4{0.0f, 0.0f, 0.0f, 0.0f}, e, p, k4, XH + (size_t)row * k,
                     XL + (size_t)row * k, nullptr);
 }
 
@@ -1060,6 +1081,21 @@ hipError_t launch_split(const float* x, size_t m, size_t k, const float* g, floa
 
 }  // namespace
 
+// Native mode (x as Q8_0 blocks hold it, the same codes and scales times the
+// same blocks): the int8 kernel of gemm.hip forms sx d and scales every int32
+// dot, three VALU instructions a result where one FMA does here, and its tiles
+// are not split over K (us, int8 kernel / here: 512 x 14336 x 4096 184 / 114,
+// 512 x 4096 x 14336 171 / 134, 2048 x 14336 x 4096 601 / 448, 65 x 4096 x 4096 25.3 /
+// 22.4, 128 x 14336 x 4096 88 / 42, 256 x 1024 x 4096 50 / 21.5, 1024 x 64 x 4096 46 /
+// 25).  It keeps short products over small matrices (128 x 2048 x 2048 10.6 / 15.4,
+// 200 x 1024 x 4096 17.4 / 19.3, 1024 x 512 x 992 15.4 / 17) and rows past one
+// workgroup's registers.
+bool gemm_native_tile_takes(size_t m, size_t n, size_t k) {
+    if (m <= GEMM_XTILE_M || k > GEMM_SPLIT_MAX_K) return false;
+    if (m < 256) return n * k >= (size_t)1 << 24;
+    return m < 1024 || n >= 2048 || k >= 2048;
+}
+
 // The small-tile kernel of gemm.hip keeps short products over small matrices:
 // its 16 x 32 tiles reach all CUs without a split over K, and its code is
 // smaller (us, here against there: Q4_0 100 x 512 x 992 10.7 / 9.1, 200 x 2048 x
@@ -1104,10 +1140,13 @@ static hipError_t launch_tile_wf(WType t, const uint8_t* w, int n, int nb, const
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
                             hipStream_t s) {
-    if (k == 0 || !gemm_tile_takes(t, m, n, k) || (pro != 0 && k > GEMM_SPLIT_MAX_K)) return hipErrorInvalidValue;
+    if (pro == 3 ? t != WType::Q4_0 || k == 0 || !gemm_native_tile_takes(m, n, k)
+                 : k == 0 || !gemm_tile_takes(t, m, n, k) || (pro != 0 && k > GEMM_SPLIT_MAX_K))
+        return hipErrorInvalidValue;
     const XSplit xo = x_split_at(scratch, m, k, t == WType::Q4_K);
     const hipError_t e = pro == 1   ? launch_split<1>(x, m, k, g, eps, xo, s)
                          : pro == 2 ? launch_split<2>(x, m, k, g, eps, xo, s)
+                         : pro == 3 ? launch_split<3>(x, m, k, g, eps, xo, s)
                                     : launch_split<0>(x, m, k, g, eps, xo, s);
     if (e != hipSuccess) return e;
     const int ni = (int)n, nb = (int)(k / QK), mi = (int)m, acc = accumulate ? 1 : 0;

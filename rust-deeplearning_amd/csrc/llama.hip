@@ -701,6 +701,9 @@ struct LlamaModel {
     hipError_t linear(const Mat& w, const float* xin, size_t m, float* y, bool native = false) {
         native = native && (w.type == WType::Q4_0 || w.type == WType::Q4_1);
         if (m <= 4) return launch_gemv_fused(w.type, native, w.dev, w.n, w.k, xin, m, y, stream);
+        if (w.type == WType::Q4_0 && native && gemm_native_tile_takes(m, w.n, w.k))
+            return launch_gemm_tile(w.type, w.dev, w.n, w.k, xin, m, y, gemm_scratch, gemm_part, gemm_cnt, 3, nullptr,
+                                    0.0f, false, stream);
         if (w.type == WType::Q4_0)
             return native ? launch_gemm_q4_0_native(w.dev, w.n, w.k, xin, m, y, nullptr, gemm_scratch, stream)
                           : launch_gemm_q4_0(w.dev, w.n, w.k, xin, m, y, gemm_scratch, gemm_part, gemm_cnt, stream);

@@ -207,6 +207,9 @@ size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k);
 // rows, Q8_0 from KQ_GEMM_MIN_M): where it is faster than the small-tile
 // kernel of gemm.hip.
 bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k);
+// Whether a native-mode Q4_0 product takes it (launch_gemm_tile with pro 3,
+// scratch gemm_scratch_bytes(m, n, k, false)).
+bool gemm_native_tile_takes(size_t m, size_t n, size_t k);
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
                             hipStream_t s);

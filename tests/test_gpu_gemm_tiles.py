@@ -106,3 +106,42 @@ def test_split_tiles_combines_and_replays_agree(rq, gpu, m, n, k):
         product(main)
         torch.cuda.synchronize()
     w.free()
+
+
+# native mode past 64 rows: the smallest product that takes the tiles below 256
+# rows, ragged tiles and slices, odd block counts, and both sides of 256 and
+# 1024 rows and of k = 16384 (the int8 kernel)
+@pytest.mark.parametrize("m,n,k", [(65, 4096, 4096), (65, 4093, 4128), (255, 100, 4096), (256, 1, 32), (300, 257, 544),
+                                   (513, 130, 4128), (1024, 64, 2080), (1030, 2049, 96), (257, 33, 16384),
+                                   (257, 33, 16416)])
+def test_native_tiles(rq, orc, gpu, m, n, k):
+    print(f"case native tiles m={m} n={n} k={k}", flush=True)
+    x = synth.activations(m, k, m + n + k)
+    w = synth.q4_0_weights(n, k, m + n)
+    got = rq.matmul_f32_q4_native(x, w, m, k, n).reshape(m, n)
+    rows = np.unique(np.linspace(0, m - 1, 12).astype(int))
+    want = orc.matmul("q4_native", x[rows], w, len(rows), k, n, 16)
+    part = orc.block_dots(x[rows], w, len(rows), k, n).reshape(len(rows), n, k // 32).astype(np.float64)
+    sw = w.reshape(n, k // 32, 18)[:, :, 0:2].copy().view(np.float16).astype(np.float64)[..., 0]
+    sx = np.stack([orc.quantize_row_q8_0(x[r])[1] for r in rows]).astype(np.float64)
+    check_parity(got[rows].reshape(-1), want, (part * sx[:, None, :] * sw[None]).sum(axis=2).reshape(-1))
+
+
+def test_native_tiles_nan_inf_and_zero_rows(rq, orc, gpu):
+    # NaN scores as code 0 and a zero block as scale 0; an overflowing block
+    # scale makes every output of its row NaN, as in the reference
+    m, n, k = 300, 70, 512
+    x = synth.activations(m, k, 95)
+    x[2, 5], x[4], x[7, 40], x[9, 300] = np.nan, 0.0, np.inf, 1e9
+    x[11] *= 1e-7
+    w = synth.q4_0_weights(n, k, 96)
+    rows = np.array([0, 2, 4, 7, 9, 11, 12])
+    got = rq.matmul_f32_q4_native(x, w, m, k, n).reshape(m, n)
+    want = orc.matmul("q4_native", x[rows], w, len(rows), k, n, 4).reshape(len(rows), n)
+    assert np.array_equal(np.isnan(got[rows]), np.isnan(want))
+    ok = ~np.isnan(want)
+    # 2^-22 of a split x element and f32 sums of 16 blocks, over sum |w x| <= 16 x
+    # the largest output of a row here
+    tol = 1e-6 * 16 * np.abs(np.where(ok, want, 0.0)).max(axis=1, keepdims=True) * np.ones_like(want)
+    assert np.all(np.abs(got[rows] - want)[ok] <= tol[ok])
+    assert np.isfinite(np.delete(got, [7, 9], axis=0)).all()
