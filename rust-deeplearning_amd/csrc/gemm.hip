@@ -1481,7 +1481,13 @@ __global__ __launch_bounds__(XT_WAVES * 64) void gemm_q4_0_xtile_kernel(
 // Launch plan of the x-tile kernel: 128-row strips, S K-slices of kbs
 // blocks (even when nb is) for about one workgroup per CU, KB the template
 // bound of kbs (8, 16 or 32; at most 16 with more than one x tile, for the
-// LDS).  ok = false (the skinny kernel runs) when a slice would exceed that.
+// LDS).  With one x tile, slices of 16 let three workgroups share a CU, where
+// the loads of one cover the x split and the sums of the others: 16 x 14336 x 4096
+// 28.5 -> 23.0 us, 11008 x 4096 27.4 -> 19.5, 8192 x 4096 15.4 -> 14.1, 4096 x 14336 30.0 ->
+// 26.9.  Slices of 32 stay where they fill one round in one slice (32000 x 1024 11.5
+// against 12.2) or in eight and more, whose partials cost more (4096 x 8192 15.8 against
+// 16.5), and where the partials would pass 12 MB (they share a 16 MB scratch).
+// ok = false (the skinny kernel runs) when a slice would exceed the bound.
 struct XtPlan {
     int strips, S, kbs, KB;
     bool even, ok;
@@ -1489,13 +1495,18 @@ struct XtPlan {
 inline XtPlan xtile_plan(size_t n, int nb, int mt = 1) {
     // LDS per workgroup: 2 * 16 mt * (64 KB + 16) + 64 KB mt bytes; at most 16
     // blocks a slice when mt > 1
-    const int kmax = mt > 1 ? 16 : 32;
+    const int cus = device_cu_count(), kmax = mt > 1 ? 16 : 32;
     XtPlan p{};
     p.strips = (int)((n + XT_ROWS - 1) / XT_ROWS);
-    const int S = std::max(1, (device_cu_count() + p.strips / 2) / p.strips);
+    const int S = std::max(1, (cus + p.strips / 2) / p.strips);
     p.kbs = std::max(1, (nb + S - 1) / S);
     p.kbs = std::min(p.kbs, kmax);
     p.even = nb % 2 == 0;
+    if (p.kbs > 16) {
+        const int S32 = (nb + p.kbs - 1) / p.kbs, S16 = (nb + 15) / 16;
+        const bool one_round = (size_t)p.strips * S32 <= (size_t)cus && S32 >= 8;
+        if (S32 > 1 && !one_round && (size_t)p.strips * S16 * XT_UNITS * 16 <= (size_t)12 << 20) p.kbs = 16;
+    }
     if (p.even) p.kbs += p.kbs & 1;
     p.S = std::max(1, (nb + p.kbs - 1) / p.kbs);  // no empty slices
     p.KB = p.kbs <= 8 ? 8 : p.kbs <= 16 ? 16 : 32;
@@ -1734,12 +1745,13 @@ hipError_t launch_zero_counters(int* counters, size_t count, hipStream_t s) {
 size_t gemm_counter_count(size_t n, size_t) { return std::max((n + 63) / 64 + 1, GEMM_SPLIT_TILES); }
 
 size_t gemm_scratch_bytes(size_t m, size_t n, size_t k, bool native) {
-    if (!native && m >= 1 && m <= GEMM_XTILE_M) {  // the K-slice partials of the x-tile kernel
+    const bool few = !native && m <= GEMM_XTILE_M && !gemm_tile_takes(WType::Q4_0, m, n, k);
+    if (few && m >= 1) {  // the K-slice partials of the x-tile kernel
         const int mt = (int)((m + 15) / 16);
         const XtPlan p = xtile_plan(n, (int)(k / QK), mt);
         if (p.ok) return p.S > 1 ? ((size_t)p.strips * p.S * XT_UNITS * mt * 16 + 255) & ~(size_t)255 : 0;
     }
-    if (!native && m <= GEMM_SMALL_M) {  // the K-slice partials of the skinny GEMM
+    if (few) {  // the K-slice partials of the skinny GEMM
         if (m == 0 || n == 0) return 0;
         const SkPlan p = skinny_plan(m, n, (int)(k / QK), true);
         return p.S > 1 ? ((size_t)p.strips * p.S * p.units * 16 + 255) & ~(size_t)255 : 0;

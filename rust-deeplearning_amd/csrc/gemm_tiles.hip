@@ -51,11 +51,16 @@ struct TilePlan {
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // x rows start on any float
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // x and y start on any float
 
 // ---- x preparation ---------------------------------------------------------
-// The row exponent e (amax 2^-e in [2^14, 2^15); 0 for a zero or non-finite
-// row) from each thread's maximum of |x| bits.
+// |x| bits of a finite x, else 0.
+__device__ __forceinline__ uint32_t finite_bits(float x) {
+    const uint32_t b = abs_bits(x);
+    return b < 0x7F800000u ? b : 0u;
+}
+// The row exponent e (amax 2^-e in [2^14, 2^15); 0 for a row of zeros) from
+// each thread's maximum of its finite |x| bits.
 template <int NT>
 __device__ __forceinline__ int split_exponent(uint32_t am, uint32_t* red) {
     am = max8_u32(am);
@@ -67,7 +72,7 @@ __device__ __forceinline__ int split_exponent(uint32_t am, uint32_t* red) {
     am = red[0];
 #pragma unroll
     for (int w = 1; w < NT / 64; w++) am = max(am, red[w]);
-    return am != 0 && am < 0x7F800000u ? ilogbf(__builtin_bit_cast(float, am)) - 14 : 0;
+    return am != 0 ? ilogbf(__builtin_bit_cast(float, am)) - 14 : 0;
 }
 
 // The split of elements 4 p .. 4 p + 3 of a row (p = t modulo 8).  Thread c = t %
@@ -84,7 +89,7 @@ __device__ __forceinline__ void split_piece(const f32x4& v, int e, int p, int k4
     for (int t = 0; t < 4; t++) {
         const float s = ldexpf(v[t], -e);
         h[t] = (_Float16)s;
-        l[t] = (_Float16)(s - (float)h[t]);
+        l[t] = (_Float16)(fabsf(s) == INFINITY ? 0.0f : s - (float)h[t]);  // (an infinite x: no inf - inf)
         bs += s;
     }
     const uint32_t h02 = __builtin_bit_cast(uint32_t, half2_t{h[0], h[2]});
@@ -182,12 +187,12 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
             if (p < k4) v[j] = (v[j] * inv) * g4[p];
         }
     }
-    // largest |x| of the row as an integer maximum of |x| bits (non-finite on top)
+    // largest finite |x| of the row as an integer maximum of |x| bits
     uint32_t am = 0;
 #pragma unroll
     for (int j = 0; j < NV; j++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) am = max(am, abs_bits(v[j][t]));
+        for (int t = 0; t < 4; t++) am = max(am, finite_bits(v[j][t]));
     const int e = split_exponent<NT>(am, red);
     if (threadIdx.x == 0) XE[row] = e;
 #pragma unroll
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(1024) void gemm_split_long_kernel(const float* __re
     for (int p = threadIdx.x; p < k4; p += 1024) {
         const f32x4 v = (f32x4)x[p];
 #pragma unroll
-        for (int t = 0; t < 4; t++) am = max(am, abs_bits(v[t]));
+        for (int t = 0; t < 4; t++) am = max(am, finite_bits(v[t]));
     }
     const int e = split_exponent<1024>(am, red);
     if (threadIdx.x == 0) XE[row] = e;
@@ -866,8 +871,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
             float* yp = Y + (size_t)i * n + j;
             // accy: y += the product (the residual add, one rounding as x + y)
             if (j + 3 < n && (n & 3) == 0) {
-                if (accy) v = *reinterpret_cast<const f32x4*>(yp) + v;
-                *reinterpret_cast<f32x4*>(yp) = v;
+                if (accy) v = (f32x4)*reinterpret_cast<const f32x4u*>(yp) + v;
+                *reinterpret_cast<f32x4u*>(yp) = v;
             } else {
 #pragma unroll
                 for (int q = 0; q < 4; q++)
@@ -1105,7 +1110,23 @@ bool gemm_native_tile_takes(size_t m, size_t n, size_t k) {
 // 2048 x 2048 16.5 / 14.7, 128 x 2048 x 2048 18.5 / 19.1, 32 x 512 x 4096 17.3 / 22.3, 16 x
 // 4096 x 4096 19.5 / 17.3, 16 x 14336 x 1024 17.6 / 24.1, 500 x 4096 x 1024 23.4 / 26.8,
 // 211 x 4096 x 1024 19.7 / 17.4; Q6_K alike).
+// Q4_0 calls of 5 to 64 rows have the x-tile kernel, one launch that splits x in
+// every strip of 128 weight rows.  The tiles compute 64 rows whatever m is, but
+// split x once: they take matrices of many strips or long rows, and short wide
+// ones whose few strips leave CUs idle there (us, here / x-tile kernel: 16 x 32000
+// x 4096 38 / 44, 16 x 14336 x 4096 27 / 23, 16 x 512 x 4096 12.8 / 14.8; 32 x 32000 x
+// 4096 39 / 53, 32 x 4096 x 14336 29.6 / 33.1, 32 x 9000 x 7168 31.6 / 30.4, 32 x 11008
+// x 4096 26.6 / 23.9, 32 x 64 x 4096 12.6 / 16.3; 33 x 6144 x 4096 19.8 / 24.2, 64 x
+// 14336 x 4096 28.6 / 54, 64 x 4096 x 14336 31 / 65, 33 x 4096 x 4096 17.1 / 14.9, 33 x
+// 1024 x 4096 14.2 / 16.5, 33 x 4096 x 2048 13.4 / 10.3).
 bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k) {
+    if (t == WType::Q4_0 && m <= GEMM_XTILE_M) {
+        if (k > GEMM_SPLIT_MAX_K) return false;
+        const size_t nk = n * k;
+        if (m <= 16) return nk >= (size_t)3 << 25 || (n <= 512 && nk >= (size_t)1 << 21);
+        if (m <= 32) return nk >= (size_t)3 << 25 || (nk >= (size_t)3 << 24 && k >= 2 * n) || (n <= 512 && nk >= (size_t)1 << 18);
+        return nk > (size_t)1 << 24 || (nk >= (size_t)1 << 18 && (n <= 512 || (n <= 1024 && nk <= (size_t)1 << 22)));
+    }
     if (t == WType::Q4_0) return m > GEMM_XTILE_M && !(m < 256 && n <= 4096 && k <= 2048 && n * k <= (size_t)1 << 22);
     if (k > GEMM_SPLIT_MAX_K) return false;
     if (t == WType::Q4_K || t == WType::Q6_K) {

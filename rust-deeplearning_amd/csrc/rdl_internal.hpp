@@ -203,8 +203,8 @@ constexpr size_t GEMM_SPLIT_MAX_K = 16384;
 constexpr size_t GEMM_PART_BYTES = 16u << 20;
 constexpr size_t GEMM_SPLIT_TILES = 256;
 size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k);
-// Whether a float-mode product takes the tile GEMM (Q4_0 beyond GEMM_XTILE_M
-// rows, Q8_0 from KQ_GEMM_MIN_M): where it is faster than the small-tile
+// Whether a float-mode product takes the tile GEMM (Q4_0 past the fused GEMV's
+// rows, the other types from KQ_GEMM_MIN_M): where it is faster than the small-tile
 // kernel of gemm.hip.
 bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k);
 // Whether a native-mode Q4_0 product takes it (launch_gemm_tile with pro 3,

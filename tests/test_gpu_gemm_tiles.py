@@ -30,6 +30,36 @@ def test_tiles(rq, orc, gpu, kind, dtype, m, n, k):
     check_parity(got[rows].reshape(-1), want, exact_f64(orc, kind, x[rows], w, len(rows), k, n))
 
 
+# 5 to 64 rows on the tiles: matrices of many strips and of few, ragged, each
+# side of 16 and 32 rows; and the x-tile kernel's slices of 16 (many strips; a
+# ragged last slice; an odd block count) and of 32 (one round)
+@pytest.mark.parametrize("m,n,k", [(5, 24601, 4096), (16, 500, 4224), (17, 510, 544), (31, 4090, 13344), (32, 64, 4096), (33, 4100, 4128),
+                                   (64, 1000, 2080), (64, 1, 16384), (16, 8200, 4096), (9, 2050, 14368),
+                                   (5, 6150, 2080), (16, 4096, 8192)])
+def test_few_rows(rq, orc, gpu, m, n, k):
+    print(f"case few rows m={m} n={n} k={k}", flush=True)
+    x = synth.activations(m, k, m + n + k)
+    w = synth.q4_0_weights(n, k, m + n)
+    got = rq.matmul_f32_q4(x, w, m, k, n).reshape(m, n)
+    rows = np.unique(np.linspace(0, m - 1, 8).astype(int))
+    want = orc.matmul("q4", x[rows], w, len(rows), k, n, threads=16)
+    check_parity(got[rows].reshape(-1), want, exact_f64(orc, "q4", x[rows], w, len(rows), k, n))
+
+
+@pytest.mark.parametrize("m", [20, 40, 300])
+def test_rows_with_an_infinite_value(rq, orc, gpu, m):
+    # +-inf where the weight is not zero, NaN where it is, as in the reference;
+    # rows beside it and a row's own finite values keep theirs
+    n, k = 300, 1024
+    x = synth.activations(m, k, 21 + m)
+    x[3, 77], x[5, 900] = np.inf, -np.inf
+    w = synth.q4_0_weights(n, k, 22)
+    got = rq.matmul_f32_q4(x, w, m, k, n).reshape(m, n)
+    want = orc.matmul("q4", x[[3, 5]], w, 2, k, n).reshape(2, n)
+    assert np.array_equal(got[[3, 5]], want, equal_nan=True)
+    assert np.isfinite(np.delete(got, [3, 5], axis=0)).all()
+
+
 # one 16-row x tile and just past one, both sides of the 128-row weight tiles,
 # one super-block a row and 17 (the last slice shorter), odd super-block counts
 # (Q6_K rows starting 2 bytes past a dword), the K split, a partial last round
