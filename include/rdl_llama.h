@@ -88,6 +88,19 @@ rdl_status rdl_llama_create(const rdl_llama_config* cfg, rdl_llama** out);
 rdl_status rdl_llama_create_typed(const rdl_llama_config* cfg, const int32_t* types, rdl_llama** out);
 rdl_status rdl_llama_free(rdl_llama* model);
 
+/* Device memory planning, no reference counterpart and no device needed:
+ * rdl_llama_gemm_scratch reports the bytes of GEMM work memory (activation
+ * splits and codes, K-slice partials of the few-row kernels) that a model of
+ * this configuration allocates, rdl_llama_product_scratch the bytes that one
+ * product of `rows` activation rows with an out_features x in_features matrix
+ * of a GGUF type writes there (mode: RDL_MODE_*, native for a layer under
+ * rdl_llama_set_native_q4).  The model's matrices are [Wq; Wk; Wv] and [gate;
+ * up] where the parts share a type, [Wq; Wk] where only Wv differs, the
+ * others as they are; a chunk of any of max_batch rows fits. */
+rdl_status rdl_llama_gemm_scratch(const rdl_llama_config* cfg, const int32_t* types, size_t* bytes);
+rdl_status rdl_llama_product_scratch(int32_t dtype, size_t rows, size_t out_features, size_t in_features,
+                                     int32_t mode, size_t* bytes);
+
 /* Copies one weight from host memory (len must equal the slot's size). */
 rdl_status rdl_llama_set_weight(rdl_llama* model, int32_t slot, int32_t layer, const void* bytes,
                                 size_t len);

@@ -23,9 +23,11 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <exception>
 #include <string>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <type_traits>
 #include <vector>
 
@@ -647,6 +649,7 @@ struct LlamaModel {
     int *tokens = nullptr, *pos = nullptr, *step = nullptr, *out_tokens = nullptr;
     size_t out_cap = 0;
     void* gemm_scratch = nullptr;
+    size_t gemm_scratch_cap = 0;  // its bytes: gemm_scratch_need()
     float* gemm_part = nullptr;  // the tile GEMM's K-slice partials
     int* gemm_cnt = nullptr;     // the split GEMMs' strip and tile counters (zero between launches)
     float* att_part = nullptr;  // [max_batch][n_heads][spans of max_seq][hd + 2]
@@ -696,11 +699,52 @@ struct LlamaModel {
     size_t kv_elem() const { return cfg.kv_f16 ? 2 : 4; }
     size_t kv_layer_elems() const { return (size_t)n_pages * cfg.n_kv_heads * KV_PAGE * cfg.head_dim; }
 
+    // Every matrix that prompt chunks multiply with.
+    template <typename F>
+    void each_product(F&& f) const {
+        for (const Layer& L : layers)
+            for (const Mat* w : {&L.qkv, &L.qk, &L.q, &L.k, &L.v, &L.o, &L.gu, &L.gate, &L.up, &L.down})
+                if (w->n > 0) f(*w);
+    }
+    // Bytes that a product of m rows writes to gemm_scratch, on the path that
+    // linear and layer_plain give it.
+    static size_t product_scratch(const Mat& w, size_t m, bool native) {
+        if (m <= 4) return 0;  // GEMVs
+        const size_t n = w.n, k = w.k;
+        if (w.type == WType::Q4_0)
+            return gemm_scratch_bytes(m, n, k, native && !gemm_native_tile_takes(m, n, k));
+        return kgemm(w, m, native) ? gemm_tiles_scratch_bytes(m, k) : 0;
+    }
+    // The most that any chunk of up to max_batch rows writes there, in float or
+    // native mode (rdl_llama_set_native_q4).
+    size_t gemm_scratch_need() const {
+        std::vector<Mat> shapes;
+        each_product([&](const Mat& w) {
+            for (const Mat& o : shapes)
+                if (o.n == w.n && o.k == w.k && o.type == w.type) return;
+            shapes.push_back(w);
+        });
+        // Q4_0's paths for few rows and their plans change with m; past those
+        // rows the bytes of each path grow with m, whichever one m takes
+        const size_t mb = cfg.max_batch;
+        size_t need = 0;
+        for (const Mat& w : shapes) {
+            for (size_t m = 1; m <= std::min(mb, GEMM_SMALL_M); m++)
+                for (bool native : {false, true}) need = std::max(need, product_scratch(w, m, native));
+            if (w.type == WType::Q4_0 && mb > GEMM_SMALL_M)
+                for (bool native : {false, true}) need = std::max(need, gemm_scratch_bytes(mb, w.n, w.k, native));
+            else
+                need = std::max(need, product_scratch(w, mb, false));
+        }
+        return need;
+    }
+
     // y[m, mat.n] = x[m, mat.k] . W^T on the model's stream; native: the
     // Linear's use_native_q4 (Q4_0 / Q4_1 weights only, as in linear.rs:119-153)
     hipError_t linear(const Mat& w, const float* xin, size_t m, float* y, bool native = false) {
         native = native && (w.type == WType::Q4_0 || w.type == WType::Q4_1);
         if (m <= 4) return launch_gemv_fused(w.type, native, w.dev, w.n, w.k, xin, m, y, stream);
+        if (product_scratch(w, m, native) > gemm_scratch_cap) return hipErrorOutOfMemory;
         if (w.type == WType::Q4_0 && native && gemm_native_tile_takes(m, w.n, w.k))
             return launch_gemm_tile(w.type, w.dev, w.n, w.k, xin, m, y, gemm_scratch, gemm_part, gemm_cnt, 3, nullptr,
                                     0.0f, false, stream);
@@ -963,7 +1007,8 @@ struct LlamaModel {
         // nothing launched, the separate launches below run instead)
         // (native layers keep their Linears' own products: no folding)
         auto q4t = [&](const Mat& w) {
-            return !L.native && ((m > GEMM_XTILE_M && w.type == WType::Q4_0) || kgemm(w, m));
+            return !L.native && ((m > GEMM_XTILE_M && w.type == WType::Q4_0) || kgemm(w, m)) &&
+                   product_scratch(w, m, false) <= gemm_scratch_cap;
         };
         auto kfold_m = [&](const Mat& w) { return kfold(w, m); };
         const bool nat = L.native;
@@ -1229,17 +1274,9 @@ rdl_status check_fused(rdl::LlamaModel& M) {
     return api_fail(RDL_ERR_HIP, "fused decode attention: a wait for the q/k/v workgroups ran out");
 }
 
-}  // namespace
-
-extern "C" {
-
-rdl_status rdl_llama_create(const rdl_llama_config* cfg, rdl_llama** out) {
-    return rdl_llama_create_typed(cfg, nullptr, out);
-}
-
-rdl_status rdl_llama_create_typed(const rdl_llama_config* cfg, const int32_t* types, rdl_llama** out) {
-    if (!cfg || !out) return api_fail(RDL_ERR_NULL_POINTER, "NULL argument");
-    *out = nullptr;
+// Checks a configuration and gives every matrix of the model its shape and
+// GGUF type (nothing is allocated).
+rdl_status lay_out(rdl::LlamaModel& M, const rdl_llama_config* cfg, const int32_t* types) {
     if (!valid_config(*cfg))
         return api_fail(RDL_ERR_INVALID_DATA,
                         "unsupported config (dim, ffn_dim, heads*head_dim multiples of 32 and <= 16384; "
@@ -1272,66 +1309,117 @@ rdl_status rdl_llama_create_typed(const rdl_llama_config* cfg, const int32_t* ty
                 return api_fail(RDL_ERR_UNSUPPORTED, "slot %d layer %d: a K-quant matrix needs in_features %% 256 "
                                 "== 0 (%d)", slot, l, in_features(slot));
         }
-    rdl_status st = rdl::api_require_device();
-    if (st != RDL_OK) return st;
-    rdl_llama* h = new rdl_llama();
-    rdl::LlamaModel& M = h->m;
     M.cfg = *cfg;
     M.cfg.output_dtype = type_of(RDL_LLAMA_OUTPUT, 0);
-    M.out.type = (rdl::WType)M.cfg.output_dtype;
-    M.emb.type = (rdl::WType)type_of(RDL_LLAMA_TOKEN_EMBEDDING, 0);
-    M.sample_embeds = M.emb.type == rdl::WType::Q4_0;
     const rdl_llama_config& c = M.cfg;
-    M.q_dim = c.n_heads * c.head_dim;
+    M.q_dim = q_dim;
     M.kv_dim = c.n_kv_heads * c.head_dim;
     M.qkv_dim = M.q_dim + 2 * M.kv_dim;
-    auto mat = [&](rdl::LlamaModel::Mat& w, int n, int k, int32_t t = RDL_DTYPE_Q4_0) -> hipError_t {
+    auto mat = [&](rdl::LlamaModel::Mat& w, int n, int k, int32_t t) {
         w.n = n;
         w.k = k;
         w.type = (rdl::WType)t;
-        return M.alloc(reinterpret_cast<void**>(&w.dev), w.bytes() + 64);
     };
-    auto fail_free = [&](hipError_t e) {
-        delete h;
-        return api_fail(RDL_ERR_HIP, "allocation failed: %s", hipGetErrorString(e));
-    };
-    hipError_t e = hipStreamCreateWithFlags(&M.stream, hipStreamNonBlocking);
-    if (e != hipSuccess) return fail_free(e);
-    for (auto& ev : M.ev)
-        if ((e = hipEventCreate(&ev)) != hipSuccess) return fail_free(e);
-    M.layers.resize(c.n_layers);
-    bool any_split_qkv = false;
+    try {
+        M.layers.resize(c.n_layers);
+    } catch (const std::exception&) {
+        return api_fail(RDL_ERR_INVALID_DATA, "%d layers", c.n_layers);
+    }
     for (int l = 0; l < c.n_layers; l++) {
         rdl::LlamaModel::Layer& L = M.layers[l];
         const int32_t tq = type_of(RDL_LLAMA_WQ, l), tk = type_of(RDL_LLAMA_WK, l), tv = type_of(RDL_LLAMA_WV, l);
         const int32_t tg = type_of(RDL_LLAMA_W_GATE, l), tu = type_of(RDL_LLAMA_W_UP, l);
         L.split_qkv = tq != tk || tq != tv;
         L.split_gu = tg != tu;
-        any_split_qkv |= L.split_qkv;
         L.qk_joint = L.split_qkv && tq == tk;
-        if (L.qk_joint) {
-            if ((e = mat(L.qk, M.q_dim + M.kv_dim, c.dim, tq)) != hipSuccess) return fail_free(e);
-            if ((e = mat(L.v, M.kv_dim, c.dim, tv)) != hipSuccess) return fail_free(e);
-        } else if (L.split_qkv) {
-            if ((e = mat(L.q, M.q_dim, c.dim, tq)) != hipSuccess) return fail_free(e);
-            if ((e = mat(L.k, M.kv_dim, c.dim, tk)) != hipSuccess) return fail_free(e);
-            if ((e = mat(L.v, M.kv_dim, c.dim, tv)) != hipSuccess) return fail_free(e);
-        } else if ((e = mat(L.qkv, M.qkv_dim, c.dim, tq)) != hipSuccess) {
-            return fail_free(e);
+        if (!L.split_qkv) {
+            mat(L.qkv, M.qkv_dim, c.dim, tq);
+        } else {
+            if (L.qk_joint) {
+                mat(L.qk, M.q_dim + M.kv_dim, c.dim, tq);
+            } else {
+                mat(L.q, M.q_dim, c.dim, tq);
+                mat(L.k, M.kv_dim, c.dim, tk);
+            }
+            mat(L.v, M.kv_dim, c.dim, tv);
         }
-        if ((e = mat(L.o, c.dim, M.q_dim, type_of(RDL_LLAMA_WO, l))) != hipSuccess) return fail_free(e);
+        mat(L.o, c.dim, M.q_dim, type_of(RDL_LLAMA_WO, l));
         if (L.split_gu) {
-            if ((e = mat(L.gate, c.ffn_dim, c.dim, tg)) != hipSuccess) return fail_free(e);
-            if ((e = mat(L.up, c.ffn_dim, c.dim, tu)) != hipSuccess) return fail_free(e);
-        } else if ((e = mat(L.gu, 2 * c.ffn_dim, c.dim, tg)) != hipSuccess) {
-            return fail_free(e);
+            mat(L.gate, c.ffn_dim, c.dim, tg);
+            mat(L.up, c.ffn_dim, c.dim, tu);
+        } else {
+            mat(L.gu, 2 * c.ffn_dim, c.dim, tg);
         }
-        if ((e = mat(L.down, c.dim, c.ffn_dim, type_of(RDL_LLAMA_W_DOWN, l))) != hipSuccess) return fail_free(e);
+        mat(L.down, c.dim, c.ffn_dim, type_of(RDL_LLAMA_W_DOWN, l));
+    }
+    mat(M.emb, c.vocab, c.dim, type_of(RDL_LLAMA_TOKEN_EMBEDDING, 0));
+    mat(M.out, c.vocab, c.dim, M.cfg.output_dtype);
+    return RDL_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+rdl_status rdl_llama_product_scratch(int32_t dtype, size_t rows, size_t out_features, size_t in_features,
+                                     int32_t mode, size_t* bytes) {
+    if (!bytes) return api_fail(RDL_ERR_NULL_POINTER, "NULL argument");
+    if (dtype != RDL_DTYPE_Q4_0 && dtype != RDL_DTYPE_Q8_0 && dtype != RDL_DTYPE_Q4_1 && dtype != RDL_DTYPE_Q4_K &&
+        dtype != RDL_DTYPE_Q6_K)
+        return api_fail(RDL_ERR_DTYPE_MISMATCH, "unsupported dtype %d", dtype);
+    if (mode != RDL_MODE_FLOAT && mode != RDL_MODE_NATIVE)
+        return api_fail(RDL_ERR_INVALID_DATA, "unknown mode %d", mode);
+    rdl::LlamaModel::Mat w;
+    w.type = (rdl::WType)dtype;
+    if (out_features > INT32_MAX || in_features > 16384 || in_features % rdl::block_elems(w.type) != 0)
+        return api_fail(RDL_ERR_UNSUPPORTED, "%zu x %zu matrix", out_features, in_features);
+    w.n = (int)out_features;
+    w.k = (int)in_features;
+    *bytes = rdl::LlamaModel::product_scratch(w, rows, mode == RDL_MODE_NATIVE);
+    return api_ok();
+}
+
+rdl_status rdl_llama_gemm_scratch(const rdl_llama_config* cfg, const int32_t* types, size_t* bytes) {
+    if (!cfg || !bytes) return api_fail(RDL_ERR_NULL_POINTER, "NULL argument");
+    rdl::LlamaModel M;
+    const rdl_status st = lay_out(M, cfg, types);
+    if (st != RDL_OK) return st;
+    *bytes = M.gemm_scratch_need();
+    return api_ok();
+}
+
+rdl_status rdl_llama_create(const rdl_llama_config* cfg, rdl_llama** out) {
+    return rdl_llama_create_typed(cfg, nullptr, out);
+}
+
+rdl_status rdl_llama_create_typed(const rdl_llama_config* cfg, const int32_t* types, rdl_llama** out) {
+    if (!cfg || !out) return api_fail(RDL_ERR_NULL_POINTER, "NULL argument");
+    *out = nullptr;
+    std::unique_ptr<rdl_llama> own(new rdl_llama());
+    rdl::LlamaModel& M = own->m;
+    rdl_status st = lay_out(M, cfg, types);
+    if (st != RDL_OK) return st;
+    if ((st = rdl::api_require_device()) != RDL_OK) return st;
+    M.sample_embeds = M.emb.type == rdl::WType::Q4_0;
+    const rdl_llama_config& c = M.cfg;
+    auto fail_free = [&](hipError_t e) { return api_fail(RDL_ERR_HIP, "allocation failed: %s", hipGetErrorString(e)); };
+    hipError_t e = hipStreamCreateWithFlags(&M.stream, hipStreamNonBlocking);
+    if (e != hipSuccess) return fail_free(e);
+    for (auto& ev : M.ev)
+        if ((e = hipEventCreate(&ev)) != hipSuccess) return fail_free(e);
+    bool any_split_qkv = false;
+    auto alloc_mat = [&](rdl::LlamaModel::Mat& w) {
+        return w.n == 0 ? hipSuccess : M.alloc(reinterpret_cast<void**>(&w.dev), w.bytes() + 64);
+    };
+    for (rdl::LlamaModel::Layer& L : M.layers) {
+        any_split_qkv |= L.split_qkv;
+        for (rdl::LlamaModel::Mat* w : {&L.qkv, &L.qk, &L.q, &L.k, &L.v, &L.o, &L.gu, &L.gate, &L.up, &L.down})
+            if ((e = alloc_mat(*w)) != hipSuccess) return fail_free(e);
         if ((e = M.alloc_t(&L.attn_norm, c.dim)) != hipSuccess) return fail_free(e);
         if ((e = M.alloc_t(&L.ffn_norm, c.dim)) != hipSuccess) return fail_free(e);
     }
-    if ((e = mat(M.emb, c.vocab, c.dim, (int32_t)M.emb.type)) != hipSuccess) return fail_free(e);
-    if ((e = mat(M.out, c.vocab, c.dim, (int32_t)M.out.type)) != hipSuccess) return fail_free(e);
+    if ((e = alloc_mat(M.emb)) != hipSuccess) return fail_free(e);
+    if ((e = alloc_mat(M.out)) != hipSuccess) return fail_free(e);
     if ((e = M.alloc_t(&M.final_norm, c.dim)) != hipSuccess) return fail_free(e);
     M.n_pages = (c.max_seq + rdl::KV_PAGE - 1) / rdl::KV_PAGE;
     const size_t kv_bytes = (size_t)c.n_layers * M.kv_layer_elems() * M.kv_elem();
@@ -1357,25 +1445,10 @@ rdl_status rdl_llama_create_typed(const rdl_llama_config* cfg, const int32_t* ty
     if ((e = M.alloc_t(&M.step, 1)) != hipSuccess) return fail_free(e);
     M.out_cap = (size_t)c.max_seq + 1;
     if ((e = M.alloc_t(&M.out_tokens, M.out_cap)) != hipSuccess) return fail_free(e);
-    // GEMM scratch for every chunk size and matrix shape the prefill runs
-    size_t gsb = 0, nmax = 0;
-    const size_t shapes[][2] = {{(size_t)M.qkv_dim, (size_t)c.dim}, {(size_t)c.dim, (size_t)M.q_dim},
-                                {2 * (size_t)c.ffn_dim, (size_t)c.dim}, {(size_t)c.dim, (size_t)c.ffn_dim},
-                                {(size_t)M.q_dim, (size_t)c.dim}, {(size_t)c.n_kv_heads * c.head_dim, (size_t)c.dim},
-                                {(size_t)c.ffn_dim, (size_t)c.dim}};
-    size_t gcc = 1;  // GEMM counters: the most any shape needs
-    for (const auto& sh : shapes) {
-        nmax = std::max(nmax, sh[0]);
-        gcc = std::max(gcc, rdl::gemm_counter_count(sh[0], sh[1]));
-        // every skinny shape (it depends on ceil(m / 16)) and the largest
-        // chunk, in float and in native mode (rdl_llama_set_native_q4)
-        for (size_t mm : {(size_t)1, (size_t)16, (size_t)32, (size_t)48, (size_t)64, mb})
-            for (bool nat : {false, true})
-                gsb = std::max(gsb, rdl::gemm_scratch_bytes(std::min(mm, mb), sh[0], sh[1], nat));
-        // K-quant matrices on the tile GEMM (x' block sums beside the split)
-        gsb = std::max(gsb, rdl::gemm_tiles_scratch_bytes(mb, sh[1]));
-    }
-    if ((e = M.alloc(&M.gemm_scratch, gsb)) != hipSuccess) return fail_free(e);
+    M.gemm_scratch_cap = M.gemm_scratch_need();
+    size_t gcc = 1;  // GEMM counters: the most any product needs
+    M.each_product([&](const rdl::LlamaModel::Mat& w) { gcc = std::max(gcc, rdl::gemm_counter_count(w.n, w.k)); });
+    if ((e = M.alloc(&M.gemm_scratch, M.gemm_scratch_cap)) != hipSuccess) return fail_free(e);
     if ((e = M.alloc_t(&M.gemm_part, rdl::GEMM_PART_BYTES / sizeof(float))) != hipSuccess) return fail_free(e);
     if ((e = M.alloc_t(&M.gemm_cnt, gcc)) != hipSuccess) return fail_free(e);
     if ((e = hipMemset(M.gemm_cnt, 0, gcc * sizeof(int))) != hipSuccess)
@@ -1417,7 +1490,7 @@ rdl_status rdl_llama_create_typed(const rdl_llama_config* cfg, const int32_t* ty
         return fail_free(e);
     hipLaunchKernelGGL(rdl::set_int_kernel, dim3(1), dim3(64), 0, M.stream, M.pos, 0);
     if ((e = hipStreamSynchronize(M.stream)) != hipSuccess) return fail_free(e);
-    *out = h;
+    *out = own.release();
     return api_ok();
 }
 

@@ -30,6 +30,8 @@ class _Config(C.Structure):
 _decl("rdl_llama_create", _i32, C.POINTER(_Config), C.POINTER(_p))
 _decl("rdl_llama_create_typed", _i32, C.POINTER(_Config), C.POINTER(C.c_int32), C.POINTER(_p))
 _decl("rdl_llama_free", _i32, _p)
+_decl("rdl_llama_gemm_scratch", _i32, C.POINTER(_Config), C.POINTER(C.c_int32), C.POINTER(_sz))
+_decl("rdl_llama_product_scratch", _i32, _i32, _sz, _sz, _sz, _i32, C.POINTER(_sz))
 _decl("rdl_llama_set_weight", _i32, _p, _i32, _i32, _p, _sz)
 _decl("rdl_llama_init_random", _i32, _p, C.c_uint64)
 _decl("rdl_llama_reset", _i32, _p)
@@ -82,6 +84,31 @@ class LlamaConfig:
                        self.max_batch, self.output_dtype)
 
 
+def _type_array(config: LlamaConfig, types):
+    """{(slot, layer): GGML type id} as rdl_llama_create_typed takes it, or None."""
+    if not types:
+        return None
+    t = np.zeros(config.n_layers * SLOTS, dtype=np.int32)
+    for (slot, layer), v in types.items():
+        t[layer * SLOTS + slot] = v
+    return t
+
+
+def gemm_scratch_bytes(config: LlamaConfig, types=None) -> int:
+    """Bytes of GEMM work memory that a model allocates (types as LlamaModel takes them; no device needed)."""
+    n, t, cfg = _sz(), _type_array(config, types), config._c()
+    check(lib.rdl_llama_gemm_scratch(C.byref(cfg), None if t is None else t.ctypes.data_as(C.POINTER(C.c_int32)),
+                                     C.byref(n)))
+    return n.value
+
+
+def product_scratch_bytes(dtype: int, rows: int, out_features: int, in_features: int, mode: int = 0) -> int:
+    """Bytes that one product of a model writes to that memory."""
+    n = _sz()
+    check(lib.rdl_llama_product_scratch(dtype, rows, out_features, in_features, mode, C.byref(n)))
+    return n.value
+
+
 def _i32_array(tokens):
     return np.ascontiguousarray(np.asarray(tokens, dtype=np.int32).reshape(-1))
 
@@ -97,9 +124,7 @@ class LlamaModel:
         h = _p()
         cfg = config._c()
         if types:
-            t = np.zeros(config.n_layers * SLOTS, dtype=np.int32)
-            for (slot, layer), v in types.items():
-                t[layer * SLOTS + slot] = v
+            t = _type_array(config, types)
             check(lib.rdl_llama_create_typed(C.byref(cfg), t.ctypes.data_as(C.POINTER(C.c_int32)), C.byref(h)))
         else:
             check(lib.rdl_llama_create(C.byref(cfg), C.byref(h)))

@@ -402,6 +402,22 @@ def test_mixed_type_prompt_chunk_on_the_gemms(rq, gpu):
     check_typed_model(m, ref, prompt, 17, steps=2)
 
 
+@pytest.mark.parametrize("rows", [5, 32, 64])
+def test_joint_q4_0_qk_prompt_chunk(rq, gpu, rows):
+    """Q4_0 [Wq; Wk] beside a Q6_K v: the joint matrix is the product of a few
+    rows with the most K-slice partials here (2048 rows of 1024, wider than the FFN's)."""
+    import rdlquant.llama as L
+    print(f"case joint qk rows={rows}", flush=True)
+    cfg = tiny_config(dim=1024, n_layers=1, n_heads=8, n_kv_heads=8, head_dim=128, ffn_dim=2560, max_batch=64,
+                      max_seq=128)
+    types = {(L.WV, 0): 14}
+    need = L.product_scratch_bytes(2, rows, 2048, 1024)
+    assert need <= L.gemm_scratch_bytes(cfg, types)
+    m, ref, _ = build_typed(cfg, types, 515)
+    prompt = [int(v) for v in np.random.default_rng(rows).integers(0, cfg.vocab, size=rows)]
+    check_typed_model(m, ref, prompt, 17, steps=1)
+
+
 def check_typed_model(m, ref, prompt, tok, steps=4):
     """Prefill (rows four at a time through the fused GEMVs), decode steps and
     greedy generation against the oracle's forward."""
