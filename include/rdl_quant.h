@@ -237,10 +237,14 @@ rdl_status rdl_release_stream_work(void* stream);
  * array of RDL_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; its
  * last 64 KiB hold the prefill GEMM's counters (zero at load, left at zero by
  * every launch).  Products needing more than the rest return
- * RDL_ERR_UNSUPPORTED before launching anything.  Every call on one GPU
- * shares that array: calls that overlap in time on one GPU (other streams,
+ * RDL_ERR_UNSUPPORTED before launching anything (native Q4_0 ones: whose Q8_0
+ * codes and scales, 1.125 bytes an element of x, would not fit).  A second
+ * static array of 32 MiB per GPU holds the prefill GEMM's K-slice partials and,
+ * for native products whose f16 split is larger than the first, half of that
+ * split; such products run in chunks of rows.  Every call on one GPU
+ * shares these arrays: calls that overlap in time on one GPU (other streams,
  * other threads) race and must be serialized by the caller.  Results equal
- * rdl_linear_forward_dev's (same kernels). */
+ * rdl_linear_forward_dev's (same kernels, the same K slices: the same bits). */
 #define RDL_NOALLOC_SCRATCH_BYTES (16u << 20)
 rdl_status rdl_linear_forward_dev_noalloc(const rdl_weight* w, const float* x_dev, size_t m,
                                           float* y_dev, int32_t mode, void* stream);

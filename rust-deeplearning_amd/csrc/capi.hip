@@ -218,10 +218,11 @@ bool wants_counters(WType t, Path p, bool native, size_t m, size_t n, size_t k) 
 }
 
 // Run the product on `s`; `work` holds scratch_bytes(path) bytes of device
-// memory, `part` part_bytes (or is NULL: unsplit), `counters` gemm_counter_count(n, k) ints of the GEMM (zero between calls).
+// memory, `part` part_bytes (or is NULL: unsplit), `counters` gemm_counter_count(n, k) ints of the GEMM (zero between
+// calls).  NativeTile over a smaller `work`: lo and chunk as launch_gemm_tile takes them.
 rdl_status run_linear(WType t, bool native, const uint8_t* w_dev, size_t n, size_t k,
                       const float* x_dev, size_t m, float* y_dev, void* work, float* part, int* counters,
-                      hipStream_t s, Path path) {
+                      hipStream_t s, Path path, void* lo = nullptr, size_t chunk = 0) {
     if (m == 0 || n == 0) return RDL_OK;
     // k == 0: no blocks; the GEMV then writes zeros (empty dot, as in the reference).
     if (k == 0) {
@@ -234,7 +235,7 @@ rdl_status run_linear(WType t, bool native, const uint8_t* w_dev, size_t n, size
     }
     if (path == Path::NativeTile) {
         HIP_TRY(rdl::launch_gemm_tile(t, w_dev, n, k, x_dev, m, y_dev, work, part, counters, 3, nullptr, 0.0f, false,
-                                      s));
+                                      s, lo, chunk));
         return RDL_OK;
     }
     if (path == Path::Gemm) {
@@ -262,8 +263,11 @@ rdl_status run_linear(WType t, bool native, const uint8_t* w_dev, size_t n, size
 // and kept in scratch_dev[]; only that address is ever passed to kernels.
 __device__ __align__(256) uint8_t scratch[RDL_NOALLOC_SCRATCH_BYTES];
 // The tile GEMM's K-slice partials have an array of their own: a product's
-// other scratch alone decides whether it fits.
-__device__ __align__(256) float scratch_part[rdl::GEMM_PART_BYTES / sizeof(float)];
+// other scratch alone decides whether it fits.  Native products whose x split
+// is larger than `scratch` (the rest need only what their int8 codes took) put
+// x_lo behind the partials and run by row chunks.
+constexpr size_t SCRATCH_LO_BYTES = 16u << 20;
+__device__ __align__(256) float scratch_part[(rdl::GEMM_PART_BYTES + SCRATCH_LO_BYTES) / sizeof(float)];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex scratch_mu;
@@ -697,11 +701,13 @@ rdl_status rdl_linear_forward_dev_noalloc(const rdl_weight* w, const float* x_de
     if (m == 0 || w->n == 0) return ok();
     if (!x_dev || !y_dev) return fail(RDL_ERR_NULL_POINTER, "NULL activation pointer");
     const bool native = mode == RDL_MODE_NATIVE && (w->type == WType::Q4_0 || w->type == WType::Q4_1);
-    Path path = pick_path(w->type, native, m, w->n, w->k, x_dev);
-    size_t rb = scratch_bytes(w->type, path, native, m, w->n, w->k);
-    if (path == Path::NativeTile && rb > NOALLOC_DATA_BYTES) {  // int8 codes take a quarter of its x split
-        path = Path::Gemm;
-        rb = scratch_bytes(w->type, path, native, m, w->n, w->k);
+    const Path path = pick_path(w->type, native, m, w->n, w->k, x_dev);
+    size_t rb = scratch_bytes(w->type, path, native, m, w->n, w->k), chunk = 0;
+    if (path == Path::NativeTile && rb > NOALLOC_DATA_BYTES) {
+        // taken while the Q8_0 codes and scales of x would fit, as products of
+        // fewer rows are; the f16 split of as many rows as fit at a time
+        rb = rdl::gemm_scratch_bytes(m, w->n, w->k, true);
+        chunk = rdl::gemm_tile_chunk_rows(w->k, NOALLOC_DATA_BYTES, SCRATCH_LO_BYTES);
     }
     if (rb > NOALLOC_DATA_BYTES)
         return fail(RDL_ERR_UNSUPPORTED,
@@ -715,7 +721,8 @@ rdl_status rdl_linear_forward_dev_noalloc(const rdl_weight* w, const float* x_de
     int* counters = reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(work) + NOALLOC_DATA_BYTES);
     st = run_linear(w->type, native, (const uint8_t*)w->dev, w->n, w->k, x_dev, m, y_dev, work,
                     part_bytes(w->type, path, native, m, w->n, w->k) ? (float*)part : nullptr, counters,
-                    (hipStream_t)stream, path);
+                    (hipStream_t)stream, path,
+                    chunk ? reinterpret_cast<uint8_t*>(part) + rdl::GEMM_PART_BYTES : nullptr, chunk);
     return st == RDL_OK ? ok() : st;
 }
 

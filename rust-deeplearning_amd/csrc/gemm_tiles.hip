@@ -346,11 +346,14 @@ __device__ __forceinline__ void q6k_f16(uint32_t n0, uint32_t n1, uint32_t scale
     lo = half8_t{l0[0], l0[1], l1[0], l1[1], l2[0], l2[1], l3[0], l3[1]};
 }
 
+// The launch computes rows r0 .. r1 - 1 of the product's m (r0 a multiple of
+// the tile's rows): the split holds those, the tiles and their K slices are
+// the whole product's, so the results do not depend on the rows of a launch.
 template <int WF, int FI, int WJ, int KS, bool LOCAL>
 __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const uint8_t* __restrict__ W, int n, int nb, const void* __restrict__ XH, const void* __restrict__ XL,
-    const int* __restrict__ XE, int m, const uint32_t* __restrict__ XS, float* __restrict__ Y, int accy, int full, int SR, int kbs, float* __restrict__ part,
-    int* __restrict__ cnt) {
+    const int* __restrict__ XE, int m, int r0, int r1, const uint32_t* __restrict__ XS, float* __restrict__ Y,
+    int accy, int full, int SR, int kbs, float* __restrict__ part, int* __restrict__ cnt) {
     using C = TileCfg<WF, FI, WJ, KS>;
     constexpr int CB = C::CB, FJ = 4;
     constexpr bool BYTES = C::BYTES, Q4K = WF == WF_Q4_K, Q6K = WF == WF_Q6_K, CHAIN = C::CHAIN;
@@ -385,6 +388,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const int band = t / (GI * nj), rem = t % (GI * nj);
     const int bh = min(GI, ni - band * GI);
     const int j0 = (rem / bh) * C::TJ, i0 = (band * GI + rem % bh) * C::TI;
+    if (i0 < r0 || i0 >= r1) return;  // (whole workgroup)
     const int kb0 = slice * kbs, kb1 = S > 1 ? min(nb, kb0 + kbs) : nb;  // this slice's blocks (kb0 a multiple of CB)
 
     const uint32_t k = (uint32_t)nb * 32u, row_bytes = Q4K   ? (uint32_t)(nb / 8) * 144u
@@ -392,8 +396,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
                                                                    : (uint32_t)nb * BB,
                    wbytes = (uint32_t)n * row_bytes;
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(W, wbytes);
-    const __amdgpu_buffer_rsrc_t hrs = make_rsrc(XH, (uint32_t)m * k * 2u);
-    const __amdgpu_buffer_rsrc_t lrs = make_rsrc(XL, (uint32_t)m * k * 2u);
+    const __amdgpu_buffer_rsrc_t hrs = make_rsrc(XH, (uint32_t)(r1 - r0) * k * 2u);
+    const __amdgpu_buffer_rsrc_t lrs = make_rsrc(XL, (uint32_t)(r1 - r0) * k * 2u);
     const int nchunks = (kb1 - kb0 + CB - 1) / CB;
 
     struct WRegs { uint32_t w[C::WU][C::WWORDS]; };
@@ -467,13 +471,13 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         }
     };
     int* const xe = reinterpret_cast<int*>(lds + C::XE_AT);
-    if (tid < C::TI) xe[tid] = i0 + tid < m ? XE[i0 + tid] : 0;
+    if (tid < C::TI) xe[tid] = i0 + tid < r1 ? XE[i0 + tid - r0] : 0;
 
     uint32_t xbase[C::XU];
 #pragma unroll
     for (int u = 0; u < C::XU; u++) {
         const int idx = tid + u * C::NT, i = i0 + idx / (CB * 4), q = idx % (CB * 4);
-        xbase[u] = i < m ? ((uint32_t)i * k + (uint32_t)kb0 * 32u + (uint32_t)q * 8u) * 2u : RSRC_OOB;
+        xbase[u] = i < r1 ? ((uint32_t)(i - r0) * k + (uint32_t)kb0 * 32u + (uint32_t)q * 8u) * 2u : RSRC_OOB;
     }
     // part q of a chunk's x loads: unit q / 2, hi or lo
     auto load_x_part = [&](int c, XRegs& R, int q) {
@@ -482,14 +486,14 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         if (q & 1) R.l[u] = buf_load_b128(lrs, off);
         else R.h[u] = buf_load_b128(hrs, off);
     };
-    const __amdgpu_buffer_rsrc_t srs = make_rsrc(Q4K ? (const void*)XS : XH, Q4K ? (uint32_t)m * (uint32_t)nb * 4u : 0u);
+    const __amdgpu_buffer_rsrc_t srs = make_rsrc(Q4K ? (const void*)XS : XH, Q4K ? (uint32_t)(r1 - r0) * (uint32_t)nb * 4u : 0u);
     auto load_sums = [&](int c, XRegs& R) {
         if constexpr (Q4K) {
 #pragma unroll
             for (int u = 0; u < C::SU; u++) {
                 const int idx = tid + u * C::NT, i = i0 + idx / CB, b = kb0 + c * CB + idx % CB;
-                R.s[u] = buf_load_b32(srs, idx < C::TI * CB && i < m && b < kb1
-                                               ? ((uint32_t)i * (uint32_t)nb + (uint32_t)b) * 4u
+                R.s[u] = buf_load_b32(srs, idx < C::TI * CB && i < r1 && b < kb1
+                                               ? ((uint32_t)(i - r0) * (uint32_t)nb + (uint32_t)b) * 4u
                                                : RSRC_OOB);
             }
         }
@@ -865,7 +869,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int i = i0 + b * 16 + g * 4 + u;
-            if (i >= m) continue;
+            if (i >= r1) continue;
             const int e = xe[i - i0];
             f32x4 v = {ldexpf(v4[0][u], e), ldexpf(v4[1][u], e), ldexpf(v4[2][u], e), ldexpf(v4[3][u], e)};
             float* yp = Y + (size_t)i * n + j;
@@ -975,23 +979,25 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     for (int b = 0; b < FO; b++) store_rows(ks * FO + b, own[b]);
 }
 
-// x split of one product in the scratch (gemm_tiles_scratch_bytes(m, k)).
+// x split of m rows in the scratch (gemm_tiles_scratch_bytes(m, k)); lo: where
+// x_lo goes instead (m k 2 bytes), or NULL.
 struct XSplit {
     _Float16 *h, *l;
     int* e;
     uint32_t* s;  // x' sums of each block (hi / lo pairs), or NULL
 };
-XSplit x_split_at(void* scratch, size_t m, size_t k, bool sums) {
+XSplit x_split_at(void* scratch, void* lo, size_t m, size_t k, bool sums) {
     const size_t xb = (m * k * 2 + 255) & ~(size_t)255, eb = (m * 4 + 255) & ~(size_t)255;
     uint8_t* p = reinterpret_cast<uint8_t*>(scratch);
-    return {reinterpret_cast<_Float16*>(p), reinterpret_cast<_Float16*>(p + xb), reinterpret_cast<int*>(p + 2 * xb),
-            sums ? reinterpret_cast<uint32_t*>(p + 2 * xb + eb) : nullptr};
+    uint8_t* e = p + (lo ? xb : 2 * xb);
+    return {reinterpret_cast<_Float16*>(p), reinterpret_cast<_Float16*>(lo ? lo : p + xb), reinterpret_cast<int*>(e),
+            sums ? reinterpret_cast<uint32_t*>(e + eb) : nullptr};
 }
 
 // One tile shape: 64 WJ weight rows x 16 FI x rows, KS wave groups sharing
 // each chunk's blocks.
 template <int WF, int FI, int WJ, int KS>
-hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const XSplit& x, int m, float* y, int accy,
+hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const XSplit& x, int m, int r0, int r1, float* y, int accy,
                            const TilePlan& p, float* part, int* cnt, hipStream_t s) {
     using C = TileCfg<WF, FI, WJ, KS>;
     static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
@@ -1007,8 +1013,8 @@ hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const XSplit& x, int
     }
     unsigned rest = (unsigned)((n + C::TJ - 1) / C::TJ) * (unsigned)((m + C::TI - 1) / C::TI) - (unsigned)p.full;
     if (local) rest = (rest + 7) / 8 * 8;
-    launch_kernel(kern, dim3((unsigned)p.full + rest * (unsigned)p.S), dim3(C::NT), (size_t)C::LDS, s, w, n, nb, x.h, x.l, x.e, m, x.s, y,
-                  accy, p.full, p.S, p.kbs, part, cnt);
+    launch_kernel(kern, dim3((unsigned)p.full + rest * (unsigned)p.S), dim3(C::NT), (size_t)C::LDS, s, w, n, nb, x.h,
+                  x.l, x.e, m, r0, r1, x.s, y, accy, p.full, p.S, p.kbs, part, cnt);
     return hipGetLastError();
 }
 
@@ -1146,37 +1152,61 @@ size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k) {
 }
 
 template <int WF>
-static hipError_t launch_tile_wf(WType t, const uint8_t* w, int n, int nb, const XSplit& x, int m, float* y, int accy,
-                                 float* part, int* cnt, hipStream_t s) {
-    const TilePlan p = tile_plan(t, m, n, nb, part != nullptr && cnt != nullptr);
-    if constexpr (WF == WF_Q4_0 || WF == WF_Q8_0)
-        if (p.cfg == 0) return launch_tile_cfg<WF, 8, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
-    if constexpr (WF == WF_Q4_0 || WF == WF_Q8_0)
-        if (p.cfg == 1) return launch_tile_cfg<WF, 4, 4, 2>(w, n, nb, x, m, y, accy, p, part, cnt, s);
-    if constexpr (WF == WF_Q4_0 || WF == WF_Q8_0)
-        if (p.cfg == 3) return launch_tile_cfg<WF, 4, 1, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
-    return launch_tile_cfg<WF, 4, 2, 4>(w, n, nb, x, m, y, accy, p, part, cnt, s);
+static hipError_t launch_tile_wf(const uint8_t* w, int n, int nb, const XSplit& x, int m, int r0, int r1, float* y,
+                                 int accy, const TilePlan& p, float* part, int* cnt, hipStream_t s) {
+    auto go = [&](auto fi, auto wj, auto ks) {
+        return launch_tile_cfg<WF, decltype(fi)::value, decltype(wj)::value, decltype(ks)::value>(
+            w, n, nb, x, m, r0, r1, y, accy, p, part, cnt, s);
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I4 = std::integral_constant<int, 4>;
+    using I8 = std::integral_constant<int, 8>;
+    if constexpr (WF == WF_Q4_0 || WF == WF_Q8_0) {
+        if (p.cfg == 0) return go(I8{}, I4{}, I2{});
+        if (p.cfg == 1) return go(I4{}, I4{}, I2{});
+        if (p.cfg == 3) return go(I4{}, I1{}, I4{});
+    }
+    return go(I4{}, I2{}, I4{});
 }
 
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
-                            hipStream_t s) {
+                            hipStream_t s, void* lo, size_t chunk) {
     if (pro == 3 ? t != WType::Q4_0 || k == 0 || !gemm_native_tile_takes(m, n, k)
                  : k == 0 || !gemm_tile_takes(t, m, n, k) || (pro != 0 && k > GEMM_SPLIT_MAX_K))
         return hipErrorInvalidValue;
-    const XSplit xo = x_split_at(scratch, m, k, t == WType::Q4_K);
-    const hipError_t e = pro == 1   ? launch_split<1>(x, m, k, g, eps, xo, s)
-                         : pro == 2 ? launch_split<2>(x, m, k, g, eps, xo, s)
-                         : pro == 3 ? launch_split<3>(x, m, k, g, eps, xo, s)
-                                    : launch_split<0>(x, m, k, g, eps, xo, s);
-    if (e != hipSuccess) return e;
+    if (chunk == 0) chunk = m;
+    if (chunk < m && chunk % TILE_SHAPES[0].ti != 0) return hipErrorInvalidValue;
+    const TilePlan p = tile_plan(t, m, n, k / QK, part != nullptr && cnt != nullptr);
     const int ni = (int)n, nb = (int)(k / QK), mi = (int)m, acc = accumulate ? 1 : 0;
-    switch (t) {
-        case WType::Q4_0: return launch_tile_wf<WF_Q4_0>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
-        case WType::Q8_0: return launch_tile_wf<WF_Q8_0>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
-        case WType::Q4_K: return launch_tile_wf<WF_Q4_K>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
-        default: return launch_tile_wf<WF_Q6_K>(t, w, ni, nb, xo, mi, y, acc, part, cnt, s);
+    for (size_t r0 = 0; r0 < m; r0 += chunk) {
+        const size_t rows = std::min(chunk, m - r0);
+        const int a = (int)r0, b = (int)(r0 + rows);
+        const XSplit xo = x_split_at(scratch, lo, rows, k, t == WType::Q4_K);
+        const float* xr = x + r0 * k * (pro == 2 ? 2 : 1);
+        hipError_t e = pro == 1   ? launch_split<1>(xr, rows, k, g, eps, xo, s)
+                       : pro == 2 ? launch_split<2>(xr, rows, k, g, eps, xo, s)
+                       : pro == 3 ? launch_split<3>(xr, rows, k, g, eps, xo, s)
+                                  : launch_split<0>(xr, rows, k, g, eps, xo, s);
+        if (e != hipSuccess) return e;
+        switch (t) {
+            case WType::Q4_0: e = launch_tile_wf<WF_Q4_0>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s); break;
+            case WType::Q8_0: e = launch_tile_wf<WF_Q8_0>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s); break;
+            case WType::Q4_K: e = launch_tile_wf<WF_Q4_K>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s); break;
+            default: e = launch_tile_wf<WF_Q6_K>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s);
+        }
+        if (e != hipSuccess) return e;
     }
+    return hipSuccess;
+}
+
+size_t gemm_tile_chunk_rows(size_t k, size_t bytes, size_t lo_bytes) {
+    const size_t ti = TILE_SHAPES[0].ti;  // (the other shapes' rows divide it)
+    size_t rows = std::min(lo_bytes / (k * 2), bytes / (k * 2 + 4)) / ti * ti;
+    // x_hi, the exponents, each rounded up to 256 bytes
+    while (rows > 0 && ((rows * k * 2 + 255) & ~(size_t)255) + ((rows * 4 + 255) & ~(size_t)255) > bytes) rows -= ti;
+    return rows;
 }
 
 }  // namespace rdl

@@ -212,7 +212,12 @@ bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k);
 bool gemm_native_tile_takes(size_t m, size_t n, size_t k);
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
-                            hipStream_t s);
+                            hipStream_t s, void* lo = nullptr, size_t chunk = 0);
+// A scratch that does not hold the split of all m rows: x_lo in an array of its
+// own (lo) and the rows `chunk` at a time (a multiple of every tile's rows), by
+// the whole product's plan, so the results are the same bits.  The most rows
+// that `bytes` of scratch and lo_bytes of lo take.
+size_t gemm_tile_chunk_rows(size_t k, size_t bytes, size_t lo_bytes);
 hipError_t launch_gemm_q4_0_native(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                                    int32_t* partials, void* scratch, hipStream_t s);
 // Float-mode products on the LDS tile GEMM, Q4_0 (more than GEMM_XTILE_M

@@ -21,6 +21,12 @@ pytestmark = pytest.mark.gpu
     (8, 0, 512, 1024, (33, 7)),      # Q8_0 float: tile GEMM (33 rows), then records (7 rows)
     (12, 0, 1024, 4096, (40, 16)),   # Q4_K float: tile GEMM, x split and x' block sums in scratch
     (14, 0, 1000, 2048, (20, 17)),   # Q6_K float: tile GEMM, x split in scratch
+    (2, 1, 4096, 4096, (128, 65)),   # Q4_0 native on the tiles: the f16 split of the Q8_0 values in scratch
+    (2, 1, 1000, 14336, (600, 520)),  # ... in row chunks of 512, K split
+    (2, 1, 9000, 16384, (450, 300)),  # ... chunks of 384, unsplit tiles and a split last round
+    (2, 1, 64, 8160, (1500, 1030)),   # ... chunks of 896, odd block count
+    (8, 0, 1000, 4096, (100, 70)),    # Q8_0 float, K-slice partials
+    (12, 0, 1000, 4096, (100, 70)),   # Q4_K float, K-slice partials
 ])
 def test_noalloc_matches_allocating_entry_point(rq, gpu, dtype, mode, n, k, rows):
     import torch
