@@ -200,7 +200,7 @@ size_t scratch_bytes(WType t, Path p, bool native, size_t m, size_t n, size_t k)
         case Path::Fused: return 0;
         case Path::Gemm:
             return t == WType::Q4_0 ? rdl::gemm_scratch_bytes(m, n, k, native) : rdl::gemm_tiles_scratch_bytes(m, k);
-        case Path::NativeTile: return rdl::gemm_scratch_bytes(m, n, k, false);
+        case Path::NativeTile: return rdl::gemm_wide_scratch_bytes(m, k);
         case Path::Records: return rec_bytes(native, m, k);
     }
     return 0;

@@ -1756,6 +1756,7 @@ size_t gemm_scratch_bytes(size_t m, size_t n, size_t k, bool native) {
         const SkPlan p = skinny_plan(m, n, (int)(k / QK), true);
         return p.S > 1 ? ((size_t)p.strips * p.S * p.units * 16 + 255) & ~(size_t)255 : 0;
     }
+    if (!native && m <= GEMM_XTILE_M) return gemm_wide_scratch_bytes(m, k);  // (those on the tiles)
     if (native)  // int8 codes and f32 block scales, 256-byte aligned pieces
         return ((m * k + 255) & ~(size_t)255) + ((m * (k / QK) * 4 + 255) & ~(size_t)255);
     // x_hi, x_lo (f16) and the row exponents

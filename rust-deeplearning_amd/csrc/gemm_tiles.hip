@@ -2,11 +2,12 @@
 // Y[m, n] = X[m, k] . W[n, k]^T for many activation rows, weights read in
 // their GGUF block layout (matmul_f32_q4, quantize.rs:265-320).
 //
-// Numerics.  Each x row is scaled by a power of two (row max into [2^14,
-// 2^15)) and split into x_hi = f16(x') and x_lo = f16(x' - x_hi), about 22
-// significant bits; the weight operand is the exact integer code in f16, one
-// 16x16x32 MFMA K step is one 32-element block, and the block scale d
-// multiplies the block's f32 dot afterwards: acc += d (x_hi.q + x_lo.q).
+// Numerics.  Each x row (of a row of wide range each block, see WIDE_ROW) is
+// scaled by a power of two (its largest into [2^14, 2^15)) and split into x_hi =
+// f16(x') and x_lo = f16(x' - x_hi), about 22 significant bits; the weight
+// operand is the exact integer code in f16, one 16x16x32 MFMA K step is one
+// 32-element block, and the block scale d multiplies the block's f32 dot
+// afterwards: acc += d (x_hi.q + x_lo.q).
 //
 // Operands.  x is the A operand and W the B operand of
 // v_mfma_f32_16x16x32_f16: lane l = 16 g + r holds x row r and weight column
@@ -33,6 +34,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "rdl_device.hpp"
@@ -60,18 +62,34 @@ __device__ __forceinline__ uint32_t finite_bits(float x) {
     return b < 0x7F800000u ? b : 0u;
 }
 // The row exponent e (amax 2^-e in [2^14, 2^15); 0 for a row of zeros) from
-// each thread's maximum of its finite |x| bits.
+// each thread's maximum of its finite |x| bits; lo (if not NULL): each thread's
+// smallest nonzero block maximum in, the row's out (~0: none).
 template <int NT>
-__device__ __forceinline__ int split_exponent(uint32_t am, uint32_t* red) {
+__device__ __forceinline__ int split_exponent(uint32_t am, uint32_t* red, uint32_t* lo = nullptr) {
     am = max8_u32(am);
     am = max(am, (uint32_t)dpp_i32<DPP_ROW_MIRROR>((int)am));
     am = max(am, (uint32_t)__shfl_xor((int)am, 16));
     am = max(am, (uint32_t)__shfl_xor((int)am, 32));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = am;
+    uint32_t mn = ~0u;
+    if (lo) {
+        mn = min(*lo, (uint32_t)dpp_i32<DPP_ROW_MIRROR>((int)*lo));  // (alike in a block's eight threads)
+        mn = min(mn, (uint32_t)__shfl_xor((int)mn, 16));
+        mn = min(mn, (uint32_t)__shfl_xor((int)mn, 32));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6] = am;
+        if (lo) red[NT / 64 + (threadIdx.x >> 6)] = mn;
+    }
     __syncthreads();
     am = red[0];
 #pragma unroll
     for (int w = 1; w < NT / 64; w++) am = max(am, red[w]);
+    if (lo) {
+        mn = red[NT / 64];
+#pragma unroll
+        for (int w = 1; w < NT / 64; w++) mn = min(mn, red[NT / 64 + w]);
+        *lo = mn;
+    }
     return am != 0 ? ilogbf(__builtin_bit_cast(float, am)) - 14 : 0;
 }
 
@@ -108,16 +126,28 @@ __device__ __forceinline__ void split_piece(const f32x4& v, int e, int p, int k4
     }
 }
 
+// Q4_0 rows of wide range.  x_lo's last place is 2^-24 of x', so a row with a
+// block more than 2^-WB below its largest would lose bits of that block, which
+// counts for all of a result where the larger blocks meet zero weights.  Where
+// x is held with a scale a block otherwise (the x-tile kernel's rows, WB = 14: such
+// a block keeps its 22 bits; Q8_0 values, WB = 20: they stay exact), such a row has a
+// scale 2^e for every block instead: XE = WIDE_ROW and XB[block][row] = 2^e.  A
+// byte a row says which are (XF, zeros up to a multiple of XF_PAD rows).
+constexpr int XF_PAD = 128;
+constexpr int WIDE_ROW = INT_MIN;
+constexpr int WIDE_FLOAT = 14, WIDE_NATIVE = 20;
+
 // One workgroup a row: thread t holds elements 4 (t + j NT) .. +3 (k <= 4 NV
 // NT), so x is read once.  PRO 1: RMSNorm first; PRO 2: SwiGLU of rows of 2k
 // interleaved (gate_j, up_j) values; PRO 3: x as its Q8_0 blocks hold it
 // (quantize_row_q8_0, quantize.rs:164-193).
-template <int PRO, int NT, int NV>
+template <int PRO, int NT, int NV, int WB>
 __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict__ X, int k,
                                                         const float* __restrict__ g, float eps,
                                                         _Float16* __restrict__ XH, _Float16* __restrict__ XL,
-                                                        int* __restrict__ XE, uint32_t* __restrict__ XS) {
-    __shared__ uint32_t red[NT / 64];
+                                                        int* __restrict__ XE, uint32_t* __restrict__ XS,
+                                                        float* __restrict__ XB, int xb_rows, uint8_t* __restrict__ XF) {
+    __shared__ uint32_t red[(WB ? 2 : 1) * NT / 64];
     __shared__ float red2[NT / 64];
     const int row = blockIdx.x;
     const int k4 = k >> 2;  // k % 32 == 0
@@ -147,9 +177,9 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
         }
     }
     if constexpr (PRO == 3) {
-        // code times scale, 7 + 11 bits: exact in f32, and in the hi / lo pair of a
-        // block within 2^-21 of the row's largest; a NaN scores as 0 in the block
-        // maximum and as code 0, an overflowing scale makes the block NaN
+        // code times scale, 7 + 11 bits: exact in f32 and, by the row's or the block's
+        // exponent, in the hi / lo pair; a NaN scores as 0 in the block maximum and
+        // as code 0, an overflowing scale makes the block NaN
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             float am = 0.0f;
@@ -188,17 +218,38 @@ __global__ __launch_bounds__(NT) void gemm_split_kernel(const float* __restrict_
         }
     }
     // largest finite |x| of the row as an integer maximum of |x| bits
-    uint32_t am = 0;
+    uint32_t am = 0, bm[WB ? NV : 1];
 #pragma unroll
-    for (int j = 0; j < NV; j++)
+    for (int j = 0; j < NV; j++) {
+        uint32_t a = 0;
 #pragma unroll
-        for (int t = 0; t < 4; t++) am = max(am, finite_bits(v[j][t]));
-    const int e = split_exponent<NT>(am, red);
-    if (threadIdx.x == 0) XE[row] = e;
+        for (int t = 0; t < 4; t++) a = max(a, finite_bits(v[j][t]));
+        if (WB) bm[j] = a = max8_u32(a);  // the block's
+        am = max(am, a);
+    }
+    uint32_t lo = ~0u;
+    if constexpr (WB != 0)
 #pragma unroll
-    for (int j = 0; j < NV; j++)
-        split_piece(v[j], e, threadIdx.x + j * NT, k4, XH + (size_t)row * k, XL + (size_t)row * k,
+        for (int j = 0; j < NV; j++) lo = min(lo, bm[j] - 1u);  // (a block of zeros: ~0)
+    const int e = split_exponent<NT>(am, red, WB ? &lo : nullptr);
+    const bool wide = WB && lo != ~0u && ilogbf(__builtin_bit_cast(float, lo + 1u)) < e + 14 - WB;
+    if (threadIdx.x == 0) XE[row] = wide ? WIDE_ROW : e;
+    if constexpr (WB != 0) {
+        if (threadIdx.x == 0) XF[row] = wide;
+        const int pad = row + 1 + (int)threadIdx.x;
+        if (row + 1 == (int)gridDim.x && pad < ((int)gridDim.x + XF_PAD - 1) / XF_PAD * XF_PAD) XF[pad] = 0;
+    }
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int p = threadIdx.x + j * NT;
+        int eb = e;
+        if (WB && wide) {
+            eb = bm[j] != 0 ? ilogbf(__builtin_bit_cast(float, bm[j])) - 14 : 0;
+            if ((p & 7) == 0 && p < k4) XB[(size_t)(p >> 3) * xb_rows + row] = ldexpf(1.0f, eb);
+        }
+        split_piece(v[j], eb, p, k4, XH + (size_t)row * k, XL + (size_t)row * k,
                     XS ? XS + (size_t)row * (k >> 5) : nullptr);
+    }
 }
 
 // The split of rows longer than a workgroup's registers hold: two reads of x.
@@ -244,7 +295,7 @@ constexpr int CPOL_NT = 2, CPOL_SC1 = 16;
 //    product, below x's own split).
 constexpr int WF_Q4_0 = 0, WF_Q8_0 = 1, WF_Q4_K = 2, WF_Q6_K = 3;
 
-template <int WF, int FI, int WJ, int KS>
+template <int WF, int FI, int WJ, int KS, bool WIDE>
 struct TileCfg {
     static constexpr int FJ = 4;                 // weight rows of a wave: 64, four a lane
     static constexpr int NW = WJ * KS, NT = NW * 64;
@@ -262,7 +313,10 @@ struct TileCfg {
     static constexpr int D_BYTES = CB * TJ * (WF == WF_Q6_K ? 4 : 2);
     static constexpr int X_PART = 1024;          // one 16-row tile of one block, hi or lo
     static constexpr int X_BYTES = CB * (TI / 16) * 2 * X_PART;
-    static constexpr int STAGE = W_BYTES + D_BYTES + X_BYTES;
+    // WIDE: the scale of each (block, x row), and as much where threads without one store
+    static constexpr int F_AT = W_BYTES + D_BYTES + X_BYTES, F_BYTES = WIDE ? NT * 4 : 0;
+    static_assert(!WIDE || TI * CB <= NT, "a scale a thread");
+    static constexpr int STAGE = F_AT + F_BYTES;
     static constexpr int WWORDS = WF == WF_Q6_K ? 11 : WF == WF_Q4_K ? 8 : BYTES ? 9 : 5;  // dwords a unit's loads bring
     static constexpr int WU = (TJ * CB + NT - 1) / NT;      // weight blocks a thread stages
     static constexpr int XU = (TI * CB * 4 + NT - 1) / NT;  // 16-byte pieces a thread stages, hi and lo each
@@ -349,12 +403,19 @@ __device__ __forceinline__ void q6k_f16(uint32_t n0, uint32_t n1, uint32_t scale
 // The launch computes rows r0 .. r1 - 1 of the product's m (r0 a multiple of
 // the tile's rows): the split holds those, the tiles and their K slices are
 // the whole product's, so the results do not depend on the rows of a launch.
-template <int WF, int FI, int WJ, int KS, bool LOCAL>
+// WIDE: x may have rows of wide range (WIDE_ROW).  A tile with one takes the
+// loop with a scale a block and row, one multiplication a result more; the
+// others take the plain loop (a byte a row tells, read through scalar registers:
+// no barrier; 0.3 to 0.6 us a call).  us without such rows, with them, and on the
+// x-tile or int8 kernel, which always scale so: 64 x 14336 x 4096 32 / 37 / 58, 16 x
+// 32000 x 4096 43 / 52 / 57, native 512 x 14336 x 4096 135 / 199 / 190.
+template <int WF, int FI, int WJ, int KS, bool LOCAL, bool WIDE>
 __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const uint8_t* __restrict__ W, int n, int nb, const void* __restrict__ XH, const void* __restrict__ XL,
-    const int* __restrict__ XE, int m, int r0, int r1, const uint32_t* __restrict__ XS, float* __restrict__ Y,
-    int accy, int full, int SR, int kbs, float* __restrict__ part, int* __restrict__ cnt) {
-    using C = TileCfg<WF, FI, WJ, KS>;
+    const int* __restrict__ XE, int m, int r0, int r1, const uint32_t* __restrict__ XS, const float* __restrict__ XB,
+    int xb_rows, const uint32_t* __restrict__ XF, float* __restrict__ Y, int accy, int full, int SR, int kbs,
+    float* __restrict__ part, int* __restrict__ cnt) {
+    using C = TileCfg<WF, FI, WJ, KS, WIDE>;
     constexpr int CB = C::CB, FJ = 4;
     constexpr bool BYTES = C::BYTES, Q4K = WF == WF_Q4_K, Q6K = WF == WF_Q6_K, CHAIN = C::CHAIN;
     constexpr uint32_t BB = BYTES ? 34u : 18u;  // bytes a block (not CHAIN)
@@ -400,10 +461,19 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const __amdgpu_buffer_rsrc_t lrs = make_rsrc(XL, (uint32_t)(r1 - r0) * k * 2u);
     const int nchunks = (kb1 - kb0 + CB - 1) / CB;
 
+    bool wide = false;
+    if constexpr (WIDE) {
+        uint32_t any = 0;
+#pragma unroll
+        for (int q = 0; q < C::TI / 4; q++) any |= XF[(i0 - r0) / 4 + q];
+        wide = __builtin_amdgcn_readfirstlane(any) != 0;
+    }
+
     struct WRegs { uint32_t w[C::WU][C::WWORDS]; };
     struct XRegs {
         u32x4 h[C::XU], l[C::XU];
         uint32_t s[Q4K ? C::SU : 1];
+        uint32_t f;
     };
     // unit u of a thread: block b0 + c CB of row j; CB is even, so a Q4_0 or Q8_0
     // block's place within its dword (2 bytes past it when j nb + b is odd) is
@@ -498,10 +568,18 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
             }
         }
     };
-    auto load_x = [&](int c, XRegs& R) {
+    // WIDE: thread t's scale is that of block t / TI of a chunk and row t % TI
+    const __amdgpu_buffer_rsrc_t brs =
+        make_rsrc(WIDE ? (const void*)XB : XH, WIDE ? (uint32_t)xb_rows * (uint32_t)nb * 4u : 0u);
+    uint32_t fbase = RSRC_OOB;  // (a row without scales, and until the loop that uses them)
+    auto load_scale = [&](int c, XRegs& R) {  // (past the last block: out of range)
+        R.f = buf_load_b32(brs, fbase + (uint32_t)c * (uint32_t)(CB * 4) * (uint32_t)xb_rows);
+    };
+    auto load_x = [&](int c, XRegs& R, auto w_tag) {
 #pragma unroll
         for (int q = 0; q < 2 * C::XU; q++) load_x_part(c, R, q);
         load_sums(c, R);
+        if constexpr (decltype(w_tag)::value) load_scale(c, R);
     };
     // aux: the super-block's own data (CHAIN)
     auto store_w = [&](int c, uint8_t* st, uint8_t* aux, const WRegs& R) {
@@ -575,7 +653,9 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // x piece (row il, block bl, group gq) at slot 16 gq + (row ^ (4 (bl % 2) + gq)) of its tile's
     // part: eight consecutive threads (one row's pieces) and eight consecutive
     // lanes of a fragment read (one group's rows) each touch all LDS banks once
-    auto store_x = [&](int c, uint8_t* st, uint8_t* aux, const XRegs& R) {
+    auto store_x = [&](int c, uint8_t* st, uint8_t* aux, const XRegs& R, auto w_tag) {
+        if constexpr (decltype(w_tag)::value)
+            reinterpret_cast<float*>(st + C::F_AT)[tid] = fbase != RSRC_OOB ? __builtin_bit_cast(float, R.f) : 1.0f;
         uint8_t* xs = st + C::W_BYTES + C::D_BYTES;
 #pragma unroll
         for (int u = 0; u < C::XU; u++) {
@@ -618,6 +698,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     uint32_t dd[Q6K ? 4 : 2];
     half8_t wq[ONE ? 1 : 2][4], wl[Q6K ? 4 : 1];
     float dv[2][4];
+    f32x4 fv[2];  // WIDE: the scales of a step's rows
     half8_t xh[2], xl[2];
     f32x4 p[CHAIN ? 1 : 2][FJ], T[CHAIN ? FI : 1][FJ];
     // Q4_K: even sub-blocks are low nibbles, odd ones high; this wave's are all alike
@@ -669,11 +750,12 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         // into every scale FMA (v_fma_mix_f32: 1,240 against 546 us, 2048 x 14336 x 4096)
         asm volatile("" : "+v"(dv[o][a]));
     };
-    auto add = [&](int b, int o, int ps) {
+    auto add = [&](int b, int o, int ps, auto w_tag) {
 #pragma unroll
         for (int a = 0; a < FJ; a++)
 #pragma unroll
-            for (int u = 0; u < 4; u++) acc[b][a][u] = fmaf(dv[o][a], p[ps][a][u], acc[b][a][u]);
+            for (int u = 0; u < 4; u++)
+                acc[b][a][u] = fmaf(decltype(w_tag)::value ? dv[o][a] * fv[ps][u] : dv[o][a], p[ps][a][u], acc[b][a][u]);
     };
     // CHAIN: a finished super-block (its own data at aux) goes into the sums in
     // the FI steps of the next chunk: step b adds x tile b, and Q4_K's remainder
@@ -730,7 +812,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // super-block being multiplied, the next one, the previous one
     uint8_t *ac = lds + C::AUX_AT, *an = ac + C::AUX, *ap = an + C::AUX;
     // chunk c = U modulo UN (register sets by parity)
-    auto chunk = [&](int c, auto u_tag) {
+    auto chunk = [&](int c, auto u_tag, auto w_tag) {
         constexpr int U = decltype(u_tag)::value, H = U & 1, WS = (U + 1) % DW, XS1 = (U + 1) % DX;
         uint8_t* const as = CHAIN && U == UN - 1 ? an : ac;  // chunk c + 1's super-block
 #pragma unroll
@@ -769,7 +851,9 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
                     p[s & 1][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[s & 1], wq[H][a], z, 0, 0, 0);
                     p[s & 1][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[s & 1], wq[H][a], p[s & 1][a], 0, 0, 0);
                 }
-                add(s == 0 ? FI - 1 : s - 1, s == 0 ? H ^ 1 : H, (s & 1) ^ 1);
+                add(s == 0 ? FI - 1 : s - 1, s == 0 ? H ^ 1 : H, (s & 1) ^ 1, w_tag);
+                if constexpr (decltype(w_tag)::value)
+                    fv[s & 1] = *reinterpret_cast<const f32x4*>(bc + C::F_AT + (ks * C::TI + s * 16 + g * 4) * 4);
             }
             if (s > RB && !ONE) {
 #pragma unroll
@@ -780,7 +864,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
                 store_w(c + 1, bn, as, w[WS]);
                 if (DW == 1) load_w(c + 2, w[0]);
             }
-            if (s == 1) store_x(c + 1, bn, as, x1[XS1]);
+            if (s == 1) store_x(c + 1, bn, as, x1[XS1], w_tag);
             // the loads into the freed registers, spread over the later steps (a
             // burst of them stalls the waves at issue)
             if (DW == 2 && s == FI - 1) load_w(c + 3, w[WS]);
@@ -789,6 +873,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
                 for (int q = 0; q < 2 * C::XU; q++)
                     if (2 + q * (FI - 2) / (2 * C::XU) == s) load_x_part(c + 1 + DX, x1[XS1], q);
                 if (s == FI - 1) load_sums(c + 1 + DX, x1[XS1]);
+                if constexpr (decltype(w_tag)::value)
+                    if (s == FI - 1) load_scale(c + 1 + DX, x1[XS1]);
             }
             if constexpr (!Q6K) {
 #pragma unroll
@@ -817,50 +903,98 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
             an = t4;
         }
     };
-    // chunks 0 .. DW - 1 of W and 0 .. DX - 1 of x first, then on to DW / DX
-    // once chunk 0 is stored
+    constexpr std::false_type plain{};
+    if constexpr (!WIDE) {
+        // chunks 0 .. DW - 1 of W and 0 .. DX - 1 of x first, then on to DW / DX
+        // once chunk 0 is stored
 #pragma unroll
-    for (int q = 0; q < DW; q++) load_w(q, w[q]);
+        for (int q = 0; q < DW; q++) load_w(q, w[q]);
 #pragma unroll
-    for (int q = 0; q < DX; q++) load_x(q, x1[q]);
-    if constexpr (CHAIN)  // nothing to flush before the first super-block: zeros
-        for (int q = tid; q < C::AUX / 4; q += C::NT) reinterpret_cast<uint32_t*>(ap)[q] = 0;
-    store_w(0, bc, ac, w[0]);
-    store_x(0, bc, ac, x1[0]);
-    load_w(DW, w[0]);
-    load_x(DX, x1[0]);
-    __syncthreads();
-    read_w(bc);
-    read_x(bc, 0);
-    if constexpr (CHAIN) flush_begin(ap);
+        for (int q = 0; q < DX; q++) load_x(q, x1[q], plain);
+        if constexpr (CHAIN)  // nothing to flush before the first super-block: zeros
+            for (int q = tid; q < C::AUX / 4; q += C::NT) reinterpret_cast<uint32_t*>(ap)[q] = 0;
+        store_w(0, bc, ac, w[0]);
+        store_x(0, bc, ac, x1[0], plain);
+        load_w(DW, w[0]);
+        load_x(DX, x1[0], plain);
+        __syncthreads();
+        read_w(bc);
+        read_x(bc, 0);
+        if constexpr (CHAIN) flush_begin(ap);
 #pragma unroll
-    for (int a = 0; a < FJ; a++) {
-        conv(0, a);
-        if constexpr (!CHAIN) {
-            dv[1][a] = 0.0f;
-            p[1][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int a = 0; a < FJ; a++) {
+            conv(0, a);
+            if constexpr (!CHAIN) {
+                dv[1][a] = 0.0f;
+                p[1][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            } else {
+#pragma unroll
+                for (int b = 0; b < FI; b++) T[b][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (Q4K)
+#pragma unroll
+                    for (int b = 0; b < FO; b++) um[b][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+        // (chunks past the slice's end: zeros; no branch, so that the waits stay exact)
+        for (int c = 0; c < nchunks; c += UN) {
+            chunk(c, std::integral_constant<int, 0>{}, plain);
+            chunk(c + 1, std::integral_constant<int, 1>{}, plain);
+            if constexpr (UN == 4) {
+                chunk(c + 2, std::integral_constant<int, 2>{}, plain);
+                chunk(c + 3, std::integral_constant<int, 3>{}, plain);
+            }
+        }
+        if constexpr (CHAIN) {
+#pragma unroll
+            for (int b = 0; b < FI; b++) flush(b, ap);  // (begun at the end of the last chunk)
         } else {
-#pragma unroll
-            for (int b = 0; b < FI; b++) T[b][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if constexpr (Q4K)
-#pragma unroll
-                for (int b = 0; b < FO; b++) um[b][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            add(FI - 1, 1, 1, plain);
         }
-    }
-    // (chunks past the slice's end: zeros; no branch, so that the waits stay exact)
-    for (int c = 0; c < nchunks; c += UN) {
-        chunk(c, std::integral_constant<int, 0>{});
-        chunk(c + 1, std::integral_constant<int, 1>{});
-        if constexpr (UN == 4) {
-            chunk(c + 2, std::integral_constant<int, 2>{});
-            chunk(c + 3, std::integral_constant<int, 3>{});
-        }
-    }
-    if constexpr (CHAIN) {
-#pragma unroll
-        for (int b = 0; b < FI; b++) flush(b, ap);  // (begun at the end of the last chunk)
     } else {
-        add(FI - 1, 1, 1);
+        // The same steps.  The loads before the loop stay in the loop's order, for
+        // its first wait covers both (reordered it waits for all loads but two: 64 x
+        // 14336 x 4096 27.6 -> 29.4 us).
+        auto multiply = [&](auto w_tag) {
+#pragma unroll
+            for (int q = 0; q < DW; q++) {
+                load_w(q, w[q]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int q = 0; q < DX; q++) {
+                load_x(q, x1[q], w_tag);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            store_w(0, bc, ac, w[0]);
+            store_x(0, bc, ac, x1[0], w_tag);
+            load_w(DW, w[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            load_x(DX, x1[0], w_tag);
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            read_w(bc);
+            read_x(bc, 0);
+            fv[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int a = 0; a < FJ; a++) {
+                conv(0, a);
+                dv[1][a] = 0.0f;
+                p[1][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            for (int c = 0; c < nchunks; c += UN) {
+                chunk(c, std::integral_constant<int, 0>{}, w_tag);
+                chunk(c + 1, std::integral_constant<int, 1>{}, w_tag);
+            }
+            add(FI - 1, 1, 1, w_tag);
+        };
+        if (wide) {
+            __syncthreads();  // (the rows' exponents are in LDS)
+            if (tid < C::TI * CB && xe[tid % C::TI] == WIDE_ROW)
+                fbase = ((uint32_t)(kb0 + tid / C::TI) * (uint32_t)xb_rows + (uint32_t)(i0 - r0 + tid % C::TI)) * 4u;
+            multiply(std::true_type{});
+        } else {
+            multiply(plain);
+        }
     }
 
     // lane (g, r) holds y[i = 4 g + u][j = 4 r .. 4 r + 3] of 16-row tile b
@@ -870,7 +1004,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         for (int u = 0; u < 4; u++) {
             const int i = i0 + b * 16 + g * 4 + u;
             if (i >= r1) continue;
-            const int e = xe[i - i0];
+            const int e = WIDE && xe[i - i0] == WIDE_ROW ? 0 : xe[i - i0];
             f32x4 v = {ldexpf(v4[0][u], e), ldexpf(v4[1][u], e), ldexpf(v4[2][u], e), ldexpf(v4[3][u], e)};
             float* yp = Y + (size_t)i * n + j;
             // accy: y += the product (the residual add, one rounding as x + y)
@@ -979,42 +1113,50 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     for (int b = 0; b < FO; b++) store_rows(ks * FO + b, own[b]);
 }
 
-// x split of m rows in the scratch (gemm_tiles_scratch_bytes(m, k)); lo: where
-// x_lo goes instead (m k 2 bytes), or NULL.
+// x split of m rows in the scratch (gemm_tiles_scratch_bytes(m, k), or
+// gemm_wide_scratch_bytes(m, k) where rows may be wide); lo: where x_lo goes
+// instead (m k 2 bytes), or NULL.
 struct XSplit {
     _Float16 *h, *l;
     int* e;
     uint32_t* s;  // x' sums of each block (hi / lo pairs), or NULL
+    float* b;     // [block][b_rows] scales of wide rows, or NULL
+    int b_rows;
+    uint8_t* f;   // whether a row is wide
 };
-XSplit x_split_at(void* scratch, void* lo, size_t m, size_t k, bool sums) {
+XSplit x_split_at(void* scratch, void* lo, size_t m, size_t k, bool sums, bool wide) {
     const size_t xb = (m * k * 2 + 255) & ~(size_t)255, eb = (m * 4 + 255) & ~(size_t)255;
     uint8_t* p = reinterpret_cast<uint8_t*>(scratch);
     uint8_t* e = p + (lo ? xb : 2 * xb);
+    uint8_t* f = e + eb;  // (first: a multiple of XF_PAD bytes)
+    const size_t fb = (m + 255) & ~(size_t)255;
     return {reinterpret_cast<_Float16*>(p), reinterpret_cast<_Float16*>(lo ? lo : p + xb), reinterpret_cast<int*>(e),
-            sums ? reinterpret_cast<uint32_t*>(e + eb) : nullptr};
+            sums ? reinterpret_cast<uint32_t*>(e + eb) : nullptr, wide ? reinterpret_cast<float*>(f + fb) : nullptr,
+            (int)m, f};
 }
 
 // One tile shape: 64 WJ weight rows x 16 FI x rows, KS wave groups sharing
 // each chunk's blocks.
-template <int WF, int FI, int WJ, int KS>
+template <int WF, int FI, int WJ, int KS, bool WIDE>
 hipError_t launch_tile_cfg(const uint8_t* w, int n, int nb, const XSplit& x, int m, int r0, int r1, float* y, int accy,
                            const TilePlan& p, float* part, int* cnt, hipStream_t s) {
-    using C = TileCfg<WF, FI, WJ, KS>;
+    using C = TileCfg<WF, FI, WJ, KS, WIDE>;
     static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
     const bool local = p.S > 1 && xcd_round_robin(s);
-    auto kern = local ? gemm_tile_kernel<WF, FI, WJ, KS, true> : gemm_tile_kernel<WF, FI, WJ, KS, false>;
+    auto kern = local ? gemm_tile_kernel<WF, FI, WJ, KS, true, WIDE> : gemm_tile_kernel<WF, FI, WJ, KS, false, WIDE>;
     if (C::LDS > 65536) {
         static const hipError_t e[2] = {
-            hipFuncSetAttribute((const void*)gemm_tile_kernel<WF, FI, WJ, KS, false>,
+            hipFuncSetAttribute((const void*)gemm_tile_kernel<WF, FI, WJ, KS, false, WIDE>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS),
-            hipFuncSetAttribute((const void*)gemm_tile_kernel<WF, FI, WJ, KS, true>,
+            hipFuncSetAttribute((const void*)gemm_tile_kernel<WF, FI, WJ, KS, true, WIDE>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS)};  // once a process
         if (e[local] != hipSuccess) return e[local];
     }
     unsigned rest = (unsigned)((n + C::TJ - 1) / C::TJ) * (unsigned)((m + C::TI - 1) / C::TI) - (unsigned)p.full;
     if (local) rest = (rest + 7) / 8 * 8;
     launch_kernel(kern, dim3((unsigned)p.full + rest * (unsigned)p.S), dim3(C::NT), (size_t)C::LDS, s, w, n, nb, x.h,
-                  x.l, x.e, m, r0, r1, x.s, y, accy, p.full, p.S, p.kbs, part, cnt);
+                  x.l, x.e, m, r0, r1, x.s, x.b, x.b_rows,
+                  reinterpret_cast<const uint32_t*>(x.f), y, accy, p.full, p.S, p.kbs, part, cnt);
     return hipGetLastError();
 }
 
@@ -1073,20 +1215,20 @@ TilePlan tile_plan(WType t, size_t m, size_t n, size_t nb, bool can_split) {
     return best;
 }
 
-template <int PRO>
+template <int PRO, int WB>
 hipError_t launch_split(const float* x, size_t m, size_t k, const float* g, float eps, const XSplit& o, hipStream_t s) {
     // 256 threads hold 4096 elements of a row, 1024 threads GEMM_SPLIT_MAX_K
     if (k > GEMM_SPLIT_MAX_K) {
-        if (PRO != 0 || o.s) return hipErrorInvalidValue;
+        if (PRO != 0 || WB != 0 || o.s) return hipErrorInvalidValue;
         launch_kernel(gemm_split_long_kernel, dim3((unsigned)m), dim3(1024), 0, s, x, (int)k, o.h, o.l, o.e);
         return hipGetLastError();
     }
     if (k <= 4096)
-        launch_kernel(gemm_split_kernel<PRO, 256, 4>, dim3((unsigned)m), dim3(256), 0, s, x, (int)k, g, eps, o.h, o.l,
-                      o.e, o.s);
+        launch_kernel(gemm_split_kernel<PRO, 256, 4, WB>, dim3((unsigned)m), dim3(256), 0, s, x, (int)k, g, eps, o.h,
+                      o.l, o.e, o.s, o.b, o.b_rows, o.f);
     else
-        launch_kernel(gemm_split_kernel<PRO, 1024, 4>, dim3((unsigned)m), dim3(1024), 0, s, x, (int)k, g, eps, o.h,
-                      o.l, o.e, o.s);
+        launch_kernel(gemm_split_kernel<PRO, 1024, 4, WB>, dim3((unsigned)m), dim3(1024), 0, s, x, (int)k, g, eps, o.h,
+                      o.l, o.e, o.s, o.b, o.b_rows, o.f);
     return hipGetLastError();
 }
 
@@ -1151,11 +1293,11 @@ size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k) {
     return rest * p.S * sh.tj * sh.ti * sizeof(float);
 }
 
-template <int WF>
+template <int WF, bool WIDE = false>
 static hipError_t launch_tile_wf(const uint8_t* w, int n, int nb, const XSplit& x, int m, int r0, int r1, float* y,
                                  int accy, const TilePlan& p, float* part, int* cnt, hipStream_t s) {
     auto go = [&](auto fi, auto wj, auto ks) {
-        return launch_tile_cfg<WF, decltype(fi)::value, decltype(wj)::value, decltype(ks)::value>(
+        return launch_tile_cfg<WF, decltype(fi)::value, decltype(wj)::value, decltype(ks)::value, WIDE>(
             w, n, nb, x, m, r0, r1, y, accy, p, part, cnt, s);
     };
     using I1 = std::integral_constant<int, 1>;
@@ -1180,18 +1322,23 @@ hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const
     if (chunk < m && chunk % TILE_SHAPES[0].ti != 0) return hipErrorInvalidValue;
     const TilePlan p = tile_plan(t, m, n, k / QK, part != nullptr && cnt != nullptr);
     const int ni = (int)n, nb = (int)(k / QK), mi = (int)m, acc = accumulate ? 1 : 0;
+    const bool few = t == WType::Q4_0 && pro == 0 && m <= GEMM_XTILE_M;  // (the x-tile kernel's rows)
     for (size_t r0 = 0; r0 < m; r0 += chunk) {
         const size_t rows = std::min(chunk, m - r0);
         const int a = (int)r0, b = (int)(r0 + rows);
-        const XSplit xo = x_split_at(scratch, lo, rows, k, t == WType::Q4_K);
+        const XSplit xo = x_split_at(scratch, lo, rows, k, t == WType::Q4_K, few || pro == 3);
         const float* xr = x + r0 * k * (pro == 2 ? 2 : 1);
-        hipError_t e = pro == 1   ? launch_split<1>(xr, rows, k, g, eps, xo, s)
-                       : pro == 2 ? launch_split<2>(xr, rows, k, g, eps, xo, s)
-                       : pro == 3 ? launch_split<3>(xr, rows, k, g, eps, xo, s)
-                                  : launch_split<0>(xr, rows, k, g, eps, xo, s);
+        hipError_t e = pro == 1   ? launch_split<1, 0>(xr, rows, k, g, eps, xo, s)
+                       : pro == 2 ? launch_split<2, 0>(xr, rows, k, g, eps, xo, s)
+                       : pro == 3 ? launch_split<3, WIDE_NATIVE>(xr, rows, k, g, eps, xo, s)
+                       : few      ? launch_split<0, WIDE_FLOAT>(xr, rows, k, g, eps, xo, s)
+                                  : launch_split<0, 0>(xr, rows, k, g, eps, xo, s);
         if (e != hipSuccess) return e;
         switch (t) {
-            case WType::Q4_0: e = launch_tile_wf<WF_Q4_0>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s); break;
+            case WType::Q4_0:
+                e = xo.b ? launch_tile_wf<WF_Q4_0, true>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s)
+                         : launch_tile_wf<WF_Q4_0>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s);
+                break;
             case WType::Q8_0: e = launch_tile_wf<WF_Q8_0>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s); break;
             case WType::Q4_K: e = launch_tile_wf<WF_Q4_K>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s); break;
             default: e = launch_tile_wf<WF_Q6_K>(w, ni, nb, xo, mi, a, b, y, acc, p, part, cnt, s);
@@ -1201,11 +1348,16 @@ hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const
     return hipSuccess;
 }
 
+size_t gemm_wide_scratch_bytes(size_t m, size_t k) {
+    const size_t xb = (m * k * 2 + 255) & ~(size_t)255;
+    return 2 * xb + ((m * 4 + 255) & ~(size_t)255) + ((m + 255) & ~(size_t)255) + ((m * (k / QK) * 4 + 255) & ~(size_t)255);
+}
+
 size_t gemm_tile_chunk_rows(size_t k, size_t bytes, size_t lo_bytes) {
     const size_t ti = TILE_SHAPES[0].ti;  // (the other shapes' rows divide it)
-    size_t rows = std::min(lo_bytes / (k * 2), bytes / (k * 2 + 4)) / ti * ti;
-    // x_hi, the exponents, each rounded up to 256 bytes
-    while (rows > 0 && ((rows * k * 2 + 255) & ~(size_t)255) + ((rows * 4 + 255) & ~(size_t)255) > bytes) rows -= ti;
+    size_t rows = lo_bytes / (k * 2) / ti * ti;
+    // x_hi, the exponents and the blocks' scales
+    while (rows > 0 && gemm_wide_scratch_bytes(rows, k) - ((rows * k * 2 + 255) & ~(size_t)255) > bytes) rows -= ti;
     return rows;
 }
 

@@ -712,7 +712,8 @@ struct LlamaModel {
         if (m <= 4) return 0;  // GEMVs
         const size_t n = w.n, k = w.k;
         if (w.type == WType::Q4_0)
-            return gemm_scratch_bytes(m, n, k, native && !gemm_native_tile_takes(m, n, k));
+            return native && gemm_native_tile_takes(m, n, k) ? gemm_wide_scratch_bytes(m, k)
+                                                             : gemm_scratch_bytes(m, n, k, native);
         return kgemm(w, m, native) ? gemm_tiles_scratch_bytes(m, k) : 0;
     }
     // The most that any chunk of up to max_batch rows writes there, in float or
@@ -732,7 +733,8 @@ struct LlamaModel {
             for (size_t m = 1; m <= std::min(mb, GEMM_SMALL_M); m++)
                 for (bool native : {false, true}) need = std::max(need, product_scratch(w, m, native));
             if (w.type == WType::Q4_0 && mb > GEMM_SMALL_M)
-                for (bool native : {false, true}) need = std::max(need, gemm_scratch_bytes(mb, w.n, w.k, native));
+                need = std::max({need, gemm_scratch_bytes(mb, w.n, w.k, false), gemm_scratch_bytes(mb, w.n, w.k, true),
+                                 gemm_wide_scratch_bytes(mb, w.k)});
             else
                 need = std::max(need, product_scratch(w, mb, false));
         }

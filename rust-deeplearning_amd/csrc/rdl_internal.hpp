@@ -208,8 +208,11 @@ size_t gemm_part_bytes(WType t, size_t m, size_t n, size_t k);
 // kernel of gemm.hip.
 bool gemm_tile_takes(WType t, size_t m, size_t n, size_t k);
 // Whether a native-mode Q4_0 product takes it (launch_gemm_tile with pro 3,
-// scratch gemm_scratch_bytes(m, n, k, false)).
+// scratch gemm_wide_scratch_bytes(m, k)).
 bool gemm_native_tile_takes(size_t m, size_t n, size_t k);
+// The x split with a scale for every block beside it (Q4_0 rows of wide range:
+// native products, and float ones of at most GEMM_XTILE_M rows).
+size_t gemm_wide_scratch_bytes(size_t m, size_t k);
 hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* cnt, int pro, const float* g, float eps, bool accumulate,
                             hipStream_t s, void* lo = nullptr, size_t chunk = 0);

@@ -175,3 +175,69 @@ def test_native_tiles_nan_inf_and_zero_rows(rq, orc, gpu):
     tol = 1e-6 * 16 * np.abs(np.where(ok, want, 0.0)).max(axis=1, keepdims=True) * np.ones_like(want)
     assert np.all(np.abs(got[rows] - want)[ok] <= tol[ok])
     assert np.isfinite(np.delete(got, [7, 9], axis=0)).all()
+
+
+def wide_rows(m, k, seed, low):
+    """Rows of three kinds in turn: an outlier block (2^10) with every other block
+    `low` binades or more below it, an ordinary row, a row of zeros and tiny values."""
+    r = np.random.default_rng(seed)
+    x = synth.activations(m, k, seed).reshape(m, k // 32, 32)
+    x[0::3] *= (2.0 ** -(low - 10.0 + r.integers(0, 8, size=x[0::3].shape[:2])))[..., None]
+    x[0::3, 0] *= 2.0 ** (low - 10.0) * 2.0 ** 10
+    x[2::3, 1:] *= 1e-30
+    x[2::3, 0] = 0.0
+    return np.ascontiguousarray(x.reshape(m, k), dtype=np.float32)
+
+
+def weights_without_block_0(n, k, seed):
+    """Q4_0 weights whose first block has the code of zero throughout."""
+    w = synth.q4_0_weights(n, k, seed).reshape(n, k // 32, 18).copy()
+    w[:, 0, 2:] = 0x88
+    return w.reshape(-1)
+
+
+# A row's other blocks count for all of a result where its largest block meets
+# zero weights.  5 to 64 rows on each tile shape, split and unsplit, ragged, and
+# (16 x 4096 x 4096) on the x-tile kernel.  Each output within 1e-6 sum |w x|:
+# 2^-22 a split element, f32 sums of 33 to 512 blocks whose roundings (2^-24
+# each) add up as a random walk
+@pytest.mark.parametrize("low", [11, 15, 20, 27, 40])
+@pytest.mark.parametrize("m,n,k", [(16, 4096, 4096), (16, 510, 4128), (7, 24600, 4096), (32, 300, 16384), (64, 1000, 2080),
+                                   (64, 14336, 4096), (33, 4100, 4128)])
+def test_rows_of_wide_range(rq, orc, gpu, m, n, k, low):
+    print(f"case wide rows m={m} n={n} k={k} low={low}", flush=True)
+    x, w = wide_rows(m, k, m + n + low, low), weights_without_block_0(n, k, n)
+    got = rq.matmul_f32_q4(x, w, m, k, n).reshape(m, n)
+    rows = np.unique(np.linspace(0, m - 1, 9).astype(int))
+    exact, cond = exact_f64_cond(orc, "q4", x[rows], w, len(rows), k, n)
+    assert np.all(np.abs(got[rows].reshape(-1) - exact) <= 1e-6 * cond)
+
+
+# the same in native mode: the int32 dots times both scales, in 64 bits (a
+# scale of x below the f16 range is 0, as in the reference)
+@pytest.mark.parametrize("low", [11, 20, 24, 30])
+@pytest.mark.parametrize("m,n,k", [(65, 4096, 4096), (257, 70, 4128), (513, 1000, 4096), (1030, 2049, 96),
+                                   (512, 14336, 2048)])
+def test_native_rows_of_wide_range(rq, orc, gpu, m, n, k, low):
+    print(f"case native wide rows m={m} n={n} k={k} low={low}", flush=True)
+    x, w = wide_rows(m, k, m + n + low, low), weights_without_block_0(n, k, n)
+    x[2::3] = x[0:m - 2:3][:len(x[2::3])] * 2.0 ** 9  # (in the f16 scales' range)
+    got = rq.matmul_f32_q4_native(x, w, m, k, n).reshape(m, n)
+    rows = np.unique(np.linspace(0, m - 1, 9).astype(int))
+    part = orc.block_dots(x[rows], w, len(rows), k, n).reshape(len(rows), n, k // 32).astype(np.float64)
+    sw = w.reshape(n, k // 32, 18)[:, :, 0:2].copy().view(np.float16).astype(np.float64)[..., 0]
+    sx = np.stack([orc.quantize_row_q8_0(x[r])[1] for r in rows]).astype(np.float64)
+    terms = part * sx[:, None, :] * sw[None]
+    # (within a block the products cancel before the f32 sum: 16 times the block's
+    # dot covers that here)
+    assert np.all(np.abs(got[rows] - terms.sum(axis=2)) <= 1e-6 * (np.abs(terms).sum(axis=2) * 16 + 1e-30))
+
+
+def test_wide_row_with_an_infinite_value(rq, orc, gpu):
+    m, n, k = 40, 300, 1024
+    x, w = wide_rows(m, k, 3, 24), weights_without_block_0(n, k, 4)
+    x[3, 77], x[6, 900] = np.inf, -np.inf
+    got = rq.matmul_f32_q4(x, w, m, k, n).reshape(m, n)
+    want = orc.matmul("q4", x[[3, 6]], w, 2, k, n).reshape(2, n)
+    assert np.array_equal(got[[3, 6]], want, equal_nan=True)
+    assert np.isfinite(np.delete(got, [3, 6], axis=0)).all()
