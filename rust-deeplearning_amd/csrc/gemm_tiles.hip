@@ -93,6 +93,11 @@ __device__ __forceinline__ int split_exponent(uint32_t am, uint32_t* red, uint32
     return am != 0 ? ilogbf(__builtin_bit_cast(float, am)) - 14 : 0;
 }
 
+// The low half of a block's sum is stored times 2^12 (at most 8 before): its own
+// last place, 2^-24, would be that of single elements, and 10 times their error in a
+// block far below its row's largest.
+constexpr float SUM_LO = 4096.0f;
+
 // The split of elements 4 p .. 4 p + 3 of a row (p = t modulo 8).  Thread c = t %
 // 8 of a block's eight holds elements 4c .. 4c+3.  Threads c and c ^ 4 trade
 // halves: c < 4 ends with the block's x_hi piece g = c (elements of 4c and 16 +
@@ -118,10 +123,10 @@ __device__ __forceinline__ void split_piece(const f32x4& v, int e, int p, int k4
     const uint32_t r1 = (uint32_t)__shfl_xor((int)(upper ? h13 : l13), 4);
     const u32x4 o = upper ? u32x4{r0, l02, r1, l13} : u32x4{h02, r0, h13, r1};
     if (p < k4) *reinterpret_cast<u32x4*>((upper ? xl : xh) + (size_t)(p >> 3) * 32 + (p & 3) * 8) = o;
-    if (xs) {  // the block's sum of x', over 32, as an f16 hi / lo pair
+    if (xs) {  // the block's sum of x', over 32, as an f16 hi / lo pair, lo times SUM_LO
         bs = sum8_f32(bs) * 0.03125f;
         const _Float16 sh = (_Float16)bs;
-        const half2_t sp = {sh, (_Float16)(bs - (float)sh)};
+        const half2_t sp = {sh, (_Float16)((bs - (float)sh) * SUM_LO)};
         if ((threadIdx.x & 7) == 0 && p < k4) xs[p >> 3] = __builtin_bit_cast(uint32_t, sp);
     }
 }
@@ -287,7 +292,10 @@ constexpr int CPOL_NT = 2, CPOL_SC1 = 16;
 //  * Q4_K: (q - 8) sc is exact in f16.  What remains, e_j = 8 d sc_j - dmin
 //    mn_j times S_j, the sum of x' over sub-block j, is one more MFMA a
 //    super-block: eight sub-blocks times the four products of the f16 hi / lo
-//    pairs of e_j 2^-t (t by the row's larger of 8 d, dmin) and of S_j / 32.
+//    pairs of e_j 2^-t (t by the larger of the row's 8 d and dmin) and of S_j / 32
+//    (lo times SUM_LO, against e_j / SUM_LO, which is staged too: multiplied as it
+//    is read it cost the loop 7 %).  e_j keeps its 22 bits down to 2^-17 of the
+//    super-block's largest, S_j always.
 //    (e_j first, in f32: d q sc and dmin mn nearly cancel, and summing them
 //    apart doubled the error against 64 bits.)
 //  * Q6_K: (q - 32) sc has up to 13 bits: hi = f16(.) and the exact rest lo (at
@@ -322,9 +330,9 @@ struct TileCfg {
     static constexpr int XU = (TI * CB * 4 + NT - 1) / NT;  // 16-byte pieces a thread stages, hi and lo each
     static constexpr int RED = (KS - 1) * WJ * FI * FJ * 1024;
     // a super-block's own data (CHAIN): d (and Q4_K's t) of each row, Q4_K's e
-    // [row][hi / lo][8] f16 and x sums [tile][hi / lo][16 rows][8] f16
+    // [row][hi, hi / SUM_LO, lo, lo / SUM_LO][8] f16 and x sums [tile][hi / lo][16 rows][8] f16
     static constexpr int SU = WF == WF_Q4_K ? (TI * CB + NT - 1) / NT : 0;  // sum pairs a thread stages
-    static constexpr int MN_AT = TJ * 4, SS_AT = MN_AT + TJ * 32;
+    static constexpr int MN_AT = TJ * 4, SS_AT = MN_AT + TJ * 64;
     static constexpr int AUX = !CHAIN ? 0 : WF == WF_Q4_K ? SS_AT + TI * 32 : MN_AT;
     // three stages and three super-blocks' data, or the sums at the end; the x
     // rows' exponents behind them
@@ -602,13 +610,18 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
                 const uint32_t mn = j < 4 ? ti & 63u : ((ti >> 6) & 3u) | ((ui >> 2) & 60u);
                 reinterpret_cast<_Float16*>(st + C::W_BYTES)[bl * C::TJ + jl] = (_Float16)(float)sc;
                 const float d8 = 8.0f * h2f(R.w[u][0] & 0xFFFFu), dm = h2f(R.w[u][0] >> 16);
-                // t by the exponent bits of the larger: |e 2^-t| < 2^15
-                const int t = (int)(max(abs_bits(d8), abs_bits(dm)) >> 23) - 134;
+                // t by the exponent bits of the larger that any sub-block uses: |e 2^-t| < 2^15
+                const uint32_t bd = (R.w[u][1] | (R.w[u][3] & 0x0F0F0F0Fu)) != 0 ? abs_bits(d8) : 0u;
+                const uint32_t bm = (R.w[u][2] | (R.w[u][3] & 0xF0F0F0F0u)) != 0 ? abs_bits(dm) : 0u;
+                const int t = (int)(max(bd, bm) >> 23) - 134;
                 const float e = ldexpf(d8 * (float)sc - dm * (float)mn, -t);
                 const _Float16 eh = (_Float16)e;
-                _Float16* em = reinterpret_cast<_Float16*>(aux + C::MN_AT) + jl * 16 + j;
+                const _Float16 el = (_Float16)(e - (float)eh), inv = (_Float16)(1.0f / SUM_LO);
+                _Float16* em = reinterpret_cast<_Float16*>(aux + C::MN_AT) + jl * 32 + j;
                 em[0] = eh;
-                em[8] = (_Float16)(e - (float)eh);
+                em[8] = eh * inv;
+                em[16] = el;
+                em[24] = el * inv;
                 reinterpret_cast<uint32_t*>(aux)[jl] = (R.w[u][0] & 0xFFFFu) | ((uint32_t)t << 16);  // d, t
                 continue;
             }
@@ -761,7 +774,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     // the FI steps of the next chunk: step b adds x tile b, and Q4_K's remainder
     // of weight column b for the FO tiles ks FO .. that this K group ends with
     // (um, so that the KS groups share them).  K elements 8 g .. of that MFMA:
-    // S hi, lo, hi, lo times e hi, hi, lo, lo.
+    // S hi, lo, hi, lo times e hi, hi, lo, lo (against S lo: over SUM_LO).
     constexpr int FO = FI / KS;
     static_assert(!CHAIN || FI == FJ, "a weight column a step");
     f32x4 um[Q4K ? FO : 1][FJ];
@@ -769,7 +782,7 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     half8_t fs[Q4K ? FO : 1], fe;   // S of the tiles, e of the step's column
     auto flush_e = [&](int a, const uint8_t* aux) {
         if constexpr (Q4K)
-            fe = *reinterpret_cast<const half8_t*>(aux + C::MN_AT + (wj * 64 + r * 4 + a) * 32 + (g >> 1) * 16);
+            fe = *reinterpret_cast<const half8_t*>(aux + C::MN_AT + (wj * 64 + r * 4 + a) * 64 + g * 16);
     };
     auto flush_begin = [&](const uint8_t* aux) {
         fd = *reinterpret_cast<const u32x4*>(aux + (wj * 64 + r * 4) * 4);

@@ -241,3 +241,49 @@ def test_wide_row_with_an_infinite_value(rq, orc, gpu):
     want = orc.matmul("q4", x[[3, 6]], w, 2, k, n).reshape(2, n)
     assert np.array_equal(got[[3, 6]], want, equal_nan=True)
     assert np.isfinite(np.delete(got, [3, 6], axis=0)).all()
+
+
+# K-quant rows keep one power of two a row, so an element of a block 2^low below
+# the row's largest is known to 2^(low - 40) of that block's largest (half of 2^-24
+# of x' over 2^15-low); the block's sum, for Q4_K's minimums, has to be as good
+@pytest.mark.parametrize("kind,dtype", [("q4k", 12), ("q6k", 14)])
+@pytest.mark.parametrize("low", [14, 17, 20, 24, 28])
+def test_super_block_rows_of_wide_range(rq, orc, gpu, kind, dtype, low):
+    print(f"case super block wide rows {kind} low={low}", flush=True)
+    m, n, k = 70, 257, 4096
+    x = synth.activations(m, k, low).reshape(m, k // 32, 32) * np.float32(2.0 ** -low)
+    x[:, 0] *= np.float32(2.0 ** low)
+    x = np.ascontiguousarray(x.reshape(m, k))
+    w = synth.weights(dtype, n, k, 5).reshape(n, k // 256, -1).copy()
+    if dtype == 12:  # the first 32 elements: scale and min 0
+        w[:, 0, 4] &= 0xC0
+        w[:, 0, 8] &= 0xC0
+    else:
+        w[:, 0, 192:194] = 0
+    w = w.reshape(-1)
+    got = getattr(rq, "matmul_f32_q4_k" if dtype == 12 else "matmul_f32_q6_k")(x, w, m, k, n)
+    exact, cond = exact_f64_cond(orc, kind, x, w, m, k, n)
+    assert np.all(np.abs(got - exact) <= (2.0 ** -22 + 2.0 ** (low - 40)) * cond)
+
+
+def test_q4_k_minimum_scale_without_minimums(rq, orc, gpu):
+    # dmin far above d where every sub-block's minimum is 0 (and the other way round)
+    m, n, k = 70, 130, 4096
+    r = np.random.default_rng(11)
+    w = synth.weights(12, n, k, 12).reshape(n, k // 256, 144).copy()
+    small = synth.f16_bits((1.0 + r.random((n, k // 256))) * 2.0 ** -18)[..., None].view(np.uint8).reshape(n, k // 256, 2)
+    big = synth.f16_bits((1.0 + r.random((n, k // 256))) * 2.0 ** 12)[..., None].view(np.uint8).reshape(n, k // 256, 2)
+    w[..., 0:2], w[..., 2:4] = small, big
+    w[..., 4:8] &= 0x3F      # sub-blocks 0-3: scales; 4-7's high bits
+    w[..., 8:12] = 0
+    w[..., 12:16] &= 0x0F
+    half = n // 2            # these rows: d large, scales 0, minimums in use
+    w[half:, :, 0:2], w[half:, :, 2:4] = big[half:], small[half:]
+    w[half:, :, 8:12] = w[half:, :, 4:8]
+    w[half:, :, 4:8] = 0
+    w[half:, :, 12:16] <<= 4
+    w = w.reshape(-1)
+    x = synth.activations(m, k, 13)
+    got = rq.matmul_f32_q4_k(x, w, m, k, n)
+    exact, cond = exact_f64_cond(orc, "q4k", x, w, m, k, n)
+    assert np.all(np.abs(got - exact) <= 1e-6 * cond)
