@@ -752,8 +752,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         const uint32_t d16 = a & 1 ? dd[a >> 1] >> 16 : dd[a >> 1] & 0xFFFFu;
         if constexpr (Q4K) {
             const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)d16);
-            wq[ONE ? 0 : o][a] = q4k_f16(n0, n1, kmask, qc.magic, __builtin_bit_cast(half2_t, kmul),
-                                              __builtin_bit_cast(half2_t, koff), sc);
+            wq[o][a] = q4k_f16(n0, n1, kmask, qc.magic, __builtin_bit_cast(half2_t, kmul),
+                               __builtin_bit_cast(half2_t, koff), sc);
             return;
         }
         if constexpr (BYTES) wq[o][a] = q8_f16(n0, n1);
@@ -818,7 +818,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     };
     // chunks the loads run ahead (no registers for more)
     constexpr int DX = FI == 8 || CHAIN ? 1 : 2, DW = (FI == 8 && BYTES) || CHAIN ? 1 : 2;
-    constexpr int UN = CHAIN ? 8 / CB : 2;  // chunks a turn of the loop: a super-block, or two
+    constexpr int UN = 2;  // chunks a turn of the loop (CHAIN: a super-block)
+    static_assert(!CHAIN || UN * CB == 8, "a super-block a turn");
     WRegs w[DW];
     XRegs x1[DX];
     uint8_t *bc = lds, *bn = lds + C::STAGE, *bf = lds + 2 * C::STAGE;  // chunk c, c + 1, free
@@ -952,10 +953,6 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         for (int c = 0; c < nchunks; c += UN) {
             chunk(c, std::integral_constant<int, 0>{}, plain);
             chunk(c + 1, std::integral_constant<int, 1>{}, plain);
-            if constexpr (UN == 4) {
-                chunk(c + 2, std::integral_constant<int, 2>{}, plain);
-                chunk(c + 3, std::integral_constant<int, 3>{}, plain);
-            }
         }
         if constexpr (CHAIN) {
 #pragma unroll

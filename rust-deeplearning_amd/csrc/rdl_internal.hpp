@@ -165,16 +165,16 @@ int device_cu_count();
 
 // Prefill GEMM for Q4_0 weights on the matrix cores: y[m, n] = x[m, k] . W^T.
 // Float mode (matmul_f32_q4): `scratch` holds gemm_scratch_bytes(m, n, k,
-// false) bytes (the f16 x split; for m <= GEMM_SMALL_M the skinny kernel's
-// K-slice partials, none when it runs unsplit) and `counters` points to
-// gemm_counter_count(n, k) ints that are zero before the first call and that
-// every call leaves at zero (memory no other code writes; NULL runs the
-// skinny kernels unsplit).  Native mode (matmul_f32_q4_native): x quantized
+// false) bytes (where gemm_tile_takes(Q4_0, m, n, k), and past GEMM_XTILE_M
+// rows, the f16 x split; otherwise the K-slice partials of the few-row kernels,
+// none when they run unsplit) and `counters` points to gemm_counter_count(n, k)
+// ints that are zero before the first call and that every call leaves at zero
+// (memory no other code writes; NULL runs every kernel unsplit).  Native mode (matmul_f32_q4_native): x quantized
 // to Q8_0 codes, int8 MFMA block dots; gemm_scratch_bytes(m, n, k, true)
 // bytes of scratch; partials != NULL writes the int32 block dots to
 // partials[(i * n + j) * (k / 32) + b] instead of y.
 constexpr size_t GEMM_SMALL_M = 64;
-constexpr size_t GEMM_XTILE_M = 64;  // float products of at most this many rows: x tiles as MFMA A operands, 128-row strips
+constexpr size_t GEMM_XTILE_M = 64;  // float products of at most this many rows that the tile GEMM does not take: the x-tile kernel
 constexpr size_t KQ_GEMM_MIN_M = 16;  // Q4_K / Q6_K / Q8_0 / Q4_1 float products of at least this many rows: the LDS tile GEMM
 size_t gemm_scratch_bytes(size_t m, size_t n, size_t k, bool native);
 // ints of the GEMM's strip counters for out_features n, in_features k
@@ -190,7 +190,7 @@ bool combine_is_coherent();
 // probed and a rotation, switch off); does not probe.
 bool combine_local_now();
 // part: gemm_part_bytes(Q4_0, m, n, k) bytes for the K-slice partials of the tile
-// GEMM (m > GEMM_XTILE_M); NULL (or no counters): that GEMM runs unsplit.
+// GEMM where gemm_tile_takes(Q4_0, m, n, k); NULL (or no counters): it runs unsplit.
 hipError_t launch_gemm_q4_0(const uint8_t* w, size_t n, size_t k, const float* x, size_t m, float* y,
                             void* scratch, float* part, int* counters, hipStream_t s);
 // True when workgroup b of a launch runs on XCD (b + o) % 8 on the current
