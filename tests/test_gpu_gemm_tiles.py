@@ -46,17 +46,30 @@ def test_few_rows(rq, orc, gpu, m, n, k):
     check_parity(got[rows].reshape(-1), want, exact_f64(orc, "q4", x[rows], w, len(rows), k, n))
 
 
-@pytest.mark.parametrize("m", [20, 40, 300])
-def test_rows_with_an_infinite_value(rq, orc, gpu, m):
+@pytest.mark.parametrize("kind,dtype,m,k", [("q4", 2, 20, 1024), ("q4", 2, 40, 1024), ("q4", 2, 300, 1024),
+                                            ("q8", 8, 40, 4096), ("q8", 8, 300, 4096)])
+def test_rows_with_an_infinite_value(rq, orc, gpu, kind, dtype, m, k):
     # +-inf where the weight is not zero, NaN where it is, as in the reference;
     # rows beside it and a row's own finite values keep theirs
-    n, k = 300, 1024
+    n = 300
     x = synth.activations(m, k, 21 + m)
     x[3, 77], x[5, 900] = np.inf, -np.inf
-    w = synth.q4_0_weights(n, k, 22)
-    got = rq.matmul_f32_q4(x, w, m, k, n).reshape(m, n)
-    want = orc.matmul("q4", x[[3, 5]], w, 2, k, n).reshape(2, n)
+    w = synth.weights(dtype, n, k, 22)
+    got = getattr(rq, f"matmul_f32_{kind}")(x, w, m, k, n).reshape(m, n)
+    want = orc.matmul(kind, x[[3, 5]], w, 2, k, n).reshape(2, n)
     assert np.array_equal(got[[3, 5]], want, equal_nan=True)
+    assert np.isfinite(np.delete(got, [3, 5], axis=0)).all()
+
+
+# the formats whose operands or sums are split again, and the small-tile kernel: such
+# rows are infinite or NaN throughout (inf - inf, inf times a zero half), others untouched
+@pytest.mark.parametrize("kind,dtype,m,k", [("q4_k", 12, 70, 4096), ("q6_k", 14, 70, 4096), ("q4", 2, 100, 1024)])
+def test_rows_with_an_infinite_value_elsewhere(rq, gpu, kind, dtype, m, k):
+    n = 300
+    x = synth.activations(m, k, 23 + m)
+    x[3, 77], x[5, 900] = np.inf, -np.inf
+    got = getattr(rq, f"matmul_f32_{kind}")(x, synth.weights(dtype, n, k, 24), m, k, n).reshape(m, n)
+    assert not np.isfinite(got[[3, 5]]).any()
     assert np.isfinite(np.delete(got, [3, 5], axis=0)).all()
 
 
@@ -100,41 +113,56 @@ def test_super_block_tiles_extreme_scales(rq, orc, gpu, kind, dtype):
     assert np.all(got.reshape(m, n)[:, 1] == 0.0)
 
 
-@pytest.mark.parametrize("m,n,k", [(128, 1024, 4096), (100, 4096, 1024)])
-def test_split_tiles_combines_and_replays_agree(rq, gpu, m, n, k):
+# every tile split, no tile split (Q4_0: the small-tile kernel), whole tiles with a
+# split last round; two inputs in turn
+# through one workspace, so that a partial of the call before shows
+@pytest.mark.parametrize("kind,dtype", [("q4", 2), ("q8", 8), ("q4k", 12), ("q6k", 14)])
+@pytest.mark.parametrize("m,n,k", [(128, 1024, 4096), (100, 4096, 1024), (300, 7000, 4096)])
+def test_split_tiles_combines_and_replays_agree(rq, orc, gpu, kind, dtype, m, n, k):
     # the XCD-local and the agent-coherent combine and a captured call give the
-    # same bits, call after call (the counters return to zero)
+    # same bits, call after call (the counters return to zero), and each is within
+    # 1e-6 sum |w x| of the exact product
     import torch
-    print(f"case split tiles m={m} n={n} k={k}", flush=True)
-    w = rq.Weight.upload(synth.q4_0_weights(n, k, 5), rq.DTYPE_Q4_0, n, k)
-    x = torch.from_numpy(synth.activations(m, k, 6)).to(gpu)
+    print(f"case split tiles {kind} m={m} n={n} k={k}", flush=True)
+    raw = synth.weights(dtype, n, k, 5)
+    w = rq.Weight.upload(raw, dtype, n, k)
+    hosts = [synth.activations(m, k, seed) for seed in (6, 7)]
+    xs = [torch.from_numpy(h).to(gpu) for h in hosts]
+    rows = np.unique(np.linspace(0, m - 1, 16).astype(int))
+    exact = [exact_f64_cond(orc, kind, h.reshape(m, k)[rows], raw, len(rows), k, n) for h in hosts]
+    main = torch.cuda.current_stream().cuda_stream
 
-    def product(stream):
+    def product(i):
         y = torch.full((m, n), np.nan, device=gpu)
-        w.forward_dev(x.data_ptr(), m, y.data_ptr(), rq.MODE_FLOAT, stream)
+        w.forward_dev(xs[i].data_ptr(), m, y.data_ptr(), rq.MODE_FLOAT, main)
         return y
 
-    main = torch.cuda.current_stream().cuda_stream
-    want = product(main)
+    def check(i, y):
+        want, cond = exact[i]
+        assert np.all(np.abs(y.cpu().numpy()[rows].reshape(-1) - want) <= 1e-6 * cond)
+        assert torch.equal(y, first[i])
+
+    local = [product(i % 2) for i in range(6)]
     try:
         rq.set_gemm_combine(rq.COMBINE_COHERENT)
-        coherent = [product(main) for _ in range(3)]
+        coherent = [product(i % 2) for i in range(6)]
     finally:
         rq.set_gemm_combine(rq.COMBINE_AUTO)
-    local = [product(main) for _ in range(3)]
+    first = local[:2]
+    for i, (a, b) in enumerate(zip(local, coherent)):
+        check(i % 2, a)
+        check(i % 2, b)
+    g, side, x, y = torch.cuda.CUDAGraph(), torch.cuda.Stream(), xs[0].clone(), torch.empty(m, n, device=gpu)
     torch.cuda.synchronize()
-    g, side, y = torch.cuda.CUDAGraph(), torch.cuda.Stream(), torch.empty(m, n, device=gpu)
     with torch.cuda.graph(g, stream=side):
         w.forward_dev(x.data_ptr(), m, y.data_ptr(), rq.MODE_FLOAT, side.cuda_stream)
-    for got in coherent + local:
-        assert torch.equal(got, want)
-    for _ in range(3):
+    for i in (1, 0, 1, 0):
+        x.copy_(xs[i])
         y.fill_(np.nan)
         g.replay()
         torch.cuda.synchronize()
-        assert torch.equal(y, want)
-        product(main)
-        torch.cuda.synchronize()
+        check(i, y)
+        check(1 - i, product(1 - i))
     w.free()
 
 

@@ -46,6 +46,27 @@ def test_noalloc_matches_allocating_entry_point(rq, gpu, dtype, mode, n, k, rows
     w.free()
 
 
+def test_noalloc_row_chunks_with_rows_of_wide_range(rq, gpu):
+    """Native rows with a scale a block (a block far below the row's largest) in
+    both chunks of a product that runs 512 rows at a time."""
+    import torch
+    m, n, k = 600, 300, 14336
+    w = rq.Weight.upload(synth.weights(2, n, k, 41), 2, n, k)
+    x = synth.activations(m, k, 42).reshape(m, k).copy()
+    for i in (0, 130, 511, 512, 599):
+        x[i, 32:] *= np.float32(2.0 ** -8)
+        x[i, :32] *= np.float32(2.0 ** 14)
+        x[i, 64:96] *= np.float32(2.0 ** -3)
+    xd = torch.from_numpy(x).to(gpu)
+    stream = torch.cuda.current_stream().cuda_stream
+    want, got = (torch.full((m, n), np.nan, dtype=torch.float32, device=gpu) for _ in range(2))
+    w.forward_dev(xd.data_ptr(), m, want.data_ptr(), rq.MODE_NATIVE, stream)
+    w.forward_dev_noalloc(xd.data_ptr(), m, got.data_ptr(), rq.MODE_NATIVE, stream)
+    torch.cuda.synchronize()
+    assert torch.isfinite(want).all() and torch.equal(got, want)
+    w.free()
+
+
 def test_noalloc_rejects_products_beyond_its_scratch(rq, gpu):
     import torch
     n, k, m = 256, 4096, 2048  # the GEMM's activation split needs 32 MiB > 16 MiB
