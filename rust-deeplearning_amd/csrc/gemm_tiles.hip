@@ -25,8 +25,8 @@
 // through LDS as nibbles (16 bytes a block) and become f16 operands in the
 // registers of the one wave column that uses them, so LDS holds three chunks
 // of x and W and the loads run one and two chunks ahead of the matrix cores.
-// Counters at 2048 x 4096 x 14336: matrix cores busy 53 %, VALU issue 55 %,
-// bank conflicts 8 % of LDS cycles; the clock settles near 1.95 GHz.  2048
+// Counters at 2048 x 14336 x 4096 / 4096 x 14336: matrix cores busy 54 / 57 %,
+// VALU issue 58 / 59 %, bank conflicts 8 % of LDS cycles, clock 2.0 GHz.  2048
 // rows, 14336 x 4096 / 4096 x 14336: 631 / 615 -> 480 / 455 us (501 / 528
 // TFLOP/s; the matrix cores do twice that, x being two operands); 512 rows
 // 14336 x 4096: 213 -> 127 us; 128 rows 4096 x 4096 / 14336 x 4096 / 4096 x
@@ -468,14 +468,6 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
     const __amdgpu_buffer_rsrc_t hrs = make_rsrc(XH, (uint32_t)(r1 - r0) * k * 2u);
     const __amdgpu_buffer_rsrc_t lrs = make_rsrc(XL, (uint32_t)(r1 - r0) * k * 2u);
     const int nchunks = (kb1 - kb0 + CB - 1) / CB;
-
-    bool wide = false;
-    if constexpr (WIDE) {
-        uint32_t any = 0;
-#pragma unroll
-        for (int q = 0; q < C::TI / 4; q++) any |= XF[(i0 - r0) / 4 + q];
-        wide = __builtin_amdgcn_readfirstlane(any) != 0;
-    }
 
     struct WRegs { uint32_t w[C::WU][C::WWORDS]; };
     struct XRegs {
@@ -964,12 +956,22 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
         // The same steps.  The loads before the loop stay in the loop's order, for
         // its first wait covers both (reordered it waits for all loads but two: 64 x
         // 14336 x 4096 27.6 -> 29.4 us).
-        auto multiply = [&](auto w_tag) {
+        auto first_w = [&]() {
 #pragma unroll
             for (int q = 0; q < DW; q++) {
                 load_w(q, w[q]);
                 __builtin_amdgcn_sched_barrier(0);
             }
+        };
+        // weights on their way before the flags are waited for (0.5 to 1.5 us a
+        // call); the largest tile has no registers for them across the branch
+        if constexpr (FI == 4) first_w();
+        uint32_t any = 0;
+#pragma unroll
+        for (int q = 0; q < C::TI / 4; q++) any |= XF[(i0 - r0) / 4 + q];
+        const bool wide = __builtin_amdgcn_readfirstlane(any) != 0;
+        auto multiply = [&](auto w_tag) {
+            if constexpr (FI != 4) first_w();
 #pragma unroll
             for (int q = 0; q < DX; q++) {
                 load_x(q, x1[q], w_tag);
@@ -1262,7 +1264,8 @@ bool gemm_native_tile_takes(size_t m, size_t n, size_t k) {
 // The small-tile kernel of gemm.hip keeps short products over small matrices:
 // its 16 x 32 tiles reach all CUs without a split over K, and its code is
 // smaller (us, here against there: Q4_0 100 x 512 x 992 10.7 / 9.1, 200 x 2048 x
-// 992 13.6 / 12.7, 100 x 2048 x 2048 14.2 / 15.8, 100 x 64 x 4096 13.4 / 17.3;
+// 992 13.6 / 12.7, 100 x 4096 x 1024 12.9 / 11.8, 200 x 4096 x 1024 16.2 / 15.4, 200 x
+// 2048 x 2048 18.8 / 16.6 (100 rows: 14.1 / 15.0), 100 x 64 x 4096 13.4 / 17.3;
 // Q8_0 100 x 512 x 992 11.0 / 8.9, 1000 x 512 x 992 17.5 / 16.4, 333 x 4096 x 992
 // 19.5 / 25.7, 17 x 4096 x 4096 17.9 / 17.2, 33 x 4096 x 4096 18.6 / 24.4; Q4_K 64 x
 // 2048 x 2048 16.5 / 14.7, 128 x 2048 x 2048 18.5 / 19.1, 32 x 512 x 4096 17.3 / 22.3, 16 x
