@@ -36,7 +36,6 @@ sys.path.insert(0, os.path.join(ROOT, "rust-deeplearning_amd"))
 METRIC = "Q4_0/Q4_K GEMV achieved HBM GB/s (% peak); 7B Q4_0 decode tokens/s"
 PEAK_HBM_GBPS = 8000.0
 PEAK_F16_TFLOPS = 2500.0  # dense f16/bf16 MFMA, MI355X
-PEAK_I8_TOPS = 5000.0     # dense int8 MFMA, MI355X
 N_OUT, K_IN = 11008, 4096
 SEED = 0x5EED0002
 # the kernel the library launches for this workload (8-wave workgroups, 3 rows per wave)
@@ -417,7 +416,8 @@ TYPE_NAME = {2: "Q4_0", 3: "Q4_1", 8: "Q8_0", 12: "Q4_K", 14: "Q6_K"}
 def gemm_lines(rig, ms_list, seed=0x5EED0004, native=False, dtype=2):
     """Y = X W^T, W 4096x4096 Q4_0, X f32 [M, 4096]; the whole call
     (activation split or Q8_0 quantization + MFMA GEMM) timed over a loop of
-    launches.  native: matmul_f32_q4_native (int8 MFMA on the Q8_0 codes).
+    launches.  native: matmul_f32_q4_native (at these rows f16 MFMA on the
+    Q8_0 values of x).
     dtype: the same product for another weight format (not a BASELINE
     config; the tile GEMM of Q8_0, Q4_1, Q4_K and Q6_K)."""
     torch, rq = rig.torch, rig.rq
@@ -449,21 +449,21 @@ def gemm_lines(rig, ms_list, seed=0x5EED0004, native=False, dtype=2):
               else exact_check(rig, weights[0][1], x, y, m, n, k, cond=dtype != 2))
         tflops = flops / (ms * 1e-3) / 1e12
         gbps = abytes / (ms * 1e-3) / 1e9
-        peak_mm = PEAK_I8_TOPS if native else PEAK_F16_TFLOPS
+        peak_mm = PEAK_F16_TFLOPS
         bound = "mfma" if flops / abytes > peak_mm * 1e12 / (PEAK_HBM_GBPS * 1e9) else "hbm"
         out.append({
-            "workload": (f"config4 M={m}" + (" native (matmul_f32_q4_native, int8 MFMA)" if native else "")
+            "workload": (f"config4 M={m}" + (" native (matmul_f32_q4_native)" if native else "")
                          if dtype == 2 else f"{TYPE_NAME[dtype]} GEMM 4096x4096 M={m} (not a BASELINE config)"),
             "m": m,
             "value": round(tflops, 2),
-            "unit": "TOP/s" if native else "TFLOP/s",
+            "unit": "TFLOP/s",
             "ms_per_call": round(ms, 5),
             "hbm_GBs": round(gbps, 1),
             "roofline": {
                 "bound": bound,
                 "achieved": round(tflops, 2) if bound == "mfma" else round(gbps, 1),
                 "peak": peak_mm if bound == "mfma" else PEAK_HBM_GBPS,
-                "unit": ("TOP/s" if native else "TFLOP/s") if bound == "mfma" else "GB/s",
+                "unit": "TFLOP/s" if bound == "mfma" else "GB/s",
                 "frac": round(tflops / peak_mm if bound == "mfma" else gbps / PEAK_HBM_GBPS, 4),
             },
             "parity_vs_exact": ok,

@@ -147,7 +147,7 @@ rdl_status rdl_llama_set_fused_attention(rdl_llama* model, int32_t enable);
  * (TransformerBlock::set_native_q4_matmul, transformer_block.rs:248-255;
  * layer = -1: every layer, as gemma3_gguf.rs:126-128 does): the layer's
  * Q4_0 and Q4_1 products quantize their activation rows to Q8_0
- * (quantize_row_q8_0) and sum int32 block dots (matmul_f32_q4_native /
+ * (quantize_row_q8_0) as RDL_MODE_NATIVE does (matmul_f32_q4_native /
  * matmul_f32_q4_1_native, quantize.rs:326-394, 501-572); other types keep
  * their one path (linear.rs:119-177).  Such layers run their RMSNorm, RoPE,
  * SwiGLU and adds as separate launches.  The output matrix is not a layer's

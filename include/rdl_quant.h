@@ -69,8 +69,11 @@ enum {
 /* ---- arithmetic modes (Linear::use_native_q4, linear.rs:23-24, 96-98) ---- */
 enum {
     RDL_MODE_FLOAT = 0, /* f32 activations: matmul_f32_q4 / _q8 / _q4_1 semantics */
-    RDL_MODE_NATIVE = 1 /* activations quantized to Q8_0, int32 block dots:
-                           matmul_f32_q4_native / _q4_1_native semantics */
+    RDL_MODE_NATIVE = 1 /* activations quantized to Q8_0 (quantize_row_q8_0):
+                           matmul_f32_q4_native / _q4_1_native semantics.  Exact
+                           int32 block dots, except Q4_0 products of more than 64
+                           rows on the tile GEMM: the same codes times their
+                           scale, exact as f16 pairs, in f32 block dots */
 };
 
 /* Text of a status code; never NULL. */
@@ -92,10 +95,10 @@ const char* rdl_version(void);
 int32_t rdl_device_count(void);
 
 /* Testing switch (no reference counterpart).  The Q4_0 GEMMs for 5-64 rows
- * split K over workgroups whose partials the last one of each strip adds.
- * RDL_COMBINE_AUTO (the default): where the device deals each launch's
- * workgroups round-robin over its XCDs (probed once per device), a strip's
- * slices share one XCD and its L2, and the partials stay there.
+ * and the tile GEMM split K over workgroups whose partials the last one of each
+ * strip or tile adds.  RDL_COMBINE_AUTO (the default): where the device deals
+ * each launch's workgroups round-robin over its XCDs (probed once per device),
+ * a strip's slices share one XCD and its L2, and the partials stay there.
  * RDL_COMBINE_COHERENT: every launch takes the agent-coherent combine
  * (write-through partials, device-scope counter).  Both give the same bits.
  * Process-wide; set it while no call is in flight. */
@@ -168,7 +171,10 @@ rdl_status rdl_quantize_row_q8_0(const float* input, size_t input_len, uint8_t* 
 
 /* Debug view of matmul_f32_q4_native's integer stage (quantize.rs:383):
  * partials[(r*out_features + c)*(in_features/32) + b] = dot_q4q8_block(W[c,b], q8(x_r)[b]),
- * the exact int32 value the reference accumulates before scaling. */
+ * the exact int32 value the reference accumulates before scaling.  The
+ * product's own kernels compute these except where the tile GEMM takes a native
+ * product (more than 64 rows, RDL_MODE_NATIVE above), which has no integer
+ * stage: there the view shows the codes and weights it starts from. */
 rdl_status rdl_q4_0_q8_0_block_dots(const float* input_data, size_t input_len,
                                     const uint8_t* weight_bytes, size_t weight_len, size_t m,
                                     size_t in_features, size_t out_features, int32_t* partials,

@@ -566,7 +566,8 @@ rdl_status rdl_q4_0_q8_0_block_dots(const float* x, size_t x_len, const uint8_t*
     HIP_TRY(hipMemcpy(dx.p, x, m * k * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dw.p, w, n * nb * rdl::Q4_0_BYTES, hipMemcpyHostToDevice));
     if (m > FUSED_MAX_M && gemm_fits(WType::Q4_0, true, m, n, k)) {
-        // the rows matmul_f32_q4_native takes to the int8 GEMM: its own MFMA block dots
+        // the int8 GEMM's MFMA block dots (native products of more than 4 rows that
+        // the tile GEMM leaves run on it)
         HIP_TRY(dr.alloc(rdl::gemm_scratch_bytes(m, n, k, true)));
         HIP_TRY(rdl::launch_gemm_q4_0_native((const uint8_t*)dw.p, n, k, (const float*)dx.p, m, nullptr,
                                              (int32_t*)dp.p, dr.p, nullptr));
