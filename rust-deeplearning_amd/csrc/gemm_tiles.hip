@@ -1331,6 +1331,7 @@ hipError_t launch_gemm_tile(WType t, const uint8_t* w, size_t n, size_t k, const
     if (pro == 3 ? t != WType::Q4_0 || k == 0 || !gemm_native_tile_takes(m, n, k)
                  : k == 0 || !gemm_tile_takes(t, m, n, k) || (pro != 0 && k > GEMM_SPLIT_MAX_K))
         return hipErrorInvalidValue;
+    if (chunk == 0 && lo) return hipErrorInvalidValue;  // (not one row fits)
     if (chunk == 0) chunk = m;
     if (chunk < m && chunk % TILE_SHAPES[0].ti != 0) return hipErrorInvalidValue;
     const TilePlan p = tile_plan(t, m, n, k / QK, part != nullptr && cnt != nullptr);
