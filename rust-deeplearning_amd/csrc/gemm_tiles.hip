@@ -963,9 +963,15 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        // weights on their way before the flags are waited for (0.5 to 1.5 us a
-        // call); the largest tile has no registers for them across the branch
+        // weights, and chunk 0 of x, on their way before the flags are waited for
+        // (0.2 to 1 us a call) where there are registers for them across the branch
+        constexpr int EX = FI == 4 && C::NT == 512 ? 1 : 0;
         if constexpr (FI == 4) first_w();
+#pragma unroll
+        for (int q = 0; q < EX; q++) {
+            load_x(q, x1[q], plain);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         uint32_t any = 0;
 #pragma unroll
         for (int q = 0; q < C::TI / 4; q++) any |= XF[(i0 - r0) / 4 + q];
@@ -974,7 +980,8 @@ __global__ __launch_bounds__(WJ * KS * 64, 2) void gemm_tile_kernel(
             if constexpr (FI != 4) first_w();
 #pragma unroll
             for (int q = 0; q < DX; q++) {
-                load_x(q, x1[q], w_tag);
+                if (q >= EX) load_x(q, x1[q], w_tag);
+                else if constexpr (decltype(w_tag)::value) load_scale(q, x1[q]);
                 __builtin_amdgcn_sched_barrier(0);
             }
             store_w(0, bc, ac, w[0]);
