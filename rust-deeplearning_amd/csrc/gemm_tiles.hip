@@ -414,7 +414,7 @@ __device__ __forceinline__ void q6k_f16(uint32_t n0, uint32_t n1, uint32_t scale
 // WIDE: x may have rows of wide range (WIDE_ROW).  A tile with one takes the
 // loop with a scale a block and row, one multiplication a result more; the
 // others take the plain loop (a byte a row tells, read through scalar registers:
-// no barrier; 0.3 to 0.6 us a call).  us without such rows, with them, and on the
+// no barrier; 0.4 to 0.8 us a call).  us without such rows, with them, and on the
 // x-tile or int8 kernel, which always scale so: 64 x 14336 x 4096 32 / 37 / 58, 16 x
 // 32000 x 4096 43 / 52 / 57, native 512 x 14336 x 4096 135 / 199 / 190.
 template <int WF, int FI, int WJ, int KS, bool LOCAL, bool WIDE>
